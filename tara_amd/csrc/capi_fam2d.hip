@@ -9,6 +9,7 @@
 
 #include "fam2d.h"
 #include "generic_fam2d.h"
+#include "layout.h"
 
 namespace tara {
 namespace {
@@ -21,18 +22,15 @@ int check_nh(const char* name, int nx, int nh)
     return TARA_OK;
 }
 
-// host (nh, ny) contiguous <-> device (ld, ny)
-int h2d(const F2Plan& p, double2* d, const double* h, hipStream_t s)
+// nf fields, host (nh, ny) contiguous <-> device (ld, ny), through the plan's
+// inverse-transform scratch (6 or 8 fields, idle between steps of the same stream).
+int h2d(const F2Plan& p, double2* const d[], const double* const h[], int nf, hipStream_t s)
 {
-    TARA_HIP(hipMemcpy2DAsync(d, p.ld * sizeof(double2), h, p.nh * sizeof(double2), p.nh * sizeof(double2), p.ny,
-                              hipMemcpyHostToDevice, s));
-    return TARA_OK;
+    return rows_from_host(d, h, nf, p.nh, p.ld, p.ny, p.a, s);
 }
-int d2h(const F2Plan& p, double* h, const double2* d, hipStream_t s)
+int d2h(const F2Plan& p, double* const h[], const double2* const d[], int nf, hipStream_t s)
 {
-    TARA_HIP(hipMemcpy2DAsync(h, p.nh * sizeof(double2), d, p.ld * sizeof(double2), p.nh * sizeof(double2), p.ny,
-                              hipMemcpyDeviceToHost, s));
-    return TARA_OK;
+    return rows_to_host(h, d, nf, p.nh, p.ld, p.ny, p.a, s);
 }
 
 struct DropIn {
@@ -107,11 +105,10 @@ int derive_host(int family, int nx, int ny, double pi, double lx, double ly, con
     for (int f = 0; f < nf; ++f) {
         st[f] = d->st[f].as<double2>();
         out[f] = d->out[f].as<double2>();
-        if ((rc = h2d(p, st[f], state[f], nullptr))) return rc;
     }
+    if ((rc = h2d(p, st, state, nf, nullptr))) return rc;
     if ((rc = stage(p, st, out))) return rc;
-    for (int f = 0; f < nf; ++f)
-        if ((rc = d2h(p, rhs[f], out[f], nullptr))) return rc;
+    if ((rc = d2h(p, rhs, out, nf, nullptr))) return rc;
     TARA_HIP(hipDeviceSynchronize());
     return TARA_OK;
 }
@@ -291,12 +288,14 @@ static int f2_check_finite(tara_f2* c)
 extern "C" int tara_f2_upload(tara_f2* c, const double* const state[])
 {
     TARA_CHECK(c && state, TARA_ERR_ARG, "null argument");
+    double2* st[6];
     for (int f = 0; f < kFields[c->family]; ++f) {
         TARA_CHECK(state[f], TARA_ERR_ARG, "null array %d", f);
-        int rc = h2d(c->plan, c->st[f].as<double2>(), state[f], c->s);
-        if (rc) return rc;
+        st[f] = c->st[f].as<double2>();
         TARA_HIP(hipMemsetAsync(c->hist[f].p, 0, c->hist[f].bytes, c->s));
     }
+    int rc = h2d(c->plan, st, state, kFields[c->family], c->s);
+    if (rc) return rc;
     TARA_HIP(hipMemsetAsync(c->plan.bad.p, 0, sizeof(int), c->s));
     TARA_HIP(hipStreamSynchronize(c->s));
     return TARA_OK;
@@ -305,11 +304,13 @@ extern "C" int tara_f2_upload(tara_f2* c, const double* const state[])
 extern "C" int tara_f2_download(tara_f2* c, double* const state[])
 {
     TARA_CHECK(c && state, TARA_ERR_ARG, "null argument");
+    double2* st[6];
     for (int f = 0; f < kFields[c->family]; ++f) {
         TARA_CHECK(state[f], TARA_ERR_ARG, "null array %d", f);
-        int rc = d2h(c->plan, state[f], c->st[f].as<double2>(), c->s);
-        if (rc) return rc;
+        st[f] = c->st[f].as<double2>();
     }
+    int rc = d2h(c->plan, state, st, kFields[c->family], c->s);
+    if (rc) return rc;
     return f2_check_finite(c);
 }
 

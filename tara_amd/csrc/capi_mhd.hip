@@ -9,6 +9,7 @@
 
 #include "fft_api.h"
 #include "generic3d.h"
+#include "layout.h"
 #include "mhd3d.h"
 #include "philox.h"
 
@@ -24,18 +25,15 @@ int check_dims(int nx, int ny, int nz, int nh)
     return TARA_OK;
 }
 
-// host (nh, ny, nz) contiguous <-> device (ld, ny, nz)
-int h2d(const MhdPlan& p, double2* d, const double* h, hipStream_t s)
+// nf fields, host (nh, ny, nz) contiguous <-> device (ld, ny, nz), through the
+// plan's flux scratch (14 fields, idle between steps of the same stream).
+int h2d(const MhdPlan& p, double2* const d[], const double* const h[], int nf, hipStream_t s)
 {
-    TARA_HIP(hipMemcpy2DAsync(d, p.ld * sizeof(double2), h, p.nh * sizeof(double2), p.nh * sizeof(double2),
-                              (size_t)p.ny * p.nz, hipMemcpyHostToDevice, s));
-    return TARA_OK;
+    return rows_from_host(d, h, nf, p.nh, p.ld, (size_t)p.ny * p.nz, p.b, s);
 }
-int d2h(const MhdPlan& p, double* h, const double2* d, hipStream_t s)
+int d2h(const MhdPlan& p, double* const h[], const double2* const d[], int nf, hipStream_t s)
 {
-    TARA_HIP(hipMemcpy2DAsync(h, p.nh * sizeof(double2), d, p.ld * sizeof(double2), p.nh * sizeof(double2),
-                              (size_t)p.ny * p.nz, hipMemcpyDeviceToHost, s));
-    return TARA_OK;
+    return rows_to_host(h, d, nf, p.nh, p.ld, (size_t)p.ny * p.nz, p.b, s);
 }
 
 struct DropIn {
@@ -85,14 +83,17 @@ extern "C" int tara_derive3com(int nx, int ny, int nz, int nh, const tara_mhd_pa
     if ((rc = get_dropin(nx, ny, nz, prm, &d))) return rc;
     const MhdPlan& p = d->plan;
     double2 *st[7], *out[7];
+    const double* hin[7];
+    double* hout[7];
     for (int f = 0; f < 7; ++f) {
         st[f] = d->st[f].as<double2>();
         out[f] = d->out[f].as<double2>();
-        if ((rc = h2d(p, st[f], state[kLive[f]], nullptr))) return rc;
+        hin[f] = state[kLive[f]];
+        hout[f] = rhs[kLive[f]];
     }
+    if ((rc = h2d(p, st, hin, 7, nullptr))) return rc;
     if ((rc = mhd_rhs_stage(p, st, MHD_RHS, 0.0, out, nullptr, nullptr, nullptr))) return rc;
-    for (int f = 0; f < 7; ++f)
-        if ((rc = d2h(p, rhs[kLive[f]], out[f], nullptr))) return rc;
+    if ((rc = d2h(p, hout, out, 7, nullptr))) return rc;
     TARA_HIP(hipStreamSynchronize(nullptr));
     std::memset(rhs[4], 0, (size_t)nh * ny * nz * 2 * sizeof(double));
     return TARA_OK;
@@ -161,11 +162,13 @@ extern "C" int tara_mhd_create(int nx, int ny, int nz, const tara_mhd_params* pr
 extern "C" int tara_mhd_upload(tara_mhd* c, const double* const state[8])
 {
     TARA_CHECK(c && state, TARA_ERR_ARG, "null argument");
-    int rc;
+    double2* st[8];
     for (int f = 0; f < 8; ++f) {
         TARA_CHECK(state[f], TARA_ERR_ARG, "null array %d", f);
-        if ((rc = h2d(c->plan, c->st[f].as<double2>(), state[f], c->s))) return rc;
+        st[f] = c->st[f].as<double2>();
     }
+    int rc = h2d(c->plan, st, state, 8, c->s);
+    if (rc) return rc;
     for (int f = 0; f < 7; ++f) TARA_HIP(hipMemsetAsync(c->hist[f].p, 0, c->hist[f].bytes, c->s));
     TARA_HIP(hipMemsetAsync(c->plan.bad.p, 0, sizeof(int), c->s));
     TARA_HIP(hipStreamSynchronize(c->s));
@@ -188,11 +191,13 @@ int check_finite(tara_mhd* c)
 extern "C" int tara_mhd_download(tara_mhd* c, double* const state[8])
 {
     TARA_CHECK(c && state, TARA_ERR_ARG, "null argument");
-    int rc;
+    double2* st[8];
     for (int f = 0; f < 8; ++f) {
         TARA_CHECK(state[f], TARA_ERR_ARG, "null array %d", f);
-        if ((rc = d2h(c->plan, state[f], c->st[f].as<double2>(), c->s))) return rc;
+        st[f] = c->st[f].as<double2>();
     }
+    int rc = d2h(c->plan, state, st, 8, c->s);
+    if (rc) return rc;
     TARA_HIP(hipStreamSynchronize(c->s));
     return check_finite(c);  // the state is copied out either way
 }

@@ -7,11 +7,13 @@
 //
 // These are the building blocks the fused solver passes are made of, exposed
 // on their own for parity testing and for the driver-side transforms.
+#include <algorithm>
 #include <cstring>
 #include <memory>
 
 #include "common.h"
 #include "fft_api.h"
+#include "layout.h"
 #include "passes.h"
 
 namespace tara {
@@ -203,7 +205,7 @@ int check_dims(int nx, int ny, int nz)
 // calls and grown when a larger transform comes (the kept mains call the same
 // sizes every step).
 struct HostWs {
-    DevBuf spec, real;
+    DevBuf spec, real;  // real also holds the packed spectrum on its way to or from the host
 };
 std::mutex g_ws_mu;
 std::map<int, std::unique_ptr<HostWs>> g_ws;
@@ -220,7 +222,8 @@ int fft_host(int nx, int ny, int nz, const double* in, double* out, bool forward
     DevBuf& spec = ws->spec;
     DevBuf& real = ws->real;
     if (spec.bytes < drows * ld * sizeof(double2) && (rc = spec.alloc(drows * ld * sizeof(double2)))) return rc;
-    if (real.bytes < drows * nx * sizeof(double) && (rc = real.alloc(drows * nx * sizeof(double)))) return rc;
+    const size_t rb = std::max(drows * nx * sizeof(double), rows * nh * sizeof(double2));
+    if (real.bytes < rb && (rc = real.alloc(rb))) return rc;
     hipStream_t st = nullptr;
     double2* S = spec.as<double2>();
     if (forward) {
@@ -229,12 +232,10 @@ int fft_host(int nx, int ny, int nz, const double* in, double* out, bool forward
         if ((rc = row_r2c(real.as<double>(), S, nx, ld, (int)drows, st))) return rc;
         if (ny > 1 && (rc = col_fft(S, ny, ld, ld, (long)ld * ny, nz, -1, st))) return rc;
         if (nz > 1 && (rc = col_fft(S, nz, ld, (long)ld * ny, ld, ny, -1, st))) return rc;
-        TARA_HIP(hipMemcpy2D(out, nh * sizeof(double2), S, ld * sizeof(double2), nh * sizeof(double2), rows,
-                             hipMemcpyDeviceToHost));
+        if ((rc = rows_to_host(&out, &S, 1, nh, ld, rows, real, st))) return rc;
     } else {
-        TARA_HIP(hipMemset(S, 0, drows * ld * sizeof(double2)));
-        TARA_HIP(hipMemcpy2D(S, ld * sizeof(double2), in, nh * sizeof(double2), nh * sizeof(double2), rows,
-                             hipMemcpyHostToDevice));
+        if (drows > rows) TARA_HIP(hipMemset(S, 0, drows * ld * sizeof(double2)));
+        if ((rc = rows_from_host(&S, &in, 1, nh, ld, rows, real, st))) return rc;
         if (nz > 1 && (rc = col_fft(S, nz, ld, (long)ld * ny, ld, ny, +1, st))) return rc;
         if (ny > 1 && (rc = col_fft(S, ny, ld, ld, (long)ld * ny, nz, +1, st))) return rc;
         if ((rc = row_c2r(S, real.as<double>(), nx, ld, (int)drows, 1.0, st))) return rc;

@@ -1,5 +1,6 @@
 // Tiled transposes through LDS (32 x 32 complex tiles, one padding column) for
-// the kx-fastest <-> ky-major conversions at the host boundary.
+// the kx-fastest <-> ky-major conversions at the host boundary, and the packing
+// of padded rows for host copies.
 #include "layout.h"
 
 namespace tara {
@@ -39,6 +40,79 @@ int to_kymajor(const double2* src, double2* dst, int nh, int ny, int nplanes, hi
 int from_kymajor(const double2* src, double2* dst, int nh, int ny, int nplanes, hipStream_t st)
 {
     return transpose(src, dst, nh, ny, nplanes, st);
+}
+
+// One thread per element of the padded or packed rows; both streams are read
+// and written contiguously, so the kernel runs at the copy rate (0.1 ms for
+// the 270 MB above) and the host link bounds the transfer.
+template <bool PACK>
+__global__ __launch_bounds__(256) void k_rows(RowFields f, int nh, int ld, size_t rows)
+{
+    const double2* src = f.src[blockIdx.y];
+    double2* dst = f.dst[blockIdx.y];
+    const int w = PACK ? nh : ld;
+    for (size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x; q < rows * w; q += (size_t)gridDim.x * blockDim.x) {
+        const size_t r = q / w;
+        const int i = (int)(q - r * w);
+        if (PACK)
+            dst[q] = src[r * ld + i];
+        else
+            dst[q] = i < nh ? src[r * nh + i] : make_double2(0.0, 0.0);
+    }
+}
+
+template <bool PACK>
+static int launch_rows(const RowFields& f, int nfields, int nh, int ld, size_t rows, hipStream_t st)
+{
+    TARA_CHECK(nfields >= 1 && nfields <= 8 && nh <= ld, TARA_ERR_ARG, "row packing: bad shape");
+    const size_t n = rows * (PACK ? nh : ld), nb = (n + 255) / 256;
+    hipLaunchKernelGGL(k_rows<PACK>, dim3((unsigned)(nb < 16384 ? nb : 16384), nfields), dim3(256), 0, st, f, nh, ld,
+                       rows);
+    TARA_HIP(hipGetLastError());
+    return TARA_OK;
+}
+
+int pack_rows(const RowFields& f, int nfields, int nh, int ld, size_t rows, hipStream_t st)
+{
+    return launch_rows<true>(f, nfields, nh, ld, rows, st);
+}
+
+int unpack_rows(const RowFields& f, int nfields, int nh, int ld, size_t rows, hipStream_t st)
+{
+    return launch_rows<false>(f, nfields, nh, ld, rows, st);
+}
+
+int rows_from_host(double2* const dev[], const double* const host[], int nfields, int nh, int ld, size_t rows,
+                   const DevBuf& pack, hipStream_t st)
+{
+    const size_t n = rows * nh;
+    TARA_CHECK(nfields >= 1 && nfields <= 8 && pack.bytes >= nfields * n * sizeof(double2), TARA_ERR_STATE,
+               "row transfer: work space too small");
+    RowFields f{};
+    for (int k = 0; k < nfields; ++k) {
+        f.src[k] = pack.as<double2>() + k * n;
+        f.dst[k] = dev[k];
+        TARA_HIP(hipMemcpyAsync(pack.as<double2>() + k * n, host[k], n * sizeof(double2), hipMemcpyHostToDevice, st));
+    }
+    return unpack_rows(f, nfields, nh, ld, rows, st);
+}
+
+int rows_to_host(double* const host[], const double2* const dev[], int nfields, int nh, int ld, size_t rows,
+                 const DevBuf& pack, hipStream_t st)
+{
+    const size_t n = rows * nh;
+    TARA_CHECK(nfields >= 1 && nfields <= 8 && pack.bytes >= nfields * n * sizeof(double2), TARA_ERR_STATE,
+               "row transfer: work space too small");
+    RowFields f{};
+    for (int k = 0; k < nfields; ++k) {
+        f.src[k] = dev[k];
+        f.dst[k] = pack.as<double2>() + k * n;
+    }
+    int rc = pack_rows(f, nfields, nh, ld, rows, st);
+    if (rc) return rc;
+    for (int k = 0; k < nfields; ++k)
+        TARA_HIP(hipMemcpyAsync(host[k], pack.as<double2>() + k * n, n * sizeof(double2), hipMemcpyDeviceToHost, st));
+    return TARA_OK;
 }
 
 }  // namespace tara
