@@ -44,10 +44,6 @@ MEASURED_TRAFFIC = {
     ("k_csh_x", 4096, 3): 2.7163e9,
     ("k_csh_x", 4096, 4): 7.1465e8,
     ("k_csh_x", 4096, 5): 6.9267e8,
-    ("k_mhd_col_inverse_zy", 256): 3.9932e9,   # two launches (z, then y), 1.9966e9 each
-    ("k_mhd_x", 256): 2.9069e9,
-    ("k_mhd_col_forward", 256): 3.9931e9,
-    ("k_mhd_zfwd", 256): 6.1173e9,
 }
 METRIC = "grid-pt steps/s FP64 (2D 4096², 3D 256³ MHD); FNO sim-time/s at ≤5% L2 err"
 
@@ -67,6 +63,28 @@ def model_2d(n, nsteps):
         return ({0: 5 * S, 1: 5 * S, 2: (36 * nsteps - 4) * S / (4 * nsteps)},
                 {0: "k_csh_yinv", 1: "k_csh_x", 2: "k_csh_yfwd_inv"}, 56 * S)
     return {0: 5 * S, 1: 5 * S, 2: 5 * S}, {0: "k_csh_yinv", 1: "k_csh_x", 2: "k_csh_yfwd"}, 60 * S
+
+
+def model_mhd(n, nsteps):
+    """Algorithmic bytes of the 3D AB2 path at n^3 in a 2 pi box per step, for
+    one advance call of nsteps steps: inverse z and y, x, forward y, forward z.
+    Only modes inside the dealiasing sphere |k| < n/3 ever change, so the passes
+    after the x pass's reads carry tiles of 8 kx columns that hold one, and the
+    inverse passes redo only theirs after the call's first step."""
+    S3 = 16.0 * (n // 2 + 1) * n * n
+    nh, cut = n // 2 + 1, (3 * n / 3.0) / 3.0
+    half = range(n // 2 + 1)
+    width = [math.ceil(math.sqrt(max(cut * cut - j * j, 0.0))) for j in half]  # kx columns alive at ky = j, kz = 0
+    mult = [1 if j in (0, n // 2) else 2 for j in half]                       # +-ky
+    tiles = [(w + 7) // 8 for w in width]
+    kt = max(tiles)
+    fk = min(8 * kt, nh) / nh                                                  # kx columns kept
+    fl = sum(t * m for t, m in zip(tiles, mult)) * 8 / (nh * n)                # z columns kept
+    fs = 2.0 / 3.0 * math.pi * cut ** 3 / (nh * n * n)                         # modes alive
+    inv = (14 * fk * (nsteps - 1) + 28) / nsteps
+    # z: 12 fluxes, 7 state fields and the momentum again for the density, the
+    # histories and updates of the live modes, the new state's inverse transform
+    return [inv * S3, (7 + 12 * fk) * S3, 12 * (fk + fl) * S3, ((12 + 10 + 7) * fl + 21 * fs) * S3]
 
 
 def cpu_baseline(case, n, steps):
@@ -169,19 +187,15 @@ def bench_mhd(steps, warmup, n=256):
     s.sync()
     counts, kms = s.kernel_stats(4)
     s.close()
-    S3 = 16.0 * (n // 2 + 1) * n * n
-    # algorithmic bytes per timed region: inverse z and y passes (two launches)
-    # 7 fields in + 7 out each;
-    # x pass 7 in, 14 out; forward y 14 + 14; forward z reads 14 fluxes + 7 state
-    # + 7 history and writes 7 state + 7 history.  119 S3 per step.
+    # algorithmic bytes per timed region (see model_mhd)
     names = ["k_mhd_col_inverse_zy", "k_mhd_x", "k_mhd_col_forward", "k_mhd_zfwd"]
-    model = [28 * S3, 21 * S3, 28 * S3, 42 * S3]
+    model = model_mhd(n, steps)
     avg = {c: kms[c] / counts[c] for c in range(4) if counts[c]}
     dom = max(avg, key=lambda c: kms[c])
     achieved = model[dom] / (avg[dom] * 1e-3) / 1e9
     return {"workload": f"3D compressible isothermal MHD, AB2, {n}^3, FP64, nu = eta = 1e-3, dt = 5e-4",
             "value": n ** 3 / (ms * 1e-3), "unit": "grid-pt steps/s", "ms_per_step": ms,
-            "step_model_bytes": 119 * S3, "step_model_GBps": round(119 * S3 / (ms * 1e-3) / 1e9, 1),
+            "step_model_bytes": sum(model), "step_model_GBps": round(sum(model) / (ms * 1e-3) / 1e9, 1),
             "roofline": {"bound": "hbm", "kernel": names[dom], "achieved": round(achieved, 1),
                          "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                          "traffic": MEASURED_TRAFFIC.get((names[dom], n))},

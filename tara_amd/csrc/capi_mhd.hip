@@ -26,7 +26,7 @@ int check_dims(int nx, int ny, int nz, int nh)
 }
 
 // nf fields, host (nh, ny, nz) contiguous <-> device (ld, ny, nz), through the
-// plan's flux scratch (14 fields, idle between steps of the same stream).
+// plan's flux scratch (12 fields, idle between steps of the same stream).
 int h2d(const MhdPlan& p, double2* const d[], const double* const h[], int nf, hipStream_t s)
 {
     return rows_from_host(d, h, nf, p.nh, p.ld, (size_t)p.ny * p.nz, p.b, s);
@@ -55,6 +55,7 @@ int get_dropin(int nx, int ny, int nz, const tara_mhd_params* prm, DropIn** out)
         for (int f = 0; f < 7; ++f) {
             if ((rc = d->st[f].alloc(bytes)) || (rc = d->out[f].alloc(bytes))) return rc;
             TARA_HIP(hipMemset(d->st[f].p, 0, bytes));
+            TARA_HIP(hipMemset(d->out[f].p, 0, bytes));  // modes that never live stay zero
         }
         it = g_dropin.emplace(key, std::move(d)).first;
     }
@@ -92,7 +93,7 @@ extern "C" int tara_derive3com(int nx, int ny, int nz, int nh, const tara_mhd_pa
         hout[f] = rhs[kLive[f]];
     }
     if ((rc = h2d(p, st, hin, 7, nullptr))) return rc;
-    if ((rc = mhd_rhs_stage(p, st, MHD_RHS, 0.0, out, nullptr, nullptr, nullptr))) return rc;
+    if ((rc = mhd_rhs_stage(p, st, out, nullptr, nullptr))) return rc;
     if ((rc = d2h(p, hout, out, 7, nullptr))) return rc;
     TARA_HIP(hipStreamSynchronize(nullptr));
     std::memset(rhs[4], 0, (size_t)nh * ny * nz * 2 * sizeof(double));
@@ -128,6 +129,8 @@ extern "C" int tara_ab3com(int nx, int ny, int nz, int nh, double dt, const doub
 struct tara_mhd {
     MhdPlan plan;
     DevBuf st[8], hist[7];
+    DevBuf mom[3];         // the other set of momentum fields a step writes (mhd_advance)
+    bool mom_set = false;  // mom holds st's values outside the live modes (false: a new state was set)
     hipStream_t s = nullptr;
     double dt = 0;
     std::unique_ptr<EventTimer> tm;
@@ -143,7 +146,7 @@ extern "C" int tara_mhd_create(int nx, int ny, int nz, const tara_mhd_params* pr
     *out = nullptr;
     auto c = std::make_unique<tara_mhd>();
     int rc = mhd_plan_init(c->plan, nx, ny, nz, prm->lx, prm->ly, prm->lz, prm->mu, prm->eta, prm->cs);
-    if (rc) return rc;
+    if (rc || (rc = mhd_plan_stepping(c->plan))) return rc;
     const size_t bytes = c->plan.fsz * sizeof(double2);
     for (int f = 0; f < 8; ++f) {
         if ((rc = c->st[f].alloc(bytes))) return rc;
@@ -153,6 +156,8 @@ extern "C" int tara_mhd_create(int nx, int ny, int nz, const tara_mhd_params* pr
         if ((rc = c->hist[f].alloc(bytes))) return rc;
         TARA_HIP(hipMemset(c->hist[f].p, 0, bytes));
     }
+    for (int f = 0; f < 3; ++f)
+        if ((rc = c->mom[f].alloc(bytes))) return rc;
     TARA_HIP(hipStreamCreate(&c->s));
     c->dt = prm->dt;
     *out = c.release();
@@ -170,6 +175,7 @@ extern "C" int tara_mhd_upload(tara_mhd* c, const double* const state[8])
     int rc = h2d(c->plan, st, state, 8, c->s);
     if (rc) return rc;
     for (int f = 0; f < 7; ++f) TARA_HIP(hipMemsetAsync(c->hist[f].p, 0, c->hist[f].bytes, c->s));
+    c->mom_set = false;
     TARA_HIP(hipMemsetAsync(c->plan.bad.p, 0, sizeof(int), c->s));
     TARA_HIP(hipStreamSynchronize(c->s));
     return TARA_OK;
@@ -205,16 +211,23 @@ extern "C" int tara_mhd_download(tara_mhd* c, double* const state[8])
 extern "C" int tara_mhd_advance(tara_mhd* c, int nsteps)
 {
     TARA_CHECK(c && nsteps >= 0, TARA_ERR_ARG, "bad argument");
-    double2 *st[7], *h[7];
+    if (nsteps == 0) return TARA_OK;
+    double2 *st[7], *h[7], *mom[3];
     for (int f = 0; f < 7; ++f) {
         st[f] = c->st[kLive[f]].as<double2>();
         h[f] = c->hist[f].as<double2>();
     }
-    for (int k = 0; k < nsteps; ++k) {
-        int rc = mhd_rhs_stage(c->plan, st, MHD_AB2, c->dt, nullptr, h, c->s, c->tm.get());
-        if (rc) return rc;
+    for (int f = 0; f < 3; ++f) {
+        mom[f] = c->mom[f].as<double2>();
+        if (!c->mom_set) TARA_HIP(hipMemcpyAsync(mom[f], st[1 + f], c->mom[f].bytes, hipMemcpyDeviceToDevice, c->s));
     }
-    return TARA_OK;
+    c->mom_set = true;
+    int rc = mhd_advance(c->plan, st, mom, h, nsteps, c->dt, c->s, c->tm.get());
+    for (int f = 0; f < 3; ++f) {
+        c->st[1 + f].p = st[1 + f];
+        c->mom[f].p = mom[f];
+    }
+    return rc;
 }
 
 extern "C" int tara_mhd_sync(tara_mhd* c)
@@ -277,6 +290,7 @@ extern "C" int tara_mhd_ic_abc(tara_mhd* c, double rho0, double u0, double b0, d
         if ((rc = col_fft(s, p.nz, p.ld, (long)p.ld * p.ny, p.ld, p.ny, -1, c->s))) return rc;
     }
     for (int f = 0; f < 7; ++f) TARA_HIP(hipMemsetAsync(c->hist[f].p, 0, c->hist[f].bytes, c->s));
+    c->mom_set = false;
     TARA_HIP(hipMemsetAsync(c->plan.bad.p, 0, sizeof(int), c->s));
     TARA_HIP(hipStreamSynchronize(c->s));
     return TARA_OK;
@@ -462,6 +476,7 @@ extern "C" int tara_mhd_ic_random(tara_mhd* c, unsigned seed, double k0, double 
     if ((rc = col_fft(e, p.ny, p.ld, p.ld, (long)p.ld * p.ny, p.nz, -1, s))) return rc;
     if ((rc = col_fft(e, p.nz, p.ld, (long)p.ld * p.ny, p.ld, p.ny, -1, s))) return rc;
     for (int f = 0; f < 7; ++f) TARA_HIP(hipMemsetAsync(c->hist[f].p, 0, c->hist[f].bytes, s));
+    c->mom_set = false;
     TARA_HIP(hipMemsetAsync(c->plan.bad.p, 0, sizeof(int), s));
     TARA_HIP(hipStreamSynchronize(s));
     return TARA_OK;

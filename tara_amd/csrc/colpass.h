@@ -20,6 +20,7 @@ struct ColArgs {
     long es;       // element stride along the transform (complex elements)
     long pstride;  // plane stride
     int tpp;       // tiles (of 8 columns) per plane
+    const int2* skip = nullptr;  // per tile of a plane: rows [x, y) of the result that nobody reads (null: none)
 };
 
 // Column FFT over tiles of 8 adjacent kx columns; blockIdx.y selects the field.
@@ -38,8 +39,12 @@ __global__ __launch_bounds__(CShape<N>::NT) void k_col_fft(ColArgs a, const doub
 #pragma unroll
     for (int e = 0; e < E; ++e) v[e] = src[(size_t)rf_first_idx<N>(t, e) * a.es];
     rf_fft<N, DIR>(v, t, lds + c * S::LP, tw);
+    const int2 skip = a.skip ? a.skip[tile % a.tpp] : make_int2(N, N);
 #pragma unroll
-    for (int e = 0; e < E; ++e) dst[(size_t)rf_final_idx<N>(t, e) * a.es] = v[e];
+    for (int e = 0; e < E; ++e) {
+        const int j = rf_final_idx<N>(t, e);
+        if (j < skip.x || j >= skip.y) dst[(size_t)j * a.es] = v[e];
+    }
 }
 
 // Launch over ntiles tiles x nfields fields (lengths 16..256).

@@ -415,12 +415,6 @@ __global__ __launch_bounds__(YShape<NY>::NT) void k_csh_yfwd(YfwdArgs a, const d
 // state) in registers, and the four spectra of it are transformed and written
 // to G0..G3 without reading it back: one field read less per stage.  Shape and
 // LDS as the inverse y pass; the forward y pass of H uses the same lanes.
-template <int N, int EM>
-constexpr bool rf_final_is_first()
-{
-    return fft_radix(N, RF<N, EM>::E) == RF<N, EM>::E && N / rf_last_span(N, RF<N, EM>::E) == RF<N, EM>::E;
-}
-
 template <int NY, int MODE, int GS>
 __global__ __launch_bounds__((YiShape<NY, false>::NT), (YiShape<NY, false>::IL ? 4 : 1)) void k_csh_yfwd_inv(
     YfwdArgs a, const double2* tw, double2* __restrict__ g0, double2* __restrict__ g1, double2* __restrict__ g2,
@@ -498,7 +492,7 @@ __global__ __launch_bounds__((YiShape<NY, false>::NT), (YiShape<NY, false>::IL ?
         v[e] = wn;
     }
     if (!finite && a.bad) a.bad[blockIdx.y] = 1;
-    if constexpr (!rf_final_is_first<NY, csh_yem(NY)>()) rf_final_to_first<NY, csh_yem(NY)>(v, t, xl);
+    rf_final_to_first<NY, csh_yem(NY)>(v, t, xl);
     csh_yinv_column<NY, false, GS, S::IL>(v, i, live, t, xl, tw, 0.0, ld, g0, g1, g2, g3);
 }
 

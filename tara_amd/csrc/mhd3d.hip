@@ -8,19 +8,36 @@
 //
 // Five sweeps per right-hand side (device layout: kx-fastest, row length
 // padded to ld = Nh rounded up to 8; element (i, j, k) at (k*Ny + j)*ld + i):
-//   1 k_col_fft (z, backward)  state (7 fields) -> A, tiles of 8 kx columns
-//   2 k_col_fft (y, backward)  A in place
+//   1 k_col_fft (z, backward)  state (7 fields) -> Az, tiles of 8 kx columns
+//   2 k_col_fft (y, backward)  Az -> A
 //   3 k_mhd_x                  per x row: 7 c2r as 4 paired complex FFTs,
-//                              u = rho u / rho, P, B^2 and the 14 live fluxes
-//                              (derive3com.f95:176-186, 395-436), 7 paired
-//                              forward FFTs -> B (14 fields)
+//                              u = rho u / rho, P, B^2 and the 12 distinct live
+//                              fluxes (derive3com.f95:176-186, 395-436), 6
+//                              paired forward FFTs -> B (12 fields)
 //   4 k_col_fft (y, forward)   B in place
-//   5 k_mhd_zfwd               z forward of the 14 fields, i k . flux, k^2
+//   5 k_mhd_zfwd               z forward of the 12 fields, i k . flux, k^2
 //                              diffusion, spherical dealias on all terms
 //                              (derive3com.f95:574-843), assembly
-//                              (:1018-1037), then RHS out or AB2 in place.
+//                              (:1018-1037), then RHS out, or AB2 in place and
+//                              the inverse z transform of the new state -> Az.
 // The diffusion coefficients are parameters (the reference hard-wires 1/450,
 // derive3com.f95:1023-1037).
+//
+// The dealiasing zeroes every term of every field outside the sphere
+// k < (Nx+Ny+Nz)/9, so a mode outside it never changes: at 256^3 in a 2 pi box
+// 14 % of the modes live, in 35 % of the z columns and 86 of 129 kx columns.
+//   - Sweeps 3 to 5 carry only what a live mode reads: x writes the kx tiles that
+//     hold one, y transforms them and stores the rows that hold one, z runs over
+//     the tiles that hold one.
+//   - Within one advance call the inverse transform of the rest is the same at
+//     every step: sweep 1 runs once, sweep 5 replaces the live tiles of Az, and
+//     sweep 2 redoes the kx tiles that hold a live mode (the others' A stays).
+// Mom_x_3 = Mom_z_1 and Mom_y_3 = Mom_z_2 (the same products in another order)
+// are formed once.  Per step, in half spectra of 16 Nh Ny Nz bytes at 256^3:
+// 9.4 (y) + 15 (x) + 13.6 (y) + 14 (z) = 52, against 119 when every sweep carried
+// every mode and 14 fluxes; 3.72 -> 1.65 ms (0.25 + 0.57 + 0.33 + 0.46 ms; the
+// first step of a call adds 0.5 ms).
+#include <algorithm>
 #include <cmath>
 
 #include "mhd3d.h"
@@ -43,9 +60,10 @@ struct MXShape {
 
 struct XArgs {
     const double2* a;  // 7 inverse-transformed fields, field stride fs
-    double2* b;        // 14 flux fields
+    double2* b;        // 12 flux fields
     size_t fs;
     int ld;
+    int nk;            // kx columns of the fluxes that are kept
     double norm;       // 1 / (Nx Ny Nz)
     double cs2;
 };
@@ -106,9 +124,9 @@ __global__ __launch_bounds__(256, 3) void k_mhd_x(XArgs x, const double2* tw)
         pp[e] = x.cs2 * rho;
         hb2[e] = (pr[4][e] * pr[4][e] + pr[5][e] * pr[5][e] + pr[6][e] * pr[6][e]) / 2.0;
     }
-    // forward pairs: (ux, uy) (uz, MX1) (MX2, MX3) (MY2, MY3) (MZ1, MZ2) (MZ3, MG1) (MG2, MG3)
+    // forward pairs: (ux, uy) (uz, MXX) (MXY, MXZ) (MYY, MYZ) (MZZ, MG1) (MG2, MG3)
 #pragma unroll 1
-    for (int p = 0; p < 7; ++p) {
+    for (int p = 0; p < 6; ++p) {
         double2 v[E];
 #pragma unroll
         for (int e = 0; e < E; ++e) {
@@ -120,8 +138,7 @@ __global__ __launch_bounds__(256, 3) void k_mhd_x(XArgs x, const double2* tw)
                 case 1: f0 = uz[e]; f1 = rux * ux[e] + pp[e] + hb2[e] - bx * bx; break;
                 case 2: f0 = rux * uy[e] - bx * by; f1 = rux * uz[e] - bx * bz; break;
                 case 3: f0 = ruy * uy[e] + pp[e] + hb2[e] - by * by; f1 = ruy * uz[e] - by * bz; break;
-                case 4: f0 = ruz * ux[e] - bz * bx; f1 = ruz * uy[e] - bz * by; break;
-                case 5: f0 = ruz * uz[e] + pp[e] + hb2[e] - bz * bz; f1 = ux[e] * by - uy[e] * bx; break;
+                case 4: f0 = ruz * uz[e] + pp[e] + hb2[e] - bz * bz; f1 = ux[e] * by - uy[e] * bx; break;
                 default: f0 = ux[e] * bz - uz[e] * bx; f1 = uy[e] * bz - uz[e] * by; break;
             }
             v[e] = make_double2(f0, f1);
@@ -133,7 +150,7 @@ __global__ __launch_bounds__(256, 3) void k_mhd_x(XArgs x, const double2* tw)
         rf_sync<true>();
         double2* oa = x.b + (size_t)(2 * p) * x.fs + ro;
         double2* ob = x.b + (size_t)(2 * p + 1) * x.fs + ro;
-        for (int k = t; k <= M; k += T) {
+        for (int k = t; k < x.nk; k += T) {
             const double2 z = xl[rf_pad(k)], zm = xl[rf_pad(k == 0 ? 0 : NX - k)];
             oa[k] = make_double2(0.5 * (z.x + zm.x), 0.5 * (z.y - zm.y));
             ob[k] = make_double2(0.5 * (z.y + zm.y), -0.5 * (z.x - zm.x));
@@ -144,28 +161,39 @@ __global__ __launch_bounds__(256, 3) void k_mhd_x(XArgs x, const double2* tw)
 
 // ----------------------------------------------------- z forward + assembly
 struct ZArgs {
-    const double2* b;  // 14 flux fields after the y pass
+    const double2* b;      // 12 flux fields after the y pass
     size_t fs;
-    double2* st[7];    // state (rho, rho ux, rho uy, rho uz, Bx, By, Bz)
-    double2* out[7];   // RHS (MHD_RHS) or history f_{n-1} -> f_n (MHD_AB2)
+    const double2* st[7];  // state (rho, rho ux, rho uy, rho uz, Bx, By, Bz)
+    double2* sn[7];        // MHD_AB2: new state; for rho and B the same fields as st
+    double2* out[7];       // RHS (MHD_RHS) or history f_{n-1} -> f_n (MHD_AB2)
+    double2* az;           // with INV: 7 fields, the new state's inverse z transform
     const double* kx;
     const double* ky;
     const double* kz;
-    const int* imin;   // per (k, j) row: modes with i >= imin are dealiased away
+    const int* imin;       // per (k, j) row: modes with i >= imin are dealiased away
+    const int* live;       // tiles j*(ld/8) + x that hold a live mode
     int ny, ld;
     double mu, eta, dt;
-    int* bad;          // AB2: set to 1 when a new state value is not finite
+    int* bad;              // AB2: set to 1 when a new state value is not finite
 };
 
-// The z pass holds 14 transforms' worth of accumulators; at 4 elements per
-// thread and a bound of 4 waves per SIMD (128 VGPRs, two 512-thread workgroups
-// per CU) it ran 1.48 ms at 256^3, against 1.85 ms at 8 elements per thread
-// (256 VGPRs, one 256-thread workgroup per CU) and 1.57 ms unbounded.  The AB2
-// form's opaque slot index took it to 1.44 ms (spill 84 -> 28 bytes per lane),
-// forming the density term from the momentum loads of the updates to 1.38 ms
-// (110 VGPRs, no spill, 3 fields fewer read).
+// Flux fields of B, in the x pass's order.
+enum MhdFlux { FUX, FUY, FUZ, FXX, FXY, FXZ, FYY, FYZ, FZZ, FG1, FG2, FG3 };
+
+// One state field of one tile of 8 kx columns of one ky row per workgroup, 4
+// elements per thread; the seven fields of a tile run next to each other on one
+// XCD, which serves the fluxes that two of them read from its L2.
+// Bound by its memory traffic: 1.9 GB in 0.46 ms at 256^3 (4.1 TB/s).  One
+// workgroup for all seven fields of a tile reads each flux once, but needs three
+// accumulators beside the density's and spilled 42-63 registers per lane at the
+// 128 that four waves per SIMD allow; split by field nothing spills (123 at
+// most), a thread's chain is at most 4 + 1 transforms instead of 12 + 7, and
+// small grids fill the chip (64^3: 33.6 -> 13.0 us, with the inverse transform
+// that was a kernel of its own before).
+// The density's right-hand side needs the momentum of the step's start, which
+// other workgroups update: the new momentum goes to other buffers (sn).
 constexpr int kZfwdEM = 4;
-template <int NZ, int MODE, int EM>
+template <int NZ, int MODE, bool INV, int EM>
 __global__ __launch_bounds__((CShape<NZ, EM>::NT), 4) void k_mhd_zfwd(ZArgs a, const double2* tw)
 {
     using S = CShape<NZ, EM>;
@@ -173,152 +201,99 @@ __global__ __launch_bounds__((CShape<NZ, EM>::NT), 4) void k_mhd_zfwd(ZArgs a, c
     __shared__ double2 lds[8 * S::LP];
     const int c = threadIdx.x % 8, t = threadIdx.x / 8;
     const int tpp = a.ld / 8;
-    const int tile = xcd_remap(blockIdx.x, gridDim.x);
+    const int id = xcd_remap(blockIdx.x, gridDim.x);
+    const int tile = a.live[id / 7], fld = id % 7;
     const int j = tile / tpp, i = (tile % tpp) * 8 + c;
     const size_t base = (size_t)j * a.ld + i, es = (size_t)a.ny * a.ld;
     double2* xl = lds + c * S::LP;
     const double kxv = a.kx[i], kyv = a.ky[j];
-    bool keep[E];
     double kzv[E], k2[E];
-    size_t q[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-        const int k = rf_final_idx<NZ, EM>(t, e);
-        q[e] = base + (size_t)k * es;
-        kzv[e] = a.kz[k];
+        kzv[e] = a.kz[rf_final_idx<NZ, EM>(t, e)];
         k2[e] = (kxv * kxv + kyv * kyv) + kzv[e] * kzv[e];
-        keep[e] = i < a.imin[(size_t)k * a.ny + j];
     }
-    auto zfft = [&](int f, double2 (&v)[E]) {
-        const double2* src = a.b + (size_t)f * a.fs + base;
-        // AB2: the slot index is made opaque per transform so that the index
-        // arithmetic is redone here rather than held across all 14 transforms
-        // (110 VGPRs against 124); the RHS form spills more that way and keeps
-        // it.
-        const int tt = MODE == MHD_AB2 ? rf_opaque(t) : t;
-#pragma unroll
-        for (int e = 0; e < E; ++e) v[e] = src[(size_t)rf_first_idx<NZ, EM>(tt, e) * es];
-        rf_fft<NZ, -1, EM>(v, tt, xl, tw);
-    };
     // i k z = (-k z.y, k z.x)
     auto ik = [](double kk, double2 z) { return make_double2(-(kk * z.y), kk * z.x); };
-    // AB2: dens accumulates the density term -(i kx rho ux + i ky rho uy +
-    // i kz rho uz) from the momentum state that the updates of fields 1..3 load
-    // anyway, so the momentum spectra are read once (not again for the density
-    // term before the 14 transforms); density is finished after field 3.
-    double2 dens[E];
-    bool finite = true;  // AB2: every new state value of this lane is finite
-    // wpre: the state of field fld at this lane's positions when the caller
-    // has already loaded it (AB2), else null.
-    auto finish = [&](int fld, const double2 (&acc)[E], const double2* wpre = nullptr) {
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
-            const double2 f = keep[e] ? acc[e] : make_double2(0.0, 0.0);
-            if (MODE == MHD_RHS) {
-                a.out[fld][q[e]] = f;
-            } else {
-                const double2 fo = a.out[fld][q[e]], w = wpre ? wpre[e] : a.st[fld][q[e]];
-                if (fld == 1) dens[e] = ik(kxv, w);
-                if (fld == 2) { const double2 s2 = ik(kyv, w); dens[e] = make_double2(dens[e].x + s2.x, dens[e].y + s2.y); }
-                if (fld == 3) { const double2 s3 = ik(kzv[e], w); dens[e] = make_double2(dens[e].x + s3.x, dens[e].y + s3.y); }
-                const double2 wn = make_double2(w.x + (1.5 * f.x - 0.5 * fo.x) * a.dt, w.y + (1.5 * f.y - 0.5 * fo.y) * a.dt);
-                a.st[fld][q[e]] = wn;
-                a.out[fld][q[e]] = f;
-                finite = finite && isfinite(wn.x) && isfinite(wn.y);
-            }
-        }
-    };
-    double2 v[E], acc[E], acc2[E];
-    if (MODE == MHD_RHS) {
+    auto zk = [&](int e) { return base + (size_t)rf_final_idx<NZ, EM>(t, e) * es; };
+    double2 acc[E];
+    if (fld == 0) {
         // density: -(i kx rho ux + i ky rho uy + i kz rho uz) on the state spectra
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            const double2 s1 = ik(kxv, a.st[1][q[e]]), s2 = ik(kyv, a.st[2][q[e]]), s3 = ik(kzv[e], a.st[3][q[e]]);
+            const size_t q = zk(e);
+            const double2 s1 = ik(kxv, a.st[1][q]), s2 = ik(kyv, a.st[2][q]), s3 = ik(kzv[e], a.st[3][q]);
             acc[e] = make_double2(-((s1.x + s2.x) + s3.x), -((s1.y + s2.y) + s3.y));
         }
-        finish(0, acc);
+    } else {
+        // a sum of terms +-i k_d flux over directions d: momentum row r takes
+        // -mu k^2 u_r - i k . (row r of the symmetric flux tensor); the induction
+        // dBx = i ky MG1 + i kz MG2, dBy = -i kx MG1 + i kz MG3,
+        // dBz = -i kx MG2 - i ky MG3 (src/derive3com.f95:1030-1037)
+        const bool mom = fld < 4;
+        const int r = (fld - 1) % 3;
+#pragma unroll
+        for (int e = 0; e < E; ++e) acc[e] = make_double2(0.0, 0.0);
+#pragma unroll 1
+        for (int m = mom ? -1 : 0; m < 3; ++m) {
+            // induction: direction r has no term in row r; the flux of rows r and
+            // m is MG(r + m), its sign minus below the diagonal
+            if (!mom && m == r) continue;
+            int f;
+            if (m < 0)
+                f = FUX + r;
+            else if (mom)
+                f = FXX + (r + m) + (r && m ? 1 : 0);
+            else
+                f = FG1 + r + m - 1;
+            const double2* src = a.b + (size_t)f * a.fs + base;
+            double2 v[E];
+#pragma unroll
+            for (int e = 0; e < E; ++e) v[e] = src[(size_t)rf_first_idx<NZ, EM>(t, e) * es];
+            rf_fft<NZ, -1, EM>(v, t, xl, tw);
+            const double sg = mom || m < r ? -1.0 : 1.0;
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const double kd = sg * (m == 0 ? kxv : m == 1 ? kyv : kzv[e]);
+                const double2 d = m < 0 ? make_double2(-(a.mu * k2[e] * v[e].x), -(a.mu * k2[e] * v[e].y)) : ik(kd, v[e]);
+                acc[e] = make_double2(acc[e].x + d.x, acc[e].y + d.y);
+            }
+        }
     }
-    // rho ux: -(i k . (MX1, MX2, MX3)) - mu k^2 ux; MX2 also feeds rho uy (Mom_y_1 == Mom_x_2)
-    zfft(0, v);
-#pragma unroll
-    for (int e = 0; e < E; ++e) acc[e] = make_double2(-(a.mu * k2[e] * v[e].x), -(a.mu * k2[e] * v[e].y));
-    zfft(3, v);
-#pragma unroll
-    for (int e = 0; e < E; ++e) { const double2 d = ik(kxv, v[e]); acc[e].x -= d.x; acc[e].y -= d.y; }
-    zfft(4, v);
+    // f = acc (- eta k^2 state for the components of B), masked; stored as the
+    // RHS, or taken into the AB2 update, whose new state goes on through the
+    // inverse z transform.  A masked mode's f and history are zero: its state is
+    // read for the transform only.
+    const double2* st = a.st[fld];
+    double2* out = a.out[fld];
+    bool finite = true;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-        const double2 d = ik(kyv, v[e]), g = ik(kxv, v[e]);
-        acc[e].x -= d.x;
-        acc[e].y -= d.y;
-        acc2[e] = make_double2(-g.x, -g.y);
+        const size_t q = zk(e);
+        const bool keep = i < a.imin[(size_t)rf_final_idx<NZ, EM>(t, e) * a.ny + j];
+        double2 f = acc[e], w = make_double2(0.0, 0.0);
+        if (MODE == MHD_AB2 || fld >= 4) w = st[q];
+        if (fld >= 4) f = make_double2(f.x - a.eta * k2[e] * w.x, f.y - a.eta * k2[e] * w.y);
+        if (!keep) f = make_double2(0.0, 0.0);
+        if (MODE == MHD_RHS) {
+            out[q] = f;
+        } else if (keep) {
+            const double2 fo = out[q];
+            w = make_double2(w.x + (1.5 * f.x - 0.5 * fo.x) * a.dt, w.y + (1.5 * f.y - 0.5 * fo.y) * a.dt);
+            a.sn[fld][q] = w;
+            out[q] = f;
+            finite = finite && isfinite(w.x) && isfinite(w.y);
+        }
+        acc[e] = w;
     }
-    zfft(5, v);
-#pragma unroll
-    for (int e = 0; e < E; ++e) { const double2 d = ik(kzv[e], v[e]); acc[e].x -= d.x; acc[e].y -= d.y; }
-    finish(1, acc);
-    // rho uy: acc2 holds -i kx MY1; add -i ky MY2 - i kz MY3 - mu k^2 uy
-    zfft(1, v);
-#pragma unroll
-    for (int e = 0; e < E; ++e) { acc2[e].x -= a.mu * k2[e] * v[e].x; acc2[e].y -= a.mu * k2[e] * v[e].y; }
-    zfft(6, v);
-#pragma unroll
-    for (int e = 0; e < E; ++e) { const double2 d = ik(kyv, v[e]); acc2[e].x -= d.x; acc2[e].y -= d.y; }
-    zfft(7, v);
-#pragma unroll
-    for (int e = 0; e < E; ++e) { const double2 d = ik(kzv[e], v[e]); acc2[e].x -= d.x; acc2[e].y -= d.y; }
-    finish(2, acc2);
-    // rho uz
-    zfft(2, v);
-#pragma unroll
-    for (int e = 0; e < E; ++e) acc[e] = make_double2(-(a.mu * k2[e] * v[e].x), -(a.mu * k2[e] * v[e].y));
-    zfft(8, v);
-#pragma unroll
-    for (int e = 0; e < E; ++e) { const double2 d = ik(kxv, v[e]); acc[e].x -= d.x; acc[e].y -= d.y; }
-    zfft(9, v);
-#pragma unroll
-    for (int e = 0; e < E; ++e) { const double2 d = ik(kyv, v[e]); acc[e].x -= d.x; acc[e].y -= d.y; }
-    zfft(10, v);
-#pragma unroll
-    for (int e = 0; e < E; ++e) { const double2 d = ik(kzv[e], v[e]); acc[e].x -= d.x; acc[e].y -= d.y; }
-    finish(3, acc);
-    if (MODE == MHD_AB2) {
-#pragma unroll
-        for (int e = 0; e < E; ++e) acc[e] = make_double2(-dens[e].x, -dens[e].y);
-        finish(0, acc);
-    }
-    // induction: dBx = i ky MG1 + i kz MG2, dBy = -i kx MG1 + i kz MG3,
-    // dBz = -i kx MG2 - i ky MG3, each minus eta k^2 B (src/derive3com.f95:1030-1037)
-    zfft(11, v);  // MG1
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-        acc[e] = ik(kyv, v[e]);
-        const double2 g = ik(kxv, v[e]);
-        acc2[e] = make_double2(-g.x, -g.y);
-    }
-    zfft(12, v);  // MG2
-    double2 acc3[E], bs[E];  // bs: the B component just loaded, reused by its update
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const double2 d = ik(kzv[e], v[e]), g = ik(kxv, v[e]);
-        bs[e] = a.st[4][q[e]];
-        acc[e] = make_double2((acc[e].x + d.x) - a.eta * k2[e] * bs[e].x, (acc[e].y + d.y) - a.eta * k2[e] * bs[e].y);
-        acc3[e] = make_double2(-g.x, -g.y);
-    }
-    finish(4, acc, bs);
-    zfft(13, v);  // MG3
-    double2 bz[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const double2 d = ik(kzv[e], v[e]), g = ik(kyv, v[e]);
-        bs[e] = a.st[5][q[e]];
-        bz[e] = a.st[6][q[e]];
-        acc2[e] = make_double2((acc2[e].x + d.x) - a.eta * k2[e] * bs[e].x, (acc2[e].y + d.y) - a.eta * k2[e] * bs[e].y);
-        acc3[e] = make_double2((acc3[e].x - g.x) - a.eta * k2[e] * bz[e].x, (acc3[e].y - g.y) - a.eta * k2[e] * bz[e].y);
-    }
-    finish(5, acc2, bs);
-    finish(6, acc3, bz);
     if (MODE == MHD_AB2 && !finite && a.bad) a.bad[0] = 1;
+    if constexpr (INV) {
+        rf_final_to_first<NZ, EM>(acc, t, xl);
+        rf_fft<NZ, +1, EM>(acc, t, xl, tw);
+        double2* dst = a.az + (size_t)fld * a.fs;
+#pragma unroll
+        for (int e = 0; e < E; ++e) dst[zk(e)] = acc[e];
+    }
 }
 
 // ------------------------------------------------------------------ dispatch
@@ -363,20 +338,21 @@ static int launch_x(const MhdPlan& p, const XArgs& x, hipStream_t st)
 static int xpass(const MhdPlan& p, const XArgs& x, hipStream_t st) { TARA_MHD_SWITCH(p.nx, launch_x, p, x, st) }
 
 template <int NZ>
-static int launch_z(const MhdPlan& p, int mode, const ZArgs& z, hipStream_t st)
+static int launch_z(const MhdPlan& p, int mode, bool inv, const ZArgs& z, hipStream_t st)
 {
     constexpr int EM = kZfwdEM;
-    dim3 g(p.ny * (p.ld / 8)), b(CShape<NZ, EM>::NT);
-    const double2* tw = EM == 4 ? p.tw_z4 : p.tw_z;
+    dim3 g(7 * p.nlive), b(CShape<NZ, EM>::NT);
     if (mode == MHD_RHS)
-        hipLaunchKernelGGL((k_mhd_zfwd<NZ, MHD_RHS, EM>), g, b, 0, st, z, tw);
+        hipLaunchKernelGGL((k_mhd_zfwd<NZ, MHD_RHS, false, EM>), g, b, 0, st, z, p.tw_z4);
+    else if (inv)
+        hipLaunchKernelGGL((k_mhd_zfwd<NZ, MHD_AB2, true, EM>), g, b, 0, st, z, p.tw_z4);
     else
-        hipLaunchKernelGGL((k_mhd_zfwd<NZ, MHD_AB2, EM>), g, b, 0, st, z, tw);
+        hipLaunchKernelGGL((k_mhd_zfwd<NZ, MHD_AB2, false, EM>), g, b, 0, st, z, p.tw_z4);
     return TARA_OK;
 }
-static int zpass(const MhdPlan& p, int mode, const ZArgs& z, hipStream_t st)
+static int zpass(const MhdPlan& p, int mode, bool inv, const ZArgs& z, hipStream_t st)
 {
-    TARA_MHD_SWITCH(p.nz, launch_z, p, mode, z, st)
+    TARA_MHD_SWITCH(p.nz, launch_z, p, mode, inv, z, st)
 }
 
 // ------------------------------------------------------------------ host side
@@ -400,7 +376,7 @@ int mhd_plan_init(MhdPlan& p, int nx, int ny, int nz, double lx, double ly, doub
     p.cs = cs;
     p.fsz = (size_t)p.ld * ny * nz;
     int rc;
-    if ((rc = p.a.alloc(7 * p.fsz * sizeof(double2))) || (rc = p.b.alloc(14 * p.fsz * sizeof(double2)))) return rc;
+    if ((rc = p.a.alloc(7 * p.fsz * sizeof(double2))) || (rc = p.b.alloc(12 * p.fsz * sizeof(double2)))) return rc;
     TARA_HIP(hipMemset(p.a.p, 0, p.a.bytes));
     TARA_HIP(hipMemset(p.b.p, 0, p.b.bytes));
     // wavenumbers as derive3com forms them: 2 pi (i-1)/L with true pi
@@ -427,6 +403,29 @@ int mhd_plan_init(MhdPlan& p, int nx, int ny, int nz, double lx, double ly, doub
         (rc = p.kz.alloc(nz * sizeof(double))) || (rc = p.imin.alloc(imin.size() * sizeof(int))) ||
         (rc = p.bad.alloc(sizeof(int))))
         return rc;
+    // live tiles: imin is largest at the smallest |kz|, but every k is looked at
+    const int tpp = p.ld / 8;
+    std::vector<int> width(ny, 0), live;
+    for (int k = 0; k < nz; ++k)
+        for (int j = 0; j < ny; ++j) width[j] = std::max(width[j], imin[(size_t)k * ny + j]);
+    for (int j = 0; j < ny; ++j) {
+        const int nt = (width[j] + 7) / 8;
+        p.ktiles = std::max(p.ktiles, nt);
+        for (int x = 0; x < nt; ++x) live.push_back(j * tpp + x);
+    }
+    p.nlive = (int)live.size();  // at least the tile of k = 0, since the cut is positive
+    // rows of a kx tile without a live mode: |ky| grows towards the middle, so
+    // they are one run [lo, hi)
+    std::vector<int2> yskip(p.ktiles);
+    for (int x = 0; x < p.ktiles; ++x) {
+        int lo = 0, hi = ny;
+        while (lo < ny && width[lo] > 8 * x) ++lo;
+        while (hi > lo && width[hi - 1] > 8 * x) --hi;
+        yskip[x] = make_int2(lo, hi);
+    }
+    if ((rc = p.live.alloc(live.size() * sizeof(int))) || (rc = p.yskip.alloc(yskip.size() * sizeof(int2)))) return rc;
+    TARA_HIP(hipMemcpy(p.live.p, live.data(), live.size() * sizeof(int), hipMemcpyHostToDevice));
+    TARA_HIP(hipMemcpy(p.yskip.p, yskip.data(), yskip.size() * sizeof(int2), hipMemcpyHostToDevice));
     TARA_HIP(hipMemset(p.bad.p, 0, sizeof(int)));
     TARA_HIP(hipMemcpy(p.kx.p, kx.data(), p.ld * sizeof(double), hipMemcpyHostToDevice));
     TARA_HIP(hipMemcpy(p.ky.p, ky.data(), ny * sizeof(double), hipMemcpyHostToDevice));
@@ -440,61 +439,122 @@ int mhd_plan_init(MhdPlan& p, int nx, int ny, int nz, double lx, double ly, doub
     return TARA_OK;
 }
 
-int mhd_rhs_stage(const MhdPlan& p, double2* const st[7], int mode, double dt, double2* const out[7],
-                  double2* const hist[7], hipStream_t s, EventTimer* tm)
+int mhd_plan_stepping(MhdPlan& p) { return p.az.alloc(7 * p.fsz * sizeof(double2)); }
+
+namespace {
+
+// Backward z of every column: fields src -> dst (7 fields, stride fsz).
+int inverse_z(const MhdPlan& p, double2* const src[7], double2* dst, hipStream_t s)
 {
-    int rc;
-    double2* A = p.a.as<double2>();
-    double2* B = p.b.as<double2>();
-    const int tpp = p.ld / 8;
     ColArgs c{};
-    // 1: z backward, state -> A
     for (int f = 0; f < 7; ++f) {
-        c.src[f] = st[f];
-        c.dst[f] = A + f * p.fsz;
+        c.src[f] = src[f];
+        c.dst[f] = dst + f * p.fsz;
     }
     c.es = (long)p.ny * p.ld;
     c.pstride = p.ld;
-    c.tpp = tpp;
-    if (tm) tm->begin(0, s);
-    if ((rc = col(p.nz, c, p.ny * tpp, 7, +1, p.tw_z, s))) return rc;
-    // 2: y backward in place
-    for (int f = 0; f < 7; ++f) c.src[f] = c.dst[f] = A + f * p.fsz;
+    c.tpp = p.ld / 8;
+    return col(p.nz, c, p.ny * c.tpp, 7, +1, p.tw_z, s);
+}
+
+// Backward y of the first ktiles kx tiles of every plane: 7 fields src -> dst.
+int inverse_y(const MhdPlan& p, const double2* src, double2* dst, int ktiles, hipStream_t s)
+{
+    ColArgs c{};
+    for (int f = 0; f < 7; ++f) {
+        c.src[f] = src + f * p.fsz;
+        c.dst[f] = dst + f * p.fsz;
+    }
     c.es = p.ld;
     c.pstride = (long)p.ny * p.ld;
-    if ((rc = col(p.ny, c, p.nz * tpp, 7, +1, p.tw_y, s))) return rc;
-    if (tm) tm->end(0, s);
-    // 3: x pass
-    XArgs x{A, B, p.fsz, p.ld, 1.0 / ((double)p.nx * (double)p.ny * (double)p.nz), p.cs * p.cs};
+    c.tpp = ktiles;
+    return col(p.ny, c, p.nz * ktiles, 7, +1, p.tw_y, s);
+}
+
+// x pass A -> B and the forward y transform of B's 12 fields.
+int x_and_y(const MhdPlan& p, hipStream_t s, EventTimer* tm)
+{
+    int rc;
+    double2* B = p.b.as<double2>();
+    XArgs x{p.a.as<double2>(), B, p.fsz, p.ld, std::min(p.nh, 8 * p.ktiles),
+            1.0 / ((double)p.nx * (double)p.ny * (double)p.nz), p.cs * p.cs};
     if (tm) tm->begin(1, s);
     if ((rc = xpass(p, x, s))) return rc;
     if (tm) tm->end(1, s);
-    // 4: y forward in place on the 14 flux fields
-    for (int f = 0; f < 14; ++f) c.src[f] = c.dst[f] = B + f * p.fsz;
+    ColArgs c{};
+    for (int f = 0; f < 12; ++f) c.src[f] = c.dst[f] = B + f * p.fsz;
+    c.es = p.ld;
+    c.pstride = (long)p.ny * p.ld;
+    c.tpp = p.ktiles;
+    c.skip = p.yskip.as<int2>();
     if (tm) tm->begin(2, s);
-    if ((rc = col(p.ny, c, p.nz * tpp, 14, -1, p.tw_y, s))) return rc;
+    if ((rc = col(p.ny, c, p.nz * p.ktiles, 12, -1, p.tw_y, s))) return rc;
     if (tm) tm->end(2, s);
-    // 5: z forward + assembly + update
+    return TARA_OK;
+}
+
+ZArgs zargs(const MhdPlan& p, double2* const st[7], double2* const sn[7], double2* const out[7], double dt)
+{
     ZArgs z{};
-    z.b = B;
+    z.b = p.b.as<double2>();
     z.fs = p.fsz;
     for (int f = 0; f < 7; ++f) {
         z.st[f] = st[f];
-        z.out[f] = mode == MHD_RHS ? out[f] : hist[f];
+        z.sn[f] = sn[f];
+        z.out[f] = out[f];
     }
+    z.az = p.az.as<double2>();
     z.kx = p.kx.as<double>();
     z.ky = p.ky.as<double>();
     z.kz = p.kz.as<double>();
     z.imin = p.imin.as<int>();
+    z.live = p.live.as<int>();
     z.ny = p.ny;
     z.ld = p.ld;
     z.mu = p.mu;
     z.eta = p.eta;
     z.dt = dt;
     z.bad = p.bad.as<int>();
+    return z;
+}
+
+}  // namespace
+
+int mhd_rhs_stage(const MhdPlan& p, double2* const st[7], double2* const out[7], hipStream_t s, EventTimer* tm)
+{
+    int rc;
+    double2* A = p.a.as<double2>();
+    if (tm) tm->begin(0, s);
+    if ((rc = inverse_z(p, st, A, s)) || (rc = inverse_y(p, A, A, p.ld / 8, s))) return rc;
+    if (tm) tm->end(0, s);
+    if ((rc = x_and_y(p, s, tm))) return rc;
     if (tm) tm->begin(3, s);
-    if ((rc = zpass(p, mode, z, s))) return rc;
+    if ((rc = zpass(p, MHD_RHS, false, zargs(p, st, st, out, 0.0), s))) return rc;
     if (tm) tm->end(3, s);
+    TARA_HIP(hipGetLastError());
+    return TARA_OK;
+}
+
+int mhd_advance(const MhdPlan& p, double2* st[7], double2* mom[3], double2* const hist[7], int nsteps, double dt,
+                hipStream_t s, EventTimer* tm)
+{
+    if (nsteps <= 0) return TARA_OK;
+    int rc;
+    TARA_CHECK(p.az.p, TARA_ERR_STATE, "3D MHD: plan without its stepping work space");
+    for (int k = 0; k < nsteps; ++k) {
+        if (tm) tm->begin(0, s);
+        if (k == 0 && (rc = inverse_z(p, st, p.az.as<double2>(), s))) return rc;
+        // the first step fills all of A; later only the kx tiles with a live mode change
+        if ((rc = inverse_y(p, p.az.as<double2>(), p.a.as<double2>(), k == 0 ? p.ld / 8 : p.ktiles, s))) return rc;
+        if (tm) tm->end(0, s);
+        if ((rc = x_and_y(p, s, tm))) return rc;
+        double2* sn[7];
+        for (int f = 0; f < 7; ++f) sn[f] = f >= 1 && f <= 3 ? mom[f - 1] : st[f];
+        if (tm) tm->begin(3, s);
+        if ((rc = zpass(p, MHD_AB2, k + 1 < nsteps, zargs(p, st, sn, hist, dt), s))) return rc;
+        if (tm) tm->end(3, s);
+        for (int f = 0; f < 3; ++f) std::swap(st[1 + f], mom[f]);
+    }
     TARA_HIP(hipGetLastError());
     return TARA_OK;
 }

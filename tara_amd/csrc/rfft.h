@@ -236,12 +236,21 @@ __device__ __forceinline__ void rf_fft_barriers_only()
     for (int b = 0; b < nb; ++b) __syncthreads();
 }
 
+// Whether a thread's output positions are its input positions: every pass has
+// the full radix E (N a power of E).
+template <int N, int EM>
+constexpr bool rf_final_is_first()
+{
+    return fft_radix(N, RF<N, EM>::E) == RF<N, EM>::E && N / rf_last_span(N, RF<N, EM>::E) == RF<N, EM>::E;
+}
+
 // Reorders registers from final (output) positions to first-pass (input)
 // positions through LDS, e.g. to feed a transform's output into another
-// transform of the same length.
+// transform of the same length.  Nothing to do where the two are the same.
 template <int N, int EM = 8, bool WAVE = false>
 __device__ __forceinline__ void rf_final_to_first(double2 (&v)[(RF<N, EM>::E)], int t, double2* lds)
 {
+    if constexpr (rf_final_is_first<N, EM>()) return;
     constexpr int E = RF<N, EM>::E;
 #pragma unroll
     for (int e = 0; e < E; ++e) lds[rf_pad(rf_final_idx<N, EM>(t, e))] = v[e];
