@@ -134,6 +134,11 @@ int derive_dropin(const char* name, int nx, int ny, int nh, const CshPhys& ph, c
     const CshPlan& p = d->plan;
     const size_t bytes = (size_t)nh * ny * sizeof(double2);
     TARA_HIP(hipMemcpy(d->stage.p, omegak, bytes, hipMemcpyHostToDevice));
+    if (csh_small(p)) {
+        if ((rc = csh_rhs_direct(p, d->stage.as<double2>(), d->f.as<double2>(), ph, nullptr))) return rc;
+        TARA_HIP(hipMemcpy(dt_new, d->f.p, bytes, hipMemcpyDeviceToHost));
+        return TARA_OK;
+    }
     if ((rc = to_kymajor(d->stage.as<double2>(), d->w.as<double2>(), nh, ny, 1, nullptr))) return rc;
     rc = csh_rhs_stage(p, d->w.as<double2>(), CSH_RHS, ph, 0.0, nullptr, nullptr, d->f.as<double2>(), nullptr,
                        nullptr);
@@ -347,7 +352,7 @@ extern "C" int tara_csh_advance(tara_csh* c, int nsteps)
     double2* aux = c->aux.as<double2>();
     double2* nx = c->next.as<double2>();
     EventTimer* tm = c->tm.get();
-    if (!c->ph.screened) return csh_advance(c->plan, c->scheme, nsteps, c->ph, c->dt, w, aux, nx, c->st, tm);
+    if (csh_fused(c->plan, c->ph)) return csh_advance(c->plan, c->scheme, nsteps, c->ph, c->dt, w, aux, nx, c->st, tm);
     for (int s = 0; s < nsteps; ++s) {
         int rc;
         if (c->scheme == TARA_SCHEME_AB2) {

@@ -110,8 +110,8 @@ int csh_advance(const CshPlan& p, int scheme, int nsteps, const CshPhys& ph, dou
 // and one step that expects G0..G3 to hold it (x pass, fused forward + inverse
 // y pass per stage; plain_last: the last stage's forward y pass alone, else
 // G0..G3 are left holding the inverse y pass of the new state).  For Ny < 1024
-// the passes are not fused: csh_yinv_pass does nothing and the step runs
-// csh_rhs_stage per stage.
+// and enough columns to fill the chip the passes are not fused: csh_yinv_pass
+// does nothing and the step runs csh_rhs_stage per stage.
 int csh_yinv_pass(const CshPlan& p, const double2* w, const CshPhys& ph, hipStream_t st);
 int csh_fused_step(const CshPlan& p, int scheme, const CshPhys& ph, double dt, double2* w, double2* aux,
                    double2* next, bool plain_last, hipStream_t st, EventTimer* tm);
@@ -120,9 +120,28 @@ int csh_fused_step(const CshPlan& p, int scheme, const CshPhys& ph, double dt, d
 // 1 x pass, 2 forward y + update.
 int csh_rhs_stage(const CshPlan& p, const double2* ws, int mode, const CshPhys& ph, double dt, double2* base,
                   double2* aux, double2* next, hipStream_t st, EventTimer* tm);
-// x-pass shapes: the default for nx, how many exist, whether shape c runs on
+// Whether csh_advance covers this physics on this plan (else one csh_rhs_stage
+// per stage): derive2csh always, derive2css on small grids.
+bool csh_fused(const CshPlan& p, const CshPhys& ph);
+// One right-hand side f of w, both in the reference's kx-fastest layout (small
+// grids only, see csh_small): no conversion to the ky-major layout.
+int csh_rhs_direct(const CshPlan& p, const double2* w, double2* f, const CshPhys& ph, hipStream_t st);
+// Passes for grids too small to fill the chip (csh2d_small.hip).  csh_small: the
+// y passes run there; csh_small_xrows: the paired x pass is the better default.
+bool csh_small(const CshPlan& p);
+bool csh_small_xrows(const CshPlan& p);
+struct YfwdArgs;
+// Inverse y pass of w (element (i, j) at i*si + j*sj) into G0..G3.
+int csh_small_yinv(const CshPlan& p, const double2* w, const CshPhys& ph, size_t si, size_t sj, hipStream_t st);
+// Forward y pass and stage update; inv: and the inverse y pass of what it produced.
+int csh_small_yfwd(const CshPlan& p, int mode, const YfwdArgs& a, bool inv, hipStream_t st);
+// The x pass with a row's two field pairs side by side (x-pass shape kXPairs).
+constexpr int kXPairs = 9;
+bool csh_x_pairs_ok(int nx, int ny);
+int csh_x_pairs(const CshPlan& p, hipStream_t st);
+// x-pass shapes: the default for the plan, how many exist, whether shape c runs on
 // this plan's grid, and the x pass alone (for timing by the autotuner).
-int csh_default_xshape(int nx);
+int csh_default_xshape(const CshPlan& p);
 int csh_num_xshapes();
 int csh_xshape_ok(const CshPlan& p, int c);
 int csh_xpass(const CshPlan& p, hipStream_t st);

@@ -30,52 +30,9 @@
 // Wavenumbers: derive2csh uses pi = 3.1428 (a default-real literal) and
 // Lx = Ly = 2 pi (:16-21), so kx = i-1 and ky = j-1 or j-1-Ny are exact integers;
 // the host builds the tables with that exact expression (csh_plan_init).
-#include "common.h"
-#include "csh2d.h"
-#include "passes.h"
-#include "rfft.h"
+#include "csh2d_dev.h"
 
 namespace tara {
-
-// The register-resident transform of the y passes (csh_yem elements per thread).
-template <int NY>
-using RY = RF<NY, csh_yem(NY)>;
-
-// Columns per workgroup of the y passes: at least 256 threads.
-template <int N>
-struct YShape {
-    static constexpr int T = RY<N>::T;
-    static constexpr int CB = T >= 256 ? 1 : 256 / T;
-    static constexpr int NT = CB * T;
-};
-// Offset of element (kx = i, ky = j) in an 8-row-blocked intermediate.
-__device__ __forceinline__ size_t blk8(int i, int j, int nh)
-{
-    return ((size_t)(j >> 3) * nh + i) * 8 + (j & 7);
-}
-
-// Offset of element (i, j) in the intermediates G0..G3: groups of 2^gs rows
-// interleaved per kx, ld columns per group (CshPlan::gsh, CshPlan::gld).
-// Ny = 4096, 2-row groups: a wave of the x pass reading two rows reads
-// contiguous 32-byte pairs over consecutive kx, and the inverse y pass writes
-// its two interleaved columns' pairs together (YiShape); 0.195 ms inverse y +
-// 0.276 ms x at 4096^2, against 0.186 + 0.311 ms with 4-row groups.  Smaller
-// Ny, 4-row groups and contiguous columns: at 1024^2 0.0201 ms inverse y +
-// 0.0186 ms x, against 0.0236 + 0.0179 ms with 2-row groups and four
-// interleaved columns.  (With one column per inverse-y workgroup at 4096^2,
-// 4-row groups had measured faster than 8-row (0.20, 0.39 ms), 2-row (0.25,
-// 0.31) and plain row-major (0.34, 0.31).)
-__device__ __forceinline__ size_t blkg(int i, int j, int ld, int gs)
-{
-    return ((size_t)(j >> gs) * ld + i) * (1 << gs) + (j & ((1 << gs) - 1));
-}
-
-// derive2csh's ky: j-1 for j <= Ny/2, j-1-Ny above (exact integers, checked on the host).
-template <int NY>
-__device__ __forceinline__ double csh_ky(int j)
-{
-    return (double)(j < NY / 2 ? j : j - NY);
-}
 
 // --------------------------------------------------------------------- pass 1
 // Shape of the inverse y pass.  At Ny = 4096 (512 threads per column) two
@@ -193,35 +150,6 @@ __global__ __launch_bounds__((YiShape<NY, SCR>::NT), (YiShape<NY, SCR>::IL ? 4 :
 }
 
 // --------------------------------------------------------------------- pass 2
-// Two real c2r transforms in one complex FFT: with X_a, X_b the Hermitian half
-// spectra (kx = 0..M) of two real rows, Y[k] = X_a[k] + i X_b[k] over the full
-// length Nx (X[Nx-k] = conj X[k]) transforms to y = x_a + i x_b, so the product
-// x_a * x_b is Re(y) Im(y).  The imaginary parts of X[0] and X[M] are dropped,
-// as FFTW's c2r does.  Registers end with y at rf_final_idx<NX> positions.
-template <int NX, int EM, bool SPLIT>
-__device__ __forceinline__ void x_c2r_pair(const double2* ga, const double2* gb, int j, int t,
-                                           double2* xl, const double2* tw, double2 (&v)[RF<NX, EM>::E])
-{
-    constexpr int M = NX / 2;
-    constexpr int LD = csh_gld(M + 1), GS = csh_gshift(M + 1);
-#pragma unroll
-    for (int e = 0; e < RF<NX, EM>::E; ++e) {
-        const int k = rf_first_idx<NX, EM>(t, e);
-        const int kk = k <= M ? k : NX - k;
-        double2 a = ga[blkg(kk, j, LD, GS)], b = gb[blkg(kk, j, LD, GS)];
-        if (kk == 0 || kk == M) {
-            a.y = 0.0;
-            b.y = 0.0;
-        }
-        if (k > M) {
-            a.y = -a.y;
-            b.y = -b.y;
-        }
-        v[e] = make_double2(a.x - b.y, a.y + b.x);
-    }
-    rf_fft<NX, +1, EM, false, SPLIT>(v, t, xl, tw);
-}
-
 // Shape of the x pass: EM complex elements per thread (4, 8, 16: radix-4, -8,
 // -16 passes), RB rows per workgroup, SPLIT: the FFT exchanges go through LDS as
 // doubles in two rounds (half the LDS, so that two workgroups share a CU).
@@ -318,24 +246,6 @@ __global__ __launch_bounds__((XShape<NX, EM, RB, SPLIT>::NT)) void k_csh_x(
 }
 
 // --------------------------------------------------------------------- pass 3
-struct YfwdArgs {
-    const double2* h;      // nonlinear term, x-transformed
-    const double2* ws;     // stage input omega_s (viscous term)
-    double2* base;         // AB2: state (in/out); RK4: omega_n (stage 4: out)
-    double2* aux;          // AB2: history f_{n-1} (in/out); RK4: accumulator
-    double2* next;         // RK4: next stage input (out); RHS mode: f (out)
-    const double* kx;
-    const double* ky;
-    const int* imin;       // dealias: modes with i >= imin[j] drop the nonlinear term
-    int nh;
-    double nu, dt;
-    double alpha, lam;     // screened form: alpha * NL, viscous term on k^2 ws/(k^2 + lam)
-    int screened;
-    size_t bs;             // batched runs: field stride per run (blockIdx.y)
-    const double* nus;     // batched runs: viscosity per run (null: nu)
-    int* bad;              // per run: set to 1 when a new state value is not finite (AB2, RK4 stage 4)
-};
-
 template <int NY, int MODE>
 __global__ __launch_bounds__(YShape<NY>::NT) void k_csh_yfwd(YfwdArgs a, const double2* tw)
 {
@@ -368,42 +278,9 @@ __global__ __launch_bounds__(YShape<NY>::NT) void k_csh_yfwd(YfwdArgs a, const d
         if (i >= a.imin[j]) nl = make_double2(0.0, 0.0);
         const double kyv = csh_ky<NY>(j);
         const double k2 = kxv * kxv + kyv * kyv;
-        const double vk = a.nu * k2;
-        const double2 ws = a.ws[q];
-        double2 f;
-        if (a.screened) {
-            // derive2css.f95:118-130: -(alpha (NLx + NLy) + nu k^2 omega_d)
-            const double den = k2 + a.lam;
-            const double2 wd = (i == 0 && j == 0) ? make_double2(0.0, 0.0)
-                                                  : make_double2(k2 * (ws.x / den), k2 * (ws.y / den));
-            f = make_double2(-(a.alpha * nl.x + vk * wd.x), -(a.alpha * nl.y + vk * wd.y));
-        } else {
-            f = make_double2(-(nl.x + vk * ws.x), -(nl.y + vk * ws.y));
-        }
-        if (MODE == CSH_RHS) {
-            a.next[q] = f;
-        } else if (MODE == CSH_AB2) {
-            const double2 fo = a.aux[q];
-            const double2 wn = make_double2(ws.x + (1.5 * f.x - 0.5 * fo.x) * a.dt, ws.y + (1.5 * f.y - 0.5 * fo.y) * a.dt);
-            a.base[q] = wn;
-            a.aux[q] = f;
-            finite = finite && isfinite(wn.x) && isfinite(wn.y);
-        } else if (MODE == CSH_RK4_1) {
-            const double c6 = a.dt / 6.0, c2 = 0.5 * a.dt;
-            a.aux[q] = make_double2(ws.x + c6 * f.x, ws.y + c6 * f.y);
-            a.next[q] = make_double2(ws.x + c2 * f.x, ws.y + c2 * f.y);
-        } else if (MODE == CSH_RK4_2 || MODE == CSH_RK4_3) {
-            const double c3 = a.dt / 3.0, cn = (MODE == CSH_RK4_2) ? 0.5 * a.dt : a.dt;
-            const double2 w0 = a.base[q], acc = a.aux[q];
-            a.aux[q] = make_double2(acc.x + c3 * f.x, acc.y + c3 * f.y);
-            a.next[q] = make_double2(w0.x + cn * f.x, w0.y + cn * f.y);
-        } else {  // CSH_RK4_4
-            const double c6 = a.dt / 6.0;
-            const double2 acc = a.aux[q];
-            const double2 wn = make_double2(acc.x + c6 * f.x, acc.y + c6 * f.y);
-            a.base[q] = wn;
-            finite = finite && isfinite(wn.x) && isfinite(wn.y);
-        }
+        double2 wn, av;
+        csh_update<MODE>(a, q, i == 0 && j == 0, nl, a.ws[q], k2, &wn, &av);
+        finite = csh_store<MODE>(a, q, wn, av) && finite;
     }
     if (!finite && a.bad) a.bad[blockIdx.y] = 1;
 }
@@ -432,6 +309,7 @@ __global__ __launch_bounds__((YiShape<NY, false>::NT), (YiShape<NY, false>::IL ?
     g2 += rb;
     g3 += rb;
     if (a.nus) a.nu = a.nus[blockIdx.y];
+    a.screened = 0;  // derive2csh only
     using S = YiShape<NY, false>;
     constexpr int E = RY<NY>::E, T = S::T;
     __shared__ double2 lds[S::LDS_ELEMS];
@@ -454,41 +332,9 @@ __global__ __launch_bounds__((YiShape<NY, false>::NT), (YiShape<NY, false>::IL ?
         double2 nl = v[e];
         if (!live || i >= a.imin[j]) nl = make_double2(0.0, 0.0);
         const double kyv = csh_ky<NY>(j);
-        const double vk = a.nu * (kxv * kxv + kyv * kyv);
-        const double2 ws = live ? a.ws[q] : make_double2(0.0, 0.0);
-        const double2 f = make_double2(-(nl.x + vk * ws.x), -(nl.y + vk * ws.y));
-        double2 wn;  // the next stage's input
-        if (MODE == CSH_AB2) {
-            const double2 fo = live ? a.aux[q] : make_double2(0.0, 0.0);
-            wn = make_double2(ws.x + (1.5 * f.x - 0.5 * fo.x) * a.dt, ws.y + (1.5 * f.y - 0.5 * fo.y) * a.dt);
-            if (live) {
-                a.base[q] = wn;
-                a.aux[q] = f;
-            }
-            finite = finite && isfinite(wn.x) && isfinite(wn.y);
-        } else if (MODE == CSH_RK4_1) {
-            const double c6 = a.dt / 6.0, c2 = 0.5 * a.dt;
-            wn = make_double2(ws.x + c2 * f.x, ws.y + c2 * f.y);
-            if (live) {
-                a.aux[q] = make_double2(ws.x + c6 * f.x, ws.y + c6 * f.y);
-                a.next[q] = wn;
-            }
-        } else if (MODE == CSH_RK4_2 || MODE == CSH_RK4_3) {
-            const double c3 = a.dt / 3.0, cn = (MODE == CSH_RK4_2) ? 0.5 * a.dt : a.dt;
-            const double2 w0 = live ? a.base[q] : make_double2(0.0, 0.0);
-            const double2 acc = live ? a.aux[q] : make_double2(0.0, 0.0);
-            wn = make_double2(w0.x + cn * f.x, w0.y + cn * f.y);
-            if (live) {
-                a.aux[q] = make_double2(acc.x + c3 * f.x, acc.y + c3 * f.y);
-                a.next[q] = wn;
-            }
-        } else {  // CSH_RK4_4
-            const double c6 = a.dt / 6.0;
-            const double2 acc = live ? a.aux[q] : make_double2(0.0, 0.0);
-            wn = make_double2(acc.x + c6 * f.x, acc.y + c6 * f.y);
-            if (live) a.base[q] = wn;
-            finite = finite && isfinite(wn.x) && isfinite(wn.y);
-        }
+        double2 wn, av;  // wn: the next stage's input
+        csh_update<MODE>(a, q, false, nl, a.ws[q], kxv * kxv + kyv * kyv, &wn, &av);
+        if (live) finite = csh_store<MODE>(a, q, wn, av) && finite;
         v[e] = wn;
     }
     if (!finite && a.bad) a.bad[blockIdx.y] = 1;
@@ -526,12 +372,13 @@ static int launch_yinv(const CshPlan& p, const double2* w, const CshPhys& ph, hi
 }
 
 // x-pass shapes the autotuner chooses among: {EM, RB, SPLIT}.  Shape 0 is
-// RB = min(8, 1024 / T) at EM = 8 without splitting (the largest workgroup).
+// RB = min(8, 1024 / T) at EM = 8 without splitting (the largest workgroup);
+// shape kXPairs runs a row's two field pairs side by side (csh2d_small.hip).
 struct XCand {
     int em, rb, split;
 };
 constexpr XCand kXCands[] = {{8, 0, 0}, {16, 2, 1}, {8, 1, 1}, {16, 4, 1}, {8, 2, 1}, {16, 1, 0},
-                              {4, 1, 0}, {4, 2, 0}, {4, 4, 1}};
+                              {4, 1, 0}, {4, 2, 0}, {4, 4, 1}, {8, 0, 0}};
 constexpr int kNumXCands = sizeof(kXCands) / sizeof(kXCands[0]);
 
 template <int NX, int EM>
@@ -573,6 +420,7 @@ static int launch_x(const CshPlan& p, hipStream_t st)
         case 6: return launch_x_shape<NX, 4, 1, false>(p, st);
         case 7: return launch_x_shape<NX, 4, 2, false>(p, st);
         case 8: return launch_x_shape<NX, 4, 4, true>(p, st);
+        case kXPairs: return csh_x_pairs(p, st);
         default: set_error("x pass shape %d unknown", p.xcfg); return TARA_ERR_ARG;
     }
 }
@@ -590,6 +438,7 @@ static bool x_shape_ok(int c, int ny)
         case 6: return XShape<NX, 4, 1, false>::OK;
         case 7: return XShape<NX, 4, 2, false>::OK && ny % 2 == 0;
         case 8: return XShape<NX, 4, 4, true>::OK && ny % 4 == 0;
+        case kXPairs: return csh_x_pairs_ok(NX, ny);
         default: return false;
     }
 }
@@ -742,16 +591,11 @@ int csh_plan_init(CshPlan& p, int nx, int ny, int batch)
     p.rctw = rc_twiddles(nx);
     TARA_CHECK(p.tw_y && p.tw_x && p.tw_xn && p.tw_x16 && p.tw_xn16 && p.tw_x4 && p.tw_xn4 && p.rctw, TARA_ERR_ALLOC,
                "twiddle table allocation failed");
-    p.xcfg = csh_default_xshape(nx);
-    if (shape_ok(p, p.xcfg) != 1) p.xcfg = 0;
+    p.xcfg = csh_default_xshape(p);
     return TARA_OK;
 }
 
-int csh_default_xshape(int nx)
-{
-    (void)nx;
-    return 0;
-}
+int csh_default_xshape(const CshPlan& p) { return csh_small_xrows(p) && shape_ok(p, kXPairs) == 1 ? kXPairs : 0; }
 
 int csh_num_xshapes() { return kNumXCands; }
 
@@ -783,24 +627,12 @@ int csh_clear_nonfinite(const CshPlan& p, int r, hipStream_t st)
     return TARA_OK;
 }
 
-int csh_rhs_stage(const CshPlan& p, const double2* ws, int mode, const CshPhys& ph, double dt, double2* base,
-                  double2* aux, double2* next, hipStream_t st, EventTimer* tm)
+// The arguments of a forward y pass whose stage input, base, accumulator and
+// output are set by the caller.
+static YfwdArgs yargs(const CshPlan& p, const CshPhys& ph, double dt)
 {
-    int rc;
-    if (tm) tm->begin(0, st);
-    if ((rc = yinv(p, ws, ph, st))) return rc;
-    if (tm) tm->end(0, st);
-    if (tm) tm->begin(1, st);
-    if ((rc = xpass(p, st))) return rc;
-    if (tm) tm->end(1, st);
-    YfwdArgs a;
+    YfwdArgs a{};
     a.h = p.h.as<double2>();
-    a.ws = ws;
-    a.base = base;
-    a.aux = aux;
-    a.next = next;
-    a.kx = p.kx.as<double>();
-    a.ky = p.ky.as<double>();
     a.imin = p.imin.as<int>();
     a.nh = p.nh;
     a.nu = ph.nu;
@@ -811,23 +643,60 @@ int csh_rhs_stage(const CshPlan& p, const double2* ws, int mode, const CshPhys& 
     a.bs = p.bstride;
     a.nus = ph.nus;
     a.bad = p.bad.as<int>();
+    a.si = p.ny;
+    a.sj = 1;
+    return a;
+}
+
+int csh_rhs_stage(const CshPlan& p, const double2* ws, int mode, const CshPhys& ph, double dt, double2* base,
+                  double2* aux, double2* next, hipStream_t st, EventTimer* tm)
+{
+    int rc;
+    const bool small = csh_small(p);
+    YfwdArgs a = yargs(p, ph, dt);
+    a.ws = ws;
+    a.base = base;
+    a.aux = aux;
+    a.next = next;
+    if (tm) tm->begin(0, st);
+    if ((rc = small ? csh_small_yinv(p, ws, ph, p.ny, 1, st) : yinv(p, ws, ph, st))) return rc;
+    if (tm) tm->end(0, st);
+    if (tm) tm->begin(1, st);
+    if ((rc = xpass(p, st))) return rc;
+    if (tm) tm->end(1, st);
     if (tm) tm->begin(2, st);
-    if ((rc = yfwd(p, mode, a, st))) return rc;
+    if ((rc = small ? csh_small_yfwd(p, mode, a, false, st) : yfwd(p, mode, a, st))) return rc;
     if (tm) tm->end(2, st);
     TARA_HIP(hipGetLastError());
     return TARA_OK;
 }
 
+int csh_rhs_direct(const CshPlan& p, const double2* w, double2* f, const CshPhys& ph, hipStream_t st)
+{
+    int rc;
+    YfwdArgs a = yargs(p, ph, 0.0);
+    a.ws = w;
+    a.next = f;
+    a.si = 1;
+    a.sj = p.nh;
+    if ((rc = csh_small_yinv(p, w, ph, 1, p.nh, st)) || (rc = xpass(p, st)) ||
+        (rc = csh_small_yfwd(p, CSH_RHS, a, false, st)))
+        return rc;
+    TARA_HIP(hipGetLastError());
+    return TARA_OK;
+}
+
 // Fusing the forward y pass with the next inverse y pass pays from Ny = 1024
-// (1024^2 RK4 step 0.181 -> 0.168 ms, 4096^2 2.41 -> 2.36 ms); below, the fused
-// pass holds fewer waves per CU than the separate forward y pass, and the
-// 128-512 ensemble step measured 6.65 ms fused against 6.43 ms separate.
-static bool fuse_y(const CshPlan& p) { return p.ny >= 1024; }
+// (1024^2 RK4 step 0.181 -> 0.168 ms, 4096^2 2.41 -> 2.36 ms) and on grids too
+// small to fill the chip (csh2d_small.hip); else, below 1024, the fused pass
+// holds fewer waves per CU than the separate forward y pass, and the 128-512
+// ensemble step measured 6.65 ms fused against 6.43 ms separate.
+static bool fuse_y(const CshPlan& p) { return p.ny >= 1024 || csh_small(p); }
 
 int csh_yinv_pass(const CshPlan& p, const double2* w, const CshPhys& ph, hipStream_t st)
 {
     if (!fuse_y(p)) return TARA_OK;  // the unfused step runs its own inverse y passes
-    int rc = yinv(p, w, ph, st);
+    int rc = csh_small(p) ? csh_small_yinv(p, w, ph, p.ny, 1, st) : yinv(p, w, ph, st);
     if (rc) return rc;
     TARA_HIP(hipGetLastError());
     return TARA_OK;
@@ -836,7 +705,8 @@ int csh_yinv_pass(const CshPlan& p, const double2* w, const CshPhys& ph, hipStre
 int csh_fused_step(const CshPlan& p, int scheme, const CshPhys& ph, double dt, double2* w, double2* aux,
                    double2* next, bool plain_last, hipStream_t st, EventTimer* tm)
 {
-    TARA_CHECK(!ph.screened, TARA_ERR_ARG, "the fused step covers derive2csh only");
+    const bool small = csh_small(p);
+    TARA_CHECK(!ph.screened || small, TARA_ERR_ARG, "the fused step of large grids covers derive2csh only");
     int rc;
     if (!fuse_y(p)) {
         if (scheme == TARA_SCHEME_AB2) return csh_rhs_stage(p, w, CSH_AB2, ph, dt, w, aux, nullptr, st, tm);
@@ -844,22 +714,9 @@ int csh_fused_step(const CshPlan& p, int scheme, const CshPhys& ph, double dt, d
             if ((rc = csh_rhs_stage(p, k == 0 ? w : next, CSH_RK4_1 + k, ph, dt, w, aux, next, st, tm))) return rc;
         return TARA_OK;
     }
-    YfwdArgs a;
-    a.h = p.h.as<double2>();
+    YfwdArgs a = yargs(p, ph, dt);
     a.base = w;
     a.aux = aux;
-    a.kx = p.kx.as<double>();
-    a.ky = p.ky.as<double>();
-    a.imin = p.imin.as<int>();
-    a.nh = p.nh;
-    a.nu = ph.nu;
-    a.dt = dt;
-    a.alpha = ph.alpha;
-    a.lam = ph.lambda;
-    a.screened = 0;
-    a.bs = p.bstride;
-    a.nus = ph.nus;
-    a.bad = p.bad.as<int>();
     const int nst = scheme == TARA_SCHEME_AB2 ? 1 : 4;
     for (int k = 0; k < nst; ++k) {
         const int mode = scheme == TARA_SCHEME_AB2 ? CSH_AB2 : CSH_RK4_1 + k;
@@ -870,17 +727,20 @@ int csh_fused_step(const CshPlan& p, int scheme, const CshPhys& ph, double dt, d
         if (tm) tm->end(1, st);
         const bool plain = plain_last && k == nst - 1;
         if (tm) tm->begin(2, st);
-        if ((rc = plain ? yfwd(p, mode, a, st) : yfwd_inv(p, mode, a, st))) return rc;
+        if ((rc = small ? csh_small_yfwd(p, mode, a, !plain, st) : plain ? yfwd(p, mode, a, st) : yfwd_inv(p, mode, a, st)))
+            return rc;
         if (tm) tm->end(2, st);
     }
     TARA_HIP(hipGetLastError());
     return TARA_OK;
 }
 
+bool csh_fused(const CshPlan& p, const CshPhys& ph) { return !ph.screened || csh_small(p); }
+
 int csh_advance(const CshPlan& p, int scheme, int nsteps, const CshPhys& ph, double dt, double2* w,
                 double2* aux, double2* next, hipStream_t st, EventTimer* tm)
 {
-    TARA_CHECK(!ph.screened, TARA_ERR_ARG, "the fused advance covers derive2csh only");
+    TARA_CHECK(csh_fused(p, ph), TARA_ERR_ARG, "the fused advance of large grids covers derive2csh only");
     if (nsteps <= 0) return TARA_OK;
     int rc;
     if (tm) tm->begin(0, st);

@@ -1,0 +1,325 @@
+// The 2D incompressible passes for grids too small to fill the chip (csh2d.hip
+// holds those of large grids and batches).  There a pass's time is the latency
+// of one thread's chain of loads and transforms, not bandwidth: at 64^2 the
+// inverse y pass ran four transforms one after another in 6.9 us, the forward y
+// and x passes 4.8 and 4.7 us, against about 2.2 us for a kernel that does
+// nothing.  So the chains are cut: every transform of a pass gets its own
+// threads, sequences of at most 64 threads exchange within their wavefront, and
+// a stage is two kernels (x, forward y + next inverse y) instead of three.
+// RK4 step, three kernels a stage -> two, default x shapes: 64^2 65.4 -> 39.8 us,
+// 256^2 98.7 -> 47.2, 512^2 131.8 -> 72.5, 1024 x 512 201 -> 118; 512 x 256 screened
+// 122 -> 60; one right-hand side on device arrays at 256^2 30.1 -> 14.5 us.  What
+// is left is the chain itself: about 5 us a kernel at 64^2, of which 2.2 us is
+// what any kernel takes.
+#include "csh2d_dev.h"
+
+namespace tara {
+
+// --------------------------------------------------------------------- y pass
+// One kx column per 4 T threads: group g transforms field g of the inverse pass
+// (G0 = ux, G1 = uy, G2 = d omega/dx, G3 = d omega/dy).  The forward transform
+// and the update before it (FWD) are done by every group, so that each holds
+// the next stage's input in registers; group 0 stores it.
+template <int NY, int NG>
+struct SYShape {
+    static constexpr int T = RY<NY>::T;                      // threads per sequence
+    static constexpr bool WAVE = T <= 64;                    // a sequence sits in one wavefront
+    static constexpr int CB = NG * T >= 64 ? 1 : 64 / (NG * T);  // columns per workgroup
+    static constexpr int NT = CB * NG * T;
+    static constexpr bool OK = NT <= 1024;
+};
+
+struct SYInv {
+    double2 *g0, *g1, *g2, *g3;
+    int ld;
+};
+
+template <int NY, int MODE, int GS, bool FWD, bool INV>
+__global__ __launch_bounds__((SYShape<NY, INV ? 4 : 1>::NT)) void k_csh_small_y(YfwdArgs a, SYInv o, const double2* tw)
+{
+    constexpr int NG = INV ? 4 : 1;
+    using S = SYShape<NY, NG>;
+    constexpr int E = RY<NY>::E, T = S::T, EM = csh_yem(NY);
+    __shared__ double2 lds[S::CB * NG * RY<NY>::LDS];
+    const size_t rb = blockIdx.y * a.bs;  // batched runs
+    a.ws += rb;
+    const int t = threadIdx.x % T, seq = threadIdx.x / T, g = seq % NG;
+    const int i = xcd_remap(blockIdx.x, gridDim.x) * S::CB + seq / NG;
+    const bool live = i < a.nh;
+    const int ic = live ? i : 0;  // dead columns recompute column 0 and store nothing
+    double2* xl = lds + seq * RY<NY>::LDS;
+    const double kxv = (double)ic;
+    double2 v[E];
+    if constexpr (FWD) {
+        a.h += rb;
+        if (a.base) a.base += rb;
+        if (a.aux) a.aux += rb;
+        if (a.next) a.next += rb;
+        if (a.nus) a.nu = a.nus[blockIdx.y];
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e] = a.h[blk8(ic, rf_first_idx<NY, EM>(t, e), a.nh)];
+        rf_fft<NY, -1, EM, S::WAVE>(v, t, xl, tw);
+        double2 av[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const int j = rf_final_idx<NY, EM>(t, e);
+            const size_t q = (size_t)ic * a.si + (size_t)j * a.sj;
+            const double2 nl = ic >= a.imin[j] ? make_double2(0.0, 0.0) : v[e];
+            const double kyv = csh_ky<NY>(j);
+            csh_update<MODE>(a, q, ic == 0 && j == 0, nl, a.ws[q], kxv * kxv + kyv * kyv, &v[e], &av[e]);
+        }
+        // every group has read the column before group 0 writes it
+        if constexpr (NG > 1) __syncthreads();
+        if (live && g == 0) {
+            bool finite = true;
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const size_t q = (size_t)ic * a.si + (size_t)rf_final_idx<NY, EM>(t, e) * a.sj;
+                finite = csh_store<MODE>(a, q, v[e], av[e]) && finite;
+            }
+            if (!finite && a.bad) a.bad[blockIdx.y] = 1;
+        }
+        if constexpr (INV) rf_final_to_first<NY, EM, S::WAVE>(v, t, xl);
+    } else {
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e] = a.ws[(size_t)ic * a.si + (size_t)rf_first_idx<NY, EM>(t, e) * a.sj];
+    }
+    if constexpr (INV) {
+        // derive2csh.f95:29-71: groups 0, 1 i ky psi, -i kx psi with psi =
+        // omega/k^2, psi(0,0) = 0; groups 2, 3 i kx omega, i ky omega.  Screened
+        // (derive2css.f95:22-52): psi = omega/(k^2 + lambda), omega_d = k^2 psi.
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            const int j = rf_first_idx<NY, EM>(t, e);
+            const double kyv = csh_ky<NY>(j);
+            const double k2 = kxv * kxv + kyv * kyv;
+            const double den = a.screened ? k2 + a.lam : k2;
+            const bool zero = a.screened ? ic == 0 && j == 0 : k2 == 0.0;
+            double2 z = v[e];
+            if (g < 2 || a.screened) z = zero ? make_double2(0.0, 0.0) : make_double2(z.x / den, z.y / den);
+            if (g >= 2 && a.screened) z = make_double2(k2 * z.x, k2 * z.y);
+            const double kk = (g == 0 || g == 3) ? kyv : g == 1 ? -kxv : kxv;
+            v[e] = make_double2(-(kk * z.y), kk * z.x);
+        }
+        rf_fft<NY, +1, EM, S::WAVE>(v, t, xl, tw);
+        double2* out = (g == 0 ? o.g0 : g == 1 ? o.g1 : g == 2 ? o.g2 : o.g3) + rb;
+        if (live) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) out[blkg(i, rf_final_idx<NY, EM>(t, e), o.ld, GS)] = v[e];
+        }
+    }
+}
+
+// --------------------------------------------------------------------- x pass
+// One y row per 2 T threads: the first T transform ux + i uy, the others
+// d omega/dx + i d omega/dy; they meet in LDS, where the first T/2 threads form
+// ux d omega/dx + uy d omega/dy and run its forward half-length transform.  (A
+// pair shares its rounding error, so fields of like size are paired: k_csh_x,
+// which pairs ux with d omega/dx to hold one product instead of two fields, has
+// 5e-12 of the nonlinear term on white noise at 1024 x 128.)
+template <int NX>
+struct SXShape {
+    static constexpr int M = NX / 2;
+    static constexpr int T = RF<NX>::T, TM = RF<M>::T;
+    static constexpr bool WAVE = T <= 64;
+    static constexpr int RB = 2 * T >= 64 ? 1 : 64 / (2 * T);  // rows per workgroup
+    static constexpr int NT = 2 * T * RB;
+    static constexpr bool OK = NT <= 1024 && 2 * TM == T && 2 * RB * RF<NX>::LDS * 16 <= 160 * 1024;
+};
+
+template <int NX>
+__global__ __launch_bounds__((SXShape<NX>::NT)) void k_csh_x_pairs(const double2* g0, const double2* g1,
+                                                                   const double2* g2, const double2* g3, double scale,
+                                                                   double2* __restrict__ h, const double2* tw_n,
+                                                                   const double2* tw_m, const double2* rctw, size_t bs)
+{
+    using S = SXShape<NX>;
+    static_assert(S::OK, "paired x pass does not fit");
+    constexpr int E = RF<NX>::E, EH = RF<S::M>::E, T = S::T, M = S::M;
+    __shared__ double2 lds[2 * S::RB * RF<NX>::LDS];
+    const size_t rb = blockIdx.y * bs;  // batched runs
+    const int t = threadIdx.x % T, seq = threadIdx.x / T, p = seq % 2, r = seq / 2;
+    const int j = xcd_remap(blockIdx.x, gridDim.x) * S::RB + r;
+    double2* xl = lds + seq * RF<NX>::LDS;
+    double2* x0 = lds + 2 * r * RF<NX>::LDS;  // the row's first buffer
+    double2 v[E];
+    x_c2r_pair<NX, 8, false, S::WAVE>((p ? g2 : g0) + rb, (p ? g3 : g1) + rb, j, t, xl, tw_n, v);
+#pragma unroll
+    for (int e = 0; e < E; ++e) xl[rf_pad(rf_final_idx<NX>(t, e))] = v[e];
+    // the unpacking roots of this thread's kx, fetched before the stores
+    constexpr int NK = M / (2 * T);
+    const int tt = p * T + t;
+    double2 wk[NK];
+#pragma unroll
+    for (int u = 0; u < NK; ++u) wk[u] = rctw[tt + u * 2 * T];
+    __syncthreads();
+    const bool fwd = p == 0 && t < S::TM;
+    double2 z[EH];
+    if (fwd) {
+        const double2* x1 = x0 + RF<NX>::LDS;
+        auto nl = [&](int n) {
+            const double2 u = x0[rf_pad(n)], w = x1[rf_pad(n)];
+            return (u.x * w.x + u.y * w.y) * scale;
+        };
+#pragma unroll
+        for (int e = 0; e < EH; ++e) {
+            const int m = rf_first_idx<M>(t, e);
+            z[e] = make_double2(nl(2 * m), nl(2 * m + 1));
+        }
+    }
+    __syncthreads();
+    if (fwd) {
+        rf_fft<M, -1, 8, S::WAVE>(z, t, x0, tw_m);
+#pragma unroll
+        for (int e = 0; e < EH; ++e) x0[rf_pad(rf_final_idx<M>(t, e))] = z[e];
+    } else if constexpr (!S::WAVE) {
+        rf_fft_barriers_only<M>();  // TM >= 64: whole waves
+    }
+    __syncthreads();
+    h += rb;
+#pragma unroll
+    for (int u = 0; u < NK; ++u) {
+        const int k = tt + u * 2 * T;
+        const double2 zk = x0[rf_pad(k)];
+        const double2 zmk = x0[rf_pad(k == 0 ? 0 : M - k)];
+        double2 xm;
+        h[blk8(k, j, M + 1)] = r2c_unpack_w(zk, zmk, k, wk[u], &xm);
+        if (k == 0) h[blk8(M, j, M + 1)] = xm;
+    }
+}
+
+// ------------------------------------------------------------------- dispatch
+// The y passes run here while their threads come to at most 2112 wavefronts,
+// two per SIMD and the odd column of Nh.  RK4 step (tuned x shape) here against
+// the larger grids' passes: 1024 x 512 (2052 wavefronts) 117 / 146 us, 256 x 1024
+// (2064) 91.7 / 93.9; beyond, the repeated forward transform costs more than the
+// shorter chain gives: 512 x 1024 (4112) 139 / 112, 1024^2 (8208) 203 / 147; 64
+// runs of 128^2 (4160) 154 / 157 per ensemble step, 32 of 256^2 (8256) 242 / 242.
+//
+// The paired x pass is the default up to 2^20 points and Ny = 2048, against
+// shape 0 there: RK4 step 512^2 72.5 / 93.5 us, 1024 x 256 78.5 / 145, 1024^2
+// 153 / 192, 64^2 40 / 43; 256 x 4096 245 / 233, 2048 x 1024 276 / 260, 4096^2 2512 /
+// 2301.  (The autotuner times it among the other shapes.)
+constexpr size_t kSmallWaves = 2112, kSmallX = 1 << 20;
+
+bool csh_small(const CshPlan& p)
+{
+    const size_t threads = (size_t)p.nh * 4 * (p.ny / csh_yem(p.ny)) * p.batch;
+    return p.ny <= 1024 && threads <= 64 * kSmallWaves;
+}
+
+bool csh_small_xrows(const CshPlan& p) { return p.ny <= 2048 && (size_t)p.nx * p.ny * p.batch <= kSmallX; }
+
+template <int NY, int MODE, bool FWD, bool INV>
+static int launch_small_y(const CshPlan& p, const YfwdArgs& a, hipStream_t st)
+{
+    using S = SYShape<NY, INV ? 4 : 1>;
+    if constexpr (!S::OK) {
+        set_error("small y pass at Ny=%d", NY);
+        return TARA_ERR_UNSUPPORTED;
+    } else {
+        const SYInv o{p.g[0].as<double2>(), p.g[1].as<double2>(), p.g[2].as<double2>(), p.g[3].as<double2>(), p.gld};
+        const dim3 grid((p.nh + S::CB - 1) / S::CB, p.batch), b(S::NT);
+        if (p.gsh == 1)
+            hipLaunchKernelGGL((k_csh_small_y<NY, MODE, 1, FWD, INV>), grid, b, 0, st, a, o, p.tw_y);
+        else
+            hipLaunchKernelGGL((k_csh_small_y<NY, MODE, 2, FWD, INV>), grid, b, 0, st, a, o, p.tw_y);
+        return TARA_OK;
+    }
+}
+
+template <int NY>
+static int launch_small_yinv(const CshPlan& p, const YfwdArgs& a, hipStream_t st)
+{
+    return launch_small_y<NY, CSH_RHS, false, true>(p, a, st);
+}
+
+template <int NY>
+static int launch_small_yfwd(const CshPlan& p, int mode, const YfwdArgs& a, bool inv, hipStream_t st)
+{
+#define TARA_SMALL_MODE(M) \
+    case M: return inv ? launch_small_y<NY, M, true, true>(p, a, st) : launch_small_y<NY, M, true, false>(p, a, st);
+    switch (mode) {
+        case CSH_RHS: return launch_small_y<NY, CSH_RHS, true, false>(p, a, st);
+        TARA_SMALL_MODE(CSH_AB2)
+        TARA_SMALL_MODE(CSH_RK4_1)
+        TARA_SMALL_MODE(CSH_RK4_2)
+        TARA_SMALL_MODE(CSH_RK4_3)
+        TARA_SMALL_MODE(CSH_RK4_4)
+        default: set_error("bad mode %d", mode); return TARA_ERR_ARG;
+    }
+#undef TARA_SMALL_MODE
+}
+
+#define TARA_SMALL_Y_SWITCH(n, FN, ...)             \
+    switch (n) {                                    \
+        case 16: return FN<16>(__VA_ARGS__);        \
+        case 32: return FN<32>(__VA_ARGS__);        \
+        case 64: return FN<64>(__VA_ARGS__);        \
+        case 128: return FN<128>(__VA_ARGS__);      \
+        case 256: return FN<256>(__VA_ARGS__);      \
+        case 512: return FN<512>(__VA_ARGS__);      \
+        case 1024: return FN<1024>(__VA_ARGS__);    \
+        default: set_error("small y pass: unsupported length %d", n); return TARA_ERR_UNSUPPORTED; \
+    }
+
+int csh_small_yinv(const CshPlan& p, const double2* w, const CshPhys& ph, size_t si, size_t sj, hipStream_t st)
+{
+    YfwdArgs a{};
+    a.ws = w;
+    a.nh = p.nh;
+    a.lam = ph.lambda;
+    a.screened = ph.screened;
+    a.bs = p.bstride;
+    a.si = si;
+    a.sj = sj;
+    TARA_SMALL_Y_SWITCH(p.ny, launch_small_yinv, p, a, st)
+}
+
+int csh_small_yfwd(const CshPlan& p, int mode, const YfwdArgs& a, bool inv, hipStream_t st)
+{
+    TARA_SMALL_Y_SWITCH(p.ny, launch_small_yfwd, p, mode, a, inv, st)
+}
+
+template <int NX>
+static int launch_x_pairs(const CshPlan& p, hipStream_t st)
+{
+    using S = SXShape<NX>;
+    const double scale = 1.0 / ((double)p.nx * (double)p.ny * (double)p.nx * (double)p.ny);
+    hipLaunchKernelGGL(k_csh_x_pairs<NX>, dim3(p.ny / S::RB, p.batch), dim3(S::NT), 0, st, p.g[0].as<double2>(),
+                       p.g[1].as<double2>(), p.g[2].as<double2>(), p.g[3].as<double2>(), scale, p.h.as<double2>(),
+                       p.tw_xn, p.tw_x, p.rctw, p.bstride);
+    return TARA_OK;
+}
+
+#define TARA_X_PAIRS_SWITCH(n, FN, ...)             \
+    switch (n) {                                    \
+        case 64: return FN<64>(__VA_ARGS__);        \
+        case 128: return FN<128>(__VA_ARGS__);      \
+        case 256: return FN<256>(__VA_ARGS__);      \
+        case 512: return FN<512>(__VA_ARGS__);      \
+        case 1024: return FN<1024>(__VA_ARGS__);    \
+        case 2048: return FN<2048>(__VA_ARGS__);    \
+        case 4096: return FN<4096>(__VA_ARGS__);    \
+        default: return 0;                          \
+    }
+
+template <int NX>
+static int x_pairs_rows(int)
+{
+    return SXShape<NX>::RB;
+}
+
+// Rows per workgroup of the paired x pass, 0 where it has no kernel.
+static int pairs_rows(int nx) { TARA_X_PAIRS_SWITCH(nx, x_pairs_rows, 0) }
+
+bool csh_x_pairs_ok(int nx, int ny) { return pairs_rows(nx) > 0 && ny % pairs_rows(nx) == 0; }
+
+int csh_x_pairs(const CshPlan& p, hipStream_t st)
+{
+    TARA_CHECK(csh_x_pairs_ok(p.nx, p.ny), TARA_ERR_UNSUPPORTED, "x pass shape %d does not run on %dx%d", kXPairs, p.nx,
+               p.ny);
+    TARA_X_PAIRS_SWITCH(p.nx, launch_x_pairs, p, st)
+}
+
+}  // namespace tara

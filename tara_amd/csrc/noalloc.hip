@@ -155,12 +155,14 @@ extern "C" int tara_derive2csh_noalloc(int nx, int ny, int nh, double nu, const 
     p.tw_x16 = reinterpret_cast<const double2*>(base + L.tw_x16);
     p.tw_xn16 = reinterpret_cast<const double2*>(base + L.tw_xn16);
     p.rctw = reinterpret_cast<const double2*>(base + L.rctw);
-    p.xcfg = csh_default_xshape(nx);  // the drop-in plan's shape (csh_plan_init)
-    if (!csh_xshape_ok(p, p.xcfg)) p.xcfg = 0;
+    p.xcfg = csh_default_xshape(p);  // the drop-in plan's shape (csh_plan_init)
     double2* w = reinterpret_cast<double2*>(base + L.w);
     double2* f = reinterpret_cast<double2*>(base + L.f);
     CshPhys ph;
     ph.nu = nu;
+    if (csh_small(p))
+        return csh_rhs_direct(p, reinterpret_cast<const double2*>(omegak), reinterpret_cast<double2*>(dt_omegak_new), ph,
+                              st);
     if ((rc = to_kymajor(reinterpret_cast<const double2*>(omegak), w, nh, ny, 1, st))) return rc;
     if ((rc = csh_rhs_stage(p, w, CSH_RHS, ph, 0.0, nullptr, nullptr, f, st, nullptr))) return rc;
     if ((rc = from_kymajor(f, reinterpret_cast<double2*>(dt_omegak_new), nh, ny, 1, st))) return rc;
