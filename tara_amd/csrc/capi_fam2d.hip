@@ -133,7 +133,7 @@ extern "C" int tara_derive2coh(int nx, int ny, int nh, const tara_coh_params* pr
     ph.cs = prm->cs;
     return derive_host(0, nx, ny, prm->pi, prm->lx, prm->ly, state, rhs,
                        [&](const F2Plan& p, double2* const st[], double2* const out[]) {
-                           return coh_rhs_stage(p, ph, st, F2_RHS, 0.0, out, nullptr, nullptr);
+                           return coh_rhs(p, ph, st, out, nullptr);
                        });
 }
 
@@ -200,7 +200,7 @@ extern "C" int tara_derive2com(int nx, int ny, int nh, const tara_com_params* pr
     ph.amp = prm->a;
     return derive_host(1, nx, ny, prm->pi, prm->lx, prm->ly, state, rhs,
                        [&](const F2Plan& p, double2* const st[], double2* const out[]) {
-                           return com_rhs_stage(p, ph, st, F2_RHS, 0.0, out, nullptr, nullptr);
+                           return com_rhs(p, ph, st, out, nullptr);
                        });
 }
 
@@ -223,6 +223,7 @@ struct tara_f2 {
     ComPhys com;
     double dt = 0;
     DevBuf st[6], hist[6];
+    DevBuf alt[6];  // the other set a step writes: coh state and history (3 + 3), com momentum (2)
     hipStream_t s = nullptr;
     std::unique_ptr<EventTimer> tm;
 };
@@ -243,6 +244,8 @@ static int f2_create(int family, int nx, int ny, double pi, double lx, double ly
         TARA_HIP(hipMemset(c->st[f].p, 0, bytes));
         TARA_HIP(hipMemset(c->hist[f].p, 0, bytes));
     }
+    for (int f = 0; f < (family == 0 ? 6 : 2); ++f)
+        if ((rc = c->alt[f].alloc(bytes))) return rc;
     TARA_HIP(hipStreamCreate(&c->s));
     *made = c.get();
     *out = c.release();
@@ -323,12 +326,19 @@ extern "C" int tara_f2_advance(tara_f2* c, int nsteps)
         st[f] = c->st[f].as<double2>();
         hist[f] = c->hist[f].as<double2>();
     }
-    for (int s = 0; s < nsteps; ++s) {
-        int rc = c->family == 0 ? coh_rhs_stage(c->plan, c->coh, st, F2_AB2, c->dt, hist, c->s, c->tm.get())
-                                : com_rhs_stage(c->plan, c->com, st, F2_AB2, c->dt, hist, c->s, c->tm.get());
-        if (rc) return rc;
+    double2* alt[6];
+    for (int f = 0; f < 6; ++f) alt[f] = c->alt[f].as<double2>();
+    int rc;
+    if (c->family == 0)
+        rc = coh_advance(c->plan, c->coh, st, hist, alt, alt + 3, nsteps, c->dt, c->s, c->tm.get());
+    else
+        rc = com_advance(c->plan, c->com, st, alt, hist, nsteps, c->dt, c->s, c->tm.get());
+    for (int f = 0; f < 6; ++f) {
+        c->st[f].p = st[f];
+        c->hist[f].p = hist[f];
+        c->alt[f].p = alt[f];
     }
-    return TARA_OK;
+    return rc;
 }
 
 extern "C" int tara_f2_sync(tara_f2* c)
