@@ -69,6 +69,28 @@ struct DevBuf {
     T* as() const { return static_cast<T*>(p); }
 };
 
+// Device work space of one synchronous host-array call: opened with its size,
+// handed out in pieces, given back at the end.  Up to kScratchKeep bytes come
+// from one buffer per device that is kept between calls (a hipMalloc and a
+// hipFree cost about 50 us each time); a call holds its lock until it ends, and a
+// larger call allocates its own.
+struct Scratch {
+    static constexpr size_t kScratchKeep = (size_t)256 << 20;
+    DevBuf own;
+    std::unique_lock<std::mutex> lock;
+    char* base = nullptr;
+    size_t used = 0, size = 0;
+    int open(size_t bytes);
+    static size_t pad(size_t bytes) { return (bytes + 255) / 256 * 256; }
+    template <class T>
+    T* take(size_t n)
+    {
+        T* p = reinterpret_cast<T*>(base + used);
+        used += pad(n * sizeof(T));
+        return used <= size ? p : nullptr;
+    }
+};
+
 // Per-device immutable tables, built once and kept for the process lifetime.
 //   twiddles(n, rmax): Stockham per-pass table for a length-n complex FFT whose
 //                      schedule caps the radix at rmax (8 or 4; fft_core.h)

@@ -40,6 +40,37 @@ void DevBuf::release()
     own = true;
 }
 
+int Scratch::open(size_t bytes)
+{
+    used = 0;
+    size = bytes;
+    if (bytes > kScratchKeep) {
+        int rc = own.alloc(bytes);
+        base = static_cast<char*>(own.p);
+        return rc;
+    }
+    struct Kept {
+        std::mutex mu;
+        DevBuf buf;
+    };
+    static std::mutex g_mu;
+    static std::map<int, std::unique_ptr<Kept>> g_kept;
+    Kept* k;
+    {
+        std::lock_guard<std::mutex> lk(g_mu);
+        auto& p = g_kept[current_device()];
+        if (!p) p = std::make_unique<Kept>();
+        k = p.get();
+    }
+    lock = std::unique_lock<std::mutex>(k->mu);
+    if (k->buf.bytes < bytes) {
+        int rc = k->buf.alloc(bytes);
+        if (rc) return rc;
+    }
+    base = static_cast<char*>(k->buf.p);
+    return TARA_OK;
+}
+
 int current_device()
 {
     int d = 0;

@@ -17,8 +17,12 @@
 // real row, of which entries 0..n/2 are kept; c2r builds the Hermitian row
 // from entries 0..n/2 with the imaginary parts of entry 0 and (even n) entry
 // n/2 taken as zero, which is what FFTW's c2r reads, and keeps the real part.
-// Workspace is allocated per call and the stream is synchronised before the
-// call returns.
+//
+// Up to kAnyLds elements a workgroup runs whole sequences through all passes in
+// LDS, from and to the caller's arrays (k_any_lds): one launch per transform, no
+// work space, no synchronisation.  Longer sequences take one launch per pass over
+// two global buffers, allocated per call, and the stream is synchronised before
+// the call returns.
 #include <vector>
 
 #include "common.h"
@@ -149,6 +153,199 @@ __global__ void k_any_real_out(const double2* __restrict__ w, double* __restrict
         x[idx] = w[idx].x * s;
 }
 
+// ------------------------------------------------------------ passes in LDS
+constexpr int kAnyLds = 2048;         // two buffers of 16-byte elements in 64 KB
+constexpr int kAnyPasses = 12;        // 2048 = 4^5 2 takes 6; at most 11 (2^11) for any schedule
+
+enum AnyKind { ANY_COL, ANY_R2C, ANY_C2R };
+
+struct AnyArgs {
+    const void* src;
+    void* dst;
+    int n, dir;
+    int seqs;                 // sequences per workgroup
+    long ntrans;
+    long es, pstride;         // columns: element stride, plane stride
+    int ncols;
+    int ld;                   // rows: pitch of the half spectra
+    double scale;             // c2r
+    int npass;
+    int radix[kAnyPasses];
+};
+
+// Butterflies of radix R of one pass (span s0 done): sequence c, output
+// position group t (see k_any_lds).  x, y: this sequence's buffers.
+template <int R>
+__device__ __forceinline__ void any_butterfly(const double2* x, double2* y, int n, int s0, unsigned t, int nl,
+                                              const double2* tw, int dir)
+{
+    const int nr = n / R;
+    const unsigned p = t / (unsigned)s0, q = t - p * s0;
+    double2 a[R];
+#pragma unroll
+    for (int j = 0; j < R; ++j) a[j] = x[t + j * nr];
+    double2 y_[R];
+    if constexpr (R == 2) {
+        y_[0] = make_double2(a[0].x + a[1].x, a[0].y + a[1].y);
+        y_[1] = make_double2(a[0].x - a[1].x, a[0].y - a[1].y);
+    } else if constexpr (R == 4) {
+        const double2 s02 = make_double2(a[0].x + a[2].x, a[0].y + a[2].y), d02 = make_double2(a[0].x - a[2].x, a[0].y - a[2].y);
+        const double2 s13 = make_double2(a[1].x + a[3].x, a[1].y + a[3].y), d13 = make_double2(a[1].x - a[3].x, a[1].y - a[3].y);
+        const double2 r = dir < 0 ? make_double2(d13.y, -d13.x) : make_double2(-d13.y, d13.x);  // -+i d13
+        y_[0] = make_double2(s02.x + s13.x, s02.y + s13.y);
+        y_[1] = make_double2(d02.x + r.x, d02.y + r.y);
+        y_[2] = make_double2(s02.x - s13.x, s02.y - s13.y);
+        y_[3] = make_double2(d02.x - r.x, d02.y - r.y);
+    } else {
+        double2 w[R];
+#pragma unroll
+        for (int k = 1; k < R; ++k) w[k] = root(tw, (long)k * nr, dir);
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            y_[u] = a[0];
+#pragma unroll
+            for (int j = 1; j < R; ++j) {
+                const int k = (j * u) % R;
+                if (k == 0) {
+                    y_[u].x += a[j].x;
+                    y_[u].y += a[j].y;
+                } else {
+                    y_[u].x += a[j].x * w[k].x - a[j].y * w[k].y;
+                    y_[u].y += a[j].x * w[k].y + a[j].y * w[k].x;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < R; ++u)
+        y[q + s0 * (R * p + u)] = (u == 0 || p == 0) ? y_[u] : cmul(y_[u], root(tw, (long)p * u * nl, dir));
+}
+
+// Whole transforms of a.seqs sequences.  Bound by latency on the grids that come
+// here (a 96 x 80 right-hand side is a few hundred KB): the passes of a transform
+// were a launch each, with two buffers allocated, a copy in and out and a
+// synchronisation around them, 1.5 ms for the six transforms of a derive2csh
+// call at 96 x 80 against 0.02 ms here (four launches of 6 us).
+template <AnyKind KIND>
+__global__ __launch_bounds__(256) void k_any_lds(AnyArgs a, const double2* __restrict__ tw)
+{
+    extern __shared__ double2 lds[];
+    const unsigned n = a.n, S = a.seqs, tid = threadIdx.x, nt = blockDim.x;
+    double2* x = lds;
+    double2* y = lds + S * n;
+    const long t0 = (long)blockIdx.x * S;
+    const unsigned live = (unsigned)(a.ntrans - t0 < (long)S ? a.ntrans - t0 : S);
+    if constexpr (KIND == ANY_COL) {
+        // sequences fastest: neighbouring columns are contiguous
+        const double2* src = static_cast<const double2*>(a.src);
+        for (unsigned b = tid; b < S * n; b += nt) {
+            const unsigned c = b % S, e = b / S;
+            const long t = t0 + (c < live ? c : 0), pl = t / a.ncols;
+            x[c * n + e] = src[pl * a.pstride + (long)e * a.es + (t - pl * a.ncols)];
+        }
+    } else if constexpr (KIND == ANY_R2C) {
+        const double* src = static_cast<const double*>(a.src) + t0 * n;
+        for (unsigned b = tid; b < live * n; b += nt) x[b] = make_double2(src[b], 0.0);
+    } else {
+        const double2* src = static_cast<const double2*>(a.src) + t0 * a.ld;
+        for (unsigned b = tid; b < live * n; b += nt) {
+            const unsigned c = b / n, k = b - c * n;
+            double2 v = src[(long)c * a.ld + (2 * k <= n ? k : n - k)];
+            if (k == 0 || 2 * k == n) v.y = 0.0;
+            if (2 * k > n) v.y = -v.y;
+            x[b] = v;
+        }
+    }
+    __syncthreads();
+    int s0 = 1;  // n / L: spans done
+    for (int ip = 0; ip < a.npass; ++ip) {
+        const int r = a.radix[ip], nr = n / r;
+        if (r <= 5) {
+            for (unsigned b = tid; b < S * nr; b += nt) {
+                const unsigned c = b / nr, t = b - c * nr;
+                const double2* xs = x + c * n;
+                double2* ys = y + c * n;
+                switch (r) {
+                    case 2: any_butterfly<2>(xs, ys, n, s0, t, s0, tw, a.dir); break;
+                    case 3: any_butterfly<3>(xs, ys, n, s0, t, s0, tw, a.dir); break;
+                    case 4: any_butterfly<4>(xs, ys, n, s0, t, s0, tw, a.dir); break;
+                    default: any_butterfly<5>(xs, ys, n, s0, t, s0, tw, a.dir); break;
+                }
+            }
+        } else {
+            // one output per thread: a large prime still spreads over the workgroup
+            for (unsigned b = tid; b < S * n; b += nt) {
+                const unsigned c = b / n, e = b - c * n;
+                const unsigned rest = e / (unsigned)s0, q = e - rest * s0, p = rest / (unsigned)r, u = rest - p * r;
+                const double2* xs = x + c * n + q + s0 * p;
+                double2 acc = make_double2(0.0, 0.0);
+                unsigned k = 0;  // j u mod r
+                for (int j = 0; j < r; ++j) {
+                    const double2 v = xs[j * nr], w = root(tw, (long)k * nr, a.dir);
+                    acc.x += v.x * w.x - v.y * w.y;
+                    acc.y += v.x * w.y + v.y * w.x;
+                    k += u;
+                    if (k >= (unsigned)r) k -= r;
+                }
+                y[c * n + e] = p * u == 0 ? acc : cmul(acc, root(tw, (long)p * u * s0, a.dir));
+            }
+        }
+        __syncthreads();
+        s0 *= r;
+        double2* z = x;
+        x = y;
+        y = z;
+    }
+    if constexpr (KIND == ANY_COL) {
+        double2* dst = static_cast<double2*>(a.dst);
+        for (unsigned b = tid; b < S * n; b += nt) {
+            const unsigned c = b % S, e = b / S;
+            const long t = t0 + c, pl = t / a.ncols;
+            if (c < live) dst[pl * a.pstride + (long)e * a.es + (t - pl * a.ncols)] = x[c * n + e];
+        }
+    } else if constexpr (KIND == ANY_R2C) {
+        double2* dst = static_cast<double2*>(a.dst) + t0 * a.ld;
+        const unsigned nh = n / 2 + 1;
+        for (unsigned b = tid; b < live * a.ld; b += nt) {
+            const unsigned c = b / a.ld, k = b - c * a.ld;
+            dst[b] = k < nh ? x[c * n + k] : make_double2(0.0, 0.0);
+        }
+    } else {
+        double* dst = static_cast<double*>(a.dst) + t0 * n;
+        for (unsigned b = tid; b < live * n; b += nt) dst[b] = x[b].x * a.scale;
+    }
+}
+
+// Whether length n runs in LDS; if so, the pass schedule and how many sequences
+// share a workgroup: up to 8 (columns: a 128-byte line) that fit 64 KB and still
+// leave 256 workgroups.
+bool any_lds(int n, long ntrans, AnyArgs& a)
+{
+    if (n > kAnyLds) return false;
+    a = AnyArgs{};
+    a.n = n;
+    a.ntrans = ntrans;
+    for (int r : radices(n)) a.radix[a.npass++] = r;
+    a.seqs = 8;
+    while (a.seqs > 1 && (2L * a.seqs * n * 16 > 65536 || ntrans / a.seqs < 256)) a.seqs /= 2;
+    return true;
+}
+
+template <AnyKind KIND>
+int launch_any_lds(const AnyArgs& a, hipStream_t st)
+{
+    const double2* tw = unit_roots(a.n);
+    TARA_CHECK(tw, TARA_ERR_ALLOC, "root table allocation failed (n = %d)", a.n);
+    const int work = a.seqs * a.n / 4;  // butterflies of a pass
+    const int nt = work >= 192 ? 256 : work >= 96 ? 128 : 64;
+    const long blocks = (a.ntrans + a.seqs - 1) / a.seqs;
+    TARA_CHECK(blocks <= 0x7fffffffL, TARA_ERR_UNSUPPORTED, "transform batch too large");
+    hipLaunchKernelGGL(k_any_lds<KIND>, dim3((unsigned)blocks), dim3(nt), 2 * (size_t)a.seqs * a.n * sizeof(double2), st,
+                       a, tw);
+    TARA_HIP(hipGetLastError());
+    return TARA_OK;
+}
+
 unsigned blocks_for(long n)
 {
     long b = (n + 255) / 256;
@@ -184,6 +381,15 @@ int any_col_fft(double2* a, int n, int ncols, long es, long pstride, int nplanes
     TARA_CHECK(n >= 1 && ncols >= 1 && nplanes >= 1, TARA_ERR_ARG, "any_col_fft: bad shape");
     if (n == 1) return TARA_OK;
     const long ntrans = (long)ncols * nplanes;
+    AnyArgs q;
+    if (any_lds(n, ntrans, q)) {
+        q.src = q.dst = a;
+        q.dir = dir;
+        q.es = es;
+        q.pstride = pstride;
+        q.ncols = ncols;
+        return launch_any_lds<ANY_COL>(q, st);
+    }
     DevBuf b0, b1;
     int rc;
     if ((rc = b0.alloc((size_t)ntrans * n * sizeof(double2))) || (rc = b1.alloc((size_t)ntrans * n * sizeof(double2))))
@@ -203,6 +409,14 @@ int any_col_fft(double2* a, int n, int ncols, long es, long pstride, int nplanes
 int any_row_r2c(const double* x, double2* X, int nx, int ld, int nrows, hipStream_t st)
 {
     TARA_CHECK(nx >= 1 && nrows >= 1 && ld >= nx / 2 + 1, TARA_ERR_ARG, "any_row_r2c: bad shape");
+    AnyArgs q;
+    if (any_lds(nx, nrows, q)) {
+        q.src = x;
+        q.dst = X;
+        q.dir = -1;
+        q.ld = ld;
+        return launch_any_lds<ANY_R2C>(q, st);
+    }
     const long total = (long)nrows * nx;
     DevBuf b0, b1;
     int rc;
@@ -221,6 +435,15 @@ int any_row_r2c(const double* x, double2* X, int nx, int ld, int nrows, hipStrea
 int any_row_c2r(const double2* X, double* x, int nx, int ld, int nrows, double s, hipStream_t st)
 {
     TARA_CHECK(nx >= 1 && nrows >= 1 && ld >= nx / 2 + 1, TARA_ERR_ARG, "any_row_c2r: bad shape");
+    AnyArgs q;
+    if (any_lds(nx, nrows, q)) {
+        q.src = X;
+        q.dst = x;
+        q.dir = +1;
+        q.ld = ld;
+        q.scale = s;
+        return launch_any_lds<ANY_C2R>(q, st);
+    }
     const long total = (long)nrows * nx;
     DevBuf b0, b1;
     int rc;

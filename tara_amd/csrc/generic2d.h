@@ -1,16 +1,13 @@
-// derive2csh / derive2css and their RK4 step on any grid (see generic2d.hip).
+// derive2csh / derive2css on grids the fused passes do not take (generic2d.hip).
 #pragma once
-#include "common.h"
 #include "csh2d.h"
 
 namespace tara {
 
-// True where the fused passes take the grid (powers of two, 32..4096 x 16..4096).
+// Whether the fused csh2d passes take an nx x ny grid.
 bool csh_fast_grid(int nx, int ny);
-// RHS of derive2csh (ph.screened == 0) or derive2css on device half spectra
-// of pitch spec_ld(nx), kx fastest; synchronous on st.
-int gen_csh_rhs(int nx, int ny, const CshPhys& ph, const double2* w, double2* f, hipStream_t st);
-// One classic RK4 step of that RHS, in place; synchronous on st.
-int gen_csh_rk4(int nx, int ny, const CshPhys& ph, double dt, double2* w, hipStream_t st);
+// out = the right-hand side of the nh x ny host spectrum in, or (step) one RK4
+// step of size dt from it.  Synchronous, on the null stream.
+int gen_csh_host(int nx, int ny, const CshPhys& ph, const double* in, double* out, bool step, double dt);
 
 }  // namespace tara

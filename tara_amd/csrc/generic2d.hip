@@ -4,13 +4,14 @@
 // the two real products, two r2c and the dealiased, viscous combination
 // (src/derive2csh.f95:29-145; src/derive2css.f95:20-130), each a device
 // kernel over half spectra of pitch spec_ld(nx) (kx fastest) or real planes
-// of pitch nx.  Slower than the fused path (about ten launches and one
-// workspace allocation per call) and used only where that path has no
-// kernel; the arithmetic is the same, term by term.
+// of pitch nx.  Slower than the fused path (seven launches in kept work space)
+// and used only where that path has no kernel; the arithmetic is the same, term
+// by term.
 #include "common.h"
 #include "csh2d.h"
 #include "fft_api.h"
 #include "generic2d.h"
+#include "layout.h"
 
 namespace tara {
 
@@ -41,11 +42,13 @@ __global__ void k_gen_spec(const double2* __restrict__ w, int nx, int ny, int ld
 {
     const int nh = nx / 2 + 1;
     const size_t plane = (size_t)ld * ny;
-    for (size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x; q < (size_t)nh * ny;
-         q += (size_t)gridDim.x * blockDim.x) {
-        const int i = (int)(q % nh), j = (int)(q / nh);
+    for (size_t p = blockIdx.x * (size_t)blockDim.x + threadIdx.x; p < plane; p += (size_t)gridDim.x * blockDim.x) {
+        const int i = (int)(p % ld), j = (int)(p / ld);
+        if (i >= nh) {  // padding columns stay zero through the y transforms
+            for (int f = 0; f < (screened ? 5 : 4); ++f) S[f * plane + p] = make_double2(0.0, 0.0);
+            continue;
+        }
         const double kx = csh_k(i, nx, true), ky = csh_k(j, ny, false);
-        const size_t p = (size_t)j * ld + i;
         const double wr = w[p].x, wi = w[p].y;
         const bool origin = i == 0 && j == 0;
         double2 ukx, uky, ikx, iky;
@@ -149,55 +152,95 @@ bool csh_fast_grid(int nx, int ny)
     return is_pow2(nx) && is_pow2(ny) && nx >= 32 && ny >= 16 && nx <= 4096 && ny <= 4096;
 }
 
-int gen_csh_rhs(int nx, int ny, const CshPhys& ph, const double2* w, double2* f, hipStream_t st)
+namespace {
+
+size_t rhs_bytes(int nx, int ny)
 {
-    TARA_CHECK(nx >= 2 && ny >= 1 && (double)nx * ny <= (double)(1L << 30), TARA_ERR_UNSUPPORTED,
-               "derive2csh: grid %dx%d unsupported", nx, ny);
+    const size_t plane = (size_t)spec_ld(nx) * ny, nr = (size_t)nx * ny;
+    return Scratch::pad(5 * plane * sizeof(double2)) + Scratch::pad(4 * nr * sizeof(double)) +
+           Scratch::pad(2 * plane * sizeof(double2));
+}
+
+// f = the right-hand side of w, with work space of rhs_bytes: S, R, N.
+struct RhsWs {
+    double2* S;
+    double* R;
+    double2* N;
+};
+RhsWs rhs_ws(int nx, int ny, Scratch& ws)
+{
+    const size_t plane = (size_t)spec_ld(nx) * ny, nr = (size_t)nx * ny;
+    RhsWs r;
+    r.S = ws.take<double2>(5 * plane);
+    r.R = ws.take<double>(4 * nr);
+    r.N = ws.take<double2>(2 * plane);
+    return r;
+}
+
+int rhs(int nx, int ny, const CshPhys& ph, const double2* w, double2* f, const RhsWs& m, hipStream_t st)
+{
     const int ld = spec_ld(nx);
     const size_t plane = (size_t)ld * ny, nr = (size_t)nx * ny;
-    DevBuf spec, real, nl;
     int rc;
-    if ((rc = spec.alloc(5 * plane * sizeof(double2))) || (rc = real.alloc(4 * nr * sizeof(double))) ||
-        (rc = nl.alloc(2 * plane * sizeof(double2))))
-        return rc;
-    double2* S = spec.as<double2>();
-    double* R = real.as<double>();
-    double2* N = nl.as<double2>();
-    TARA_HIP(hipMemsetAsync(S, 0, spec.bytes, st));
-    hipLaunchKernelGGL(k_gen_spec, dim3(blocks_for((size_t)(nx / 2 + 1) * ny)), dim3(256), 0, st, w, nx, ny, ld,
-                       ph.screened, ph.lambda, S);
+    hipLaunchKernelGGL(k_gen_spec, dim3(blocks_for(plane)), dim3(256), 0, st, w, nx, ny, ld, ph.screened, ph.lambda,
+                       m.S);
     TARA_HIP(hipGetLastError());
-    if ((rc = col_fft(S, ny, ld, ld, (long)plane, 4, +1, st))) return rc;
-    if ((rc = row_c2r(S, R, nx, ld, 4 * ny, 1.0, st))) return rc;
-    hipLaunchKernelGGL(k_gen_prod, dim3(blocks_for(nr)), dim3(256), 0, st, R, nr, (double)nx * (double)ny);
+    if ((rc = col_fft(m.S, ny, ld, ld, (long)plane, 4, +1, st))) return rc;
+    if ((rc = row_c2r(m.S, m.R, nx, ld, 4 * ny, 1.0, st))) return rc;
+    hipLaunchKernelGGL(k_gen_prod, dim3(blocks_for(nr)), dim3(256), 0, st, m.R, nr, (double)nx * (double)ny);
     TARA_HIP(hipGetLastError());
-    if ((rc = row_r2c(R + 2 * nr, N, nx, ld, 2 * ny, st))) return rc;
-    if ((rc = col_fft(N, ny, ld, ld, (long)plane, 2, -1, st))) return rc;
-    hipLaunchKernelGGL(k_gen_final, dim3(blocks_for(plane)), dim3(256), 0, st, N, w, S + 4 * plane, nx, ny, ld,
+    if ((rc = row_r2c(m.R + 2 * nr, m.N, nx, ld, 2 * ny, st))) return rc;
+    if ((rc = col_fft(m.N, ny, ld, ld, (long)plane, 2, -1, st))) return rc;
+    hipLaunchKernelGGL(k_gen_final, dim3(blocks_for(plane)), dim3(256), 0, st, m.N, w, m.S + 4 * plane, nx, ny, ld,
                        ph.nu, ph.alpha, ph.screened, f);
     TARA_HIP(hipGetLastError());
-    TARA_HIP(hipStreamSynchronize(st));
     return TARA_OK;
 }
 
-int gen_csh_rk4(int nx, int ny, const CshPhys& ph, double dt, double2* w, hipStream_t st)
+int rk4(int nx, int ny, const CshPhys& ph, double dt, double2* w, const RhsWs& m, double2* k, double2* s, hipStream_t st)
 {
     const size_t n = (size_t)spec_ld(nx) * ny;
-    DevBuf kb, sb;
     int rc;
-    if ((rc = kb.alloc(4 * n * sizeof(double2))) || (rc = sb.alloc(n * sizeof(double2)))) return rc;
-    double2* k = kb.as<double2>();
-    double2* s = sb.as<double2>();
-    if ((rc = gen_csh_rhs(nx, ny, ph, w, k, st))) return rc;
+    if ((rc = rhs(nx, ny, ph, w, k, m, st))) return rc;
     hipLaunchKernelGGL(k_gen_axpy, dim3(blocks_for(n)), dim3(256), 0, st, w, k, 0.5 * dt, s, n);
-    if ((rc = gen_csh_rhs(nx, ny, ph, s, k + n, st))) return rc;
+    if ((rc = rhs(nx, ny, ph, s, k + n, m, st))) return rc;
     hipLaunchKernelGGL(k_gen_axpy, dim3(blocks_for(n)), dim3(256), 0, st, w, k + n, 0.5 * dt, s, n);
-    if ((rc = gen_csh_rhs(nx, ny, ph, s, k + 2 * n, st))) return rc;
+    if ((rc = rhs(nx, ny, ph, s, k + 2 * n, m, st))) return rc;
     hipLaunchKernelGGL(k_gen_axpy, dim3(blocks_for(n)), dim3(256), 0, st, w, k + 2 * n, dt, s, n);
-    if ((rc = gen_csh_rhs(nx, ny, ph, s, k + 3 * n, st))) return rc;
+    if ((rc = rhs(nx, ny, ph, s, k + 3 * n, m, st))) return rc;
     hipLaunchKernelGGL(k_gen_rk4, dim3(blocks_for(n)), dim3(256), 0, st, w, k, k + n, k + 2 * n, k + 3 * n, dt, n);
     TARA_HIP(hipGetLastError());
-    TARA_HIP(hipStreamSynchronize(st));
+    return TARA_OK;
+}
+
+}  // namespace
+
+int gen_csh_host(int nx, int ny, const CshPhys& ph, const double* in, double* out, bool step, double dt)
+{
+    TARA_CHECK(nx >= 2 && ny >= 1 && (double)nx * ny <= (double)(1L << 30), TARA_ERR_UNSUPPORTED,
+               "derive2csh: grid %dx%d unsupported", nx, ny);
+    const int ld = spec_ld(nx), nh = nx / 2 + 1;
+    const size_t plane = (size_t)ld * ny, host = (size_t)nh * ny, b = Scratch::pad(plane * sizeof(double2));
+    Scratch ws;
+    int rc;
+    if ((rc = ws.open(rhs_bytes(nx, ny) + 3 * b + (step ? Scratch::pad(4 * plane * sizeof(double2)) + b : 0)))) return rc;
+    hipStream_t st = nullptr;
+    double2 *pack = ws.take<double2>(plane), *w = ws.take<double2>(plane), *f = ws.take<double2>(plane);
+    const RhsWs m = rhs_ws(nx, ny, ws);
+    DevBuf pb;
+    pb.view(pack, host * sizeof(double2));
+    if ((rc = rows_from_host(&w, &in, 1, nh, ld, ny, pb, st))) return rc;
+    if (step) {
+        double2 *k = ws.take<double2>(4 * plane), *s = ws.take<double2>(plane);
+        rc = rk4(nx, ny, ph, dt, w, m, k, s, st);
+    } else {
+        rc = rhs(nx, ny, ph, w, f, m, st);
+    }
+    if (!rc) rc = rows_to_host(&out, step ? &w : &f, 1, nh, ld, ny, pb, st);
+    // the work space goes back: nothing may still run in it, after an error either
+    const hipError_t e = hipStreamSynchronize(st);
+    if (rc) return rc;
+    TARA_HIP(e);
     return TARA_OK;
 }
 

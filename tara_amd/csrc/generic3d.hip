@@ -9,6 +9,7 @@
 #include "common.h"
 #include "fft_api.h"
 #include "generic3d.h"
+#include "layout.h"
 
 namespace tara {
 
@@ -162,9 +163,16 @@ int gen_derive3com_host(int nx, int ny, int nz, const tara_mhd_params* prm, cons
     double *R = rb.as<double>(), *F = fb.as<double>();
     hipStream_t st = nullptr;
     TARA_HIP(hipMemset(S, 0, sb.bytes));
-    for (int f = 0; f < 7; ++f)
-        TARA_HIP(hipMemcpy2D(S + f * fsz, ld * sizeof(double2), state[kLive[f]], nh * sizeof(double2),
-                             nh * sizeof(double2), rows, hipMemcpyHostToDevice));
+    // the flux spectra's buffer is free until the transforms and after the assembly: it packs the rows
+    double2* dev[7];
+    const double* hin[7];
+    double* hout[7];
+    for (int f = 0; f < 7; ++f) {
+        dev[f] = S + f * fsz;
+        hin[f] = state[kLive[f]];
+        hout[f] = rhs[kLive[f]];
+    }
+    if ((rc = rows_from_host(dev, hin, 7, nh, ld, rows, kb, st))) return rc;
     TARA_HIP(hipMemcpy(Cs, S, sb.bytes, hipMemcpyDeviceToDevice));
     for (int f = 0; f < 7; ++f)
         if ((rc = c2r3(Cs + f * fsz, R + f * nr, nx, ny, nz, ld, st))) return rc;
@@ -177,9 +185,9 @@ int gen_derive3com_host(int nx, int ny, int nz, const tara_mhd_params* prm, cons
     hipLaunchKernelGGL(k3_assemble, dim3(blocks_for(fsz)), dim3(256), 0, st, S, K, O, nx, ny, nz, ld, fsz, prm->lx,
                        prm->ly, prm->lz, prm->mu, prm->eta);
     TARA_HIP(hipGetLastError());
-    for (int f = 0; f < 7; ++f)
-        TARA_HIP(hipMemcpy2D(rhs[kLive[f]], nh * sizeof(double2), O + f * fsz, ld * sizeof(double2),
-                             nh * sizeof(double2), rows, hipMemcpyDeviceToHost));
+    for (int f = 0; f < 7; ++f) dev[f] = O + f * fsz;
+    if ((rc = rows_to_host(hout, dev, 7, nh, ld, rows, kb, st))) return rc;
+    TARA_HIP(hipStreamSynchronize(st));
     for (size_t q = 0; q < 2 * (size_t)nh * rows; ++q) rhs[4][q] = 0.0;
     return TARA_OK;
 }

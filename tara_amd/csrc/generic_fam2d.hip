@@ -14,6 +14,7 @@
 #include "common.h"
 #include "fft_api.h"
 #include "generic_fam2d.h"
+#include "layout.h"
 
 namespace tara {
 
@@ -230,17 +231,23 @@ int r2c_planes(const double* r, double2* s, const Grid& g, int nf, hipStream_t s
 
 int upload(const Grid& g, double2* d, const double* const h[], int nf)
 {
-    for (int f = 0; f < nf; ++f)
-        TARA_HIP(hipMemcpy2D(d + f * g.plane, g.ld * sizeof(double2), h[f], g.nh * sizeof(double2),
-                             g.nh * sizeof(double2), g.ny, hipMemcpyHostToDevice));
+    DevBuf pack;
+    double2* dev[6];
+    for (int f = 0; f < nf; ++f) dev[f] = d + f * g.plane;
+    int rc = pack.alloc((size_t)nf * g.nh * g.ny * sizeof(double2));
+    if (rc || (rc = rows_from_host(dev, h, nf, g.nh, g.ld, g.ny, pack, nullptr))) return rc;
+    TARA_HIP(hipStreamSynchronize(nullptr));
     return TARA_OK;
 }
 
 int download(const Grid& g, double* const h[], const double2* d, int nf)
 {
-    for (int f = 0; f < nf; ++f)
-        TARA_HIP(hipMemcpy2D(h[f], g.nh * sizeof(double2), d + f * g.plane, g.ld * sizeof(double2),
-                             g.nh * sizeof(double2), g.ny, hipMemcpyDeviceToHost));
+    DevBuf pack;
+    const double2* dev[6];
+    for (int f = 0; f < nf; ++f) dev[f] = d + f * g.plane;
+    int rc = pack.alloc((size_t)nf * g.nh * g.ny * sizeof(double2));
+    if (rc || (rc = rows_to_host(h, dev, nf, g.nh, g.ld, g.ny, pack, nullptr))) return rc;
+    TARA_HIP(hipStreamSynchronize(nullptr));
     return TARA_OK;
 }
 
