@@ -11,7 +11,8 @@
 // The per-sample scale s makes the map equivariant to the field's amplitude,
 // and the residual form leaves the network the increment over T to learn.
 //
-// Every linear map is a GEMM on the MFMA units (gemm.hip).  With MX x MY
+// Every linear map is a GEMM on the MFMA units (gemm.hip; in bfloat16 the parts of
+// a layer that work on real-space rows run as one kernel, fno_layer.hip).  With MX x MY
 // retained modes, the transforms are truncated DFTs: per channel an
 // (N x N) x (N x MX) product along x and an (MY x 2N) x (2N x MX) product along
 // y, rather than full FFTs that would compute (N/2+1) N modes to keep MX MY.
@@ -36,6 +37,7 @@
 #include <vector>
 
 #include "ens.h"
+#include "fno_layer.h"
 #include "gemm.h"
 
 namespace tara {
@@ -294,6 +296,10 @@ struct tara_fno {
     DevBuf rs, rsb;                // stacked per-mode matrices of every layer (float, bfloat16)
     DevBuf fxt, fy2, g2, hx;     // truncated DFT matrices (float)
     DevBuf fxtb, fy2b, g2b, hxb;  // the same in bfloat16
+    // fused layers (bfloat16, shapes of fno_fused_ok): padded x transforms and
+    // padded copies of the mixing and projection weights
+    bool fused = false;
+    DevBuf fxp, hxtp, wp, w1p, b1p, w2p;
     // activations, sized for maxb samples
     DevBuf sig, v, vb, pre, x, xb, t1, y, yb, zf, zb, kv, hpre, hb, out, dproj, loss;
     DevBuf dva, dvb, dz, dy, dx, dt1, drs, dhpre, part;
@@ -413,9 +419,21 @@ int forward(tara_fno* f, int nb, const float* om, float* out, bool train)
     int rc;
     if ((rc = rms(f, nb, om))) return rc;
     const bool keep32 = train || !bf;  // FP32 activations needed
-    hipLaunchKernelGGL(k_lift, dim3((unsigned)((np + 255) / 256), (unsigned)F), dim3(256), 0, f->st, om,
+    const bool fused = f->fused;
+    FnoLayerArgs fl{};
+    if (fused) {
+        fl.n = n, fl.c = c, fl.q2 = q2, fl.nb = nb;
+        fl.om = om, fl.sig = P<float>(f->sig);
+        fl.wl = par + f->o_wl, fl.bl = par + f->o_bl;
+        fl.z = P<uint16_t>(f->zb);
+        fl.hxt = P<uint16_t>(f->hxtp), fl.fx = P<uint16_t>(f->fxp);
+        fl.w1 = P<uint16_t>(f->w1p), fl.b1 = P<float>(f->b1p), fl.w2 = P<float>(f->w2p), fl.b2 = par + f->o_b2;
+        fl.t1 = P<uint16_t>(f->t1);
+        if ((rc = fno_lift_x(fl, f->st))) return rc;
+    }
+    if (!fused || train) hipLaunchKernelGGL(k_lift, dim3((unsigned)((np + 255) / 256), (unsigned)F), dim3(256), 0, f->st, om,
                        P<float>(f->sig), par + f->o_wl, par + f->o_bl, keep32 ? P<float>(f->v) : nullptr,
-                       bf ? P<uint16_t>(f->vb) : nullptr, c, np);
+                       bf && !fused ? P<uint16_t>(f->vb) : nullptr, c, np);
     float* Y = P<float>(f->y);
     float* Z = P<float>(f->zf);
     float* kv = P<float>(f->kv);
@@ -424,7 +442,7 @@ int forward(tara_fno* f, int nb, const float* om, float* out, bool train)
         const size_t vo = (size_t)(train ? l : l % 2) * f->field;
         const size_t vn = (size_t)(train ? l + 1 : (l + 1) % 2) * f->field;
         const void* vin = bf ? (const void*)P<uint16_t>(f->vb, vo) : (const void*)P<float>(f->v, vo);
-        {  // 1. along x, per row y: T1[y][q][bc] = sum_x FxT[q][x] v[bc][y][x]
+        if (!fused) {  // 1. along x, per row y: T1[y][q][bc] = sum_x FxT[q][x] v[bc][y][x]
             GemmArgs g;
             g.m = q2, g.n = F, g.k = n;
             g.a = bf ? f->fxtb.p : f->fxt.p, g.sam = n, g.sak = 1;
@@ -475,6 +493,21 @@ int forward(tara_fno* f, int nb, const float* om, float* out, bool train)
             g.nb1 = mx, g.sb1 = F, g.sc1 = 1;
             if ((rc = gemm(g, dt, bf ? GEMM_STORE_BF16 : GEMM_STORE_F32, f->st))) return rc;
         }
+        if (fused) {  // 5, 6 and the next layer's 1, or (inference) the projection
+            const int CP = fno_pad(c);
+            const bool last = l == f->layers - 1;
+            fl.act = last ? 0 : 1;
+            fl.v = l == 0 ? nullptr : P<uint16_t>(f->vb, vo);
+            fl.w = P<uint16_t>(f->wp, (size_t)l * CP * CP);
+            fl.bias = par + f->o_b + (size_t)l * c;
+            fl.vn = last && !train ? nullptr : P<uint16_t>(f->vb, vn);
+            fl.t1 = last ? nullptr : P<uint16_t>(f->t1);
+            fl.pre = train ? P<float>(f->pre, (size_t)l * f->field) : nullptr;
+            fl.v32 = train ? P<float>(f->v, vn) : nullptr;
+            fl.out = last && !train ? out : nullptr;
+            if ((rc = fno_layer(fl, f->st))) return rc;
+            continue;
+        }
         {  // 5. inverse along x: Kv[bc][y][x] = sum_j Z[bc][y][j] Hx[j][x]
             GemmArgs g;
             g.m = F * n, g.n = n, g.k = q2;
@@ -501,6 +534,7 @@ int forward(tara_fno* f, int nb, const float* om, float* out, bool train)
             if ((rc = gemm(g, dt, GEMM_ADD_TO, f->st))) return rc;
         }
     }
+    if (fused && !train) return TARA_OK;  // projected by the last layer
     // projection: hpre[b][j][p] = W1[j][c] v[b][c][p] + b1[j]; out = omega + s (w2 . gelu(hpre) + b2)
     const size_t vl = (size_t)(train ? f->layers : f->layers % 2) * f->field;
     const int H = f->hdim;
@@ -676,6 +710,18 @@ int refresh_weights(tara_fno* f)
                            f->par.as<float>() + f->o_r + (size_t)l * f->r_sz, P<float>(f->rs, l * M * c2 * c2),
                            P<uint16_t>(f->rsb, l * M * c2 * c2), (int)M, c);
     TARA_HIP(hipGetLastError());
+    if (f->fused) {
+        const int CP = fno_pad(c);
+        int rc;
+        for (int l = 0; l < f->layers; ++l)
+            if ((rc = fno_pad_weights(f->par.as<float>() + f->o_w + (size_t)l * c * c, c, c,
+                                      P<uint16_t>(f->wp, (size_t)l * CP * CP), CP, CP, f->st)))
+                return rc;
+        if ((rc = fno_pad_weights(f->par.as<float>() + f->o_w1, 2 * c, c, P<uint16_t>(f->w1p), 2 * CP, CP, f->st)) ||
+            (rc = fno_pad_vector(f->par.as<float>() + f->o_b1, 2 * c, P<float>(f->b1p), 2 * CP, f->st)) ||
+            (rc = fno_pad_vector(f->par.as<float>() + f->o_w2, 2 * c, P<float>(f->w2p), 2 * CP, f->st)))
+            return rc;
+    }
     return TARA_OK;
 }
 
@@ -770,6 +816,20 @@ extern "C" int tara_fno_create(int n, int width, int mx, int my, int layers, int
         (rc = upload(f->hx, hx)) || (rc = upload_bf(f->fxtb, fxt)) || (rc = upload_bf(f->fy2b, fy2)) ||
         (rc = upload_bf(f->g2b, g2)) || (rc = upload_bf(f->hxb, hx)))
         return rc;
+    f->fused = precision == 0 && fno_fused_ok(n, width, 2 * mx) && max_batch <= 65535;
+    if (f->fused) {
+        const int q2 = 2 * mx, CP = fno_pad(width);
+        std::vector<float> fxp(32 * 256, 0.f), hxtp(256 * 32, 0.f);
+        for (int q = 0; q < q2; ++q)
+            for (int x = 0; x < n; ++x) {
+                fxp[q * 256 + x] = fxt[q * n + x];
+                hxtp[x * 32 + q] = hx[q * n + x];
+            }
+        if ((rc = upload_bf(f->fxp, fxp)) || (rc = upload_bf(f->hxtp, hxtp)) ||
+            (rc = f->wp.alloc(L * CP * CP * 2)) || (rc = f->w1p.alloc(2 * CP * CP * 2)) ||
+            (rc = f->b1p.alloc(2 * CP * 4)) || (rc = f->w2p.alloc(2 * CP * 4)))
+            return rc;
+    }
     // activations
     const size_t B = max_batch, np = f->np;
     f->field = B * c * np;
