@@ -280,7 +280,7 @@ int csh_ctx_zero_history(tara_csh* c)
     TARA_CHECK(c, TARA_ERR_ARG, "null context");
     TARA_HIP(hipMemsetAsync(c->aux.p, 0, c->aux.bytes, c->st));
     int rc = csh_clear_nonfinite(c->plan, -1, c->st);  // a new state: the guard starts over
-    if (rc) return rc;
+    if (rc || (rc = csh_state_set(c->plan, c->w.as<double2>(), 0, c->st))) return rc;
     TARA_HIP(hipStreamSynchronize(c->st));
     return TARA_OK;
 }

@@ -226,7 +226,9 @@ extern "C" int tara_ens_upload(tara_ens* e, int run, const double* omegak)
     if ((rc = to_kymajor(b->stage.as<double2>(), b->w.as<double2>() + slot * p.bstride, p.nh, p.ny, 1, nullptr)))
         return rc;
     TARA_HIP(hipMemset(b->aux.as<double2>() + slot * p.bstride, 0, p.bstride * sizeof(double2)));
-    if ((rc = csh_clear_nonfinite(p, slot, nullptr))) return rc;
+    if ((rc = csh_clear_nonfinite(p, slot, nullptr)) ||
+        (rc = csh_state_set(p, b->w.as<double2>() + slot * p.bstride, slot, nullptr)))
+        return rc;
     TARA_HIP(hipDeviceSynchronize());
     return TARA_OK;
 }
@@ -254,7 +256,9 @@ extern "C" int tara_ens_ic_random(tara_ens* e, int run, unsigned seed, double k0
     if ((rc = csh_random_phase(b->w.as<double2>() + slot * p.bstride, b->n, b->n, seed, k0, energy, e->st)))
         return rc;
     TARA_HIP(hipMemsetAsync(b->aux.as<double2>() + slot * p.bstride, 0, p.bstride * sizeof(double2), e->st));
-    if ((rc = csh_clear_nonfinite(p, slot, e->st))) return rc;
+    if ((rc = csh_clear_nonfinite(p, slot, e->st)) ||
+        (rc = csh_state_set(p, b->w.as<double2>() + slot * p.bstride, slot, e->st)))
+        return rc;
     TARA_HIP(hipStreamSynchronize(e->st));
     return TARA_OK;
 }
@@ -275,7 +279,8 @@ extern "C" int tara_ens_set_omega(tara_ens* e, int run, const float* omega)
                        b->spec.as<double2>(), ld, p.nh, n, b->w.as<double2>() + slot * p.bstride);
     TARA_HIP(hipGetLastError());
     TARA_HIP(hipMemsetAsync(b->aux.as<double2>() + slot * p.bstride, 0, p.bstride * sizeof(double2), e->st));
-    return csh_clear_nonfinite(p, slot, e->st);
+    if ((rc = csh_clear_nonfinite(p, slot, e->st))) return rc;
+    return csh_state_set(p, b->w.as<double2>() + slot * p.bstride, slot, e->st);
 }
 
 extern "C" int tara_ens_get_omega(tara_ens* e, int run, float* omega)

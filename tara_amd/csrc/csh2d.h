@@ -75,6 +75,14 @@ struct CshPlan {
     int xcfg = 0;                    // x-pass shape (see csh_xshape_ok / the autotuner)
     const double2* rctw = nullptr;
     DevBuf bad;                      // int per run: set when a step's new state holds a non-finite value
+    // The nonlinear term lives in kx < hk (and there inside the circle imin): the x
+    // pass stores and the forward y pass reads only those columns of H.
+    int hk = 0;
+    // int per run: the state is zero outside the circle (csh_state_set looks when a
+    // state is set; such a state stays zero there, since the viscous term is the only
+    // one outside).  Then the inverse y pass skips the columns kx >= hk, the x pass
+    // reads none of them, and the update touches the circle only.
+    DevBuf band;
 };
 // The per-run non-finite flags of a plan: csh_nonfinite synchronises st and
 // returns the number of flagged runs (flags[r] = 0 / 1 when flags is not null);
@@ -94,6 +102,11 @@ struct CshPhys {
     const double* nus = nullptr;  // batched runs: device array of nu per run (overrides nu)
 };
 
+// Columns kx below the dealiasing cut at ky = 0 (CshPlan::hk).
+int csh_live_columns(int nx, int ny);
+// To be called, ordered on st, whenever run `run`'s state w was set (not by the
+// steps themselves): finds its support for the passes.
+int csh_state_set(const CshPlan& p, const double2* w, int run, hipStream_t st);
 // batch: number of independent runs of this grid the launches cover; every
 // per-run field (state, G0..G3, H) is packed run after run, bstride apart.
 int csh_plan_init(CshPlan& p, int nx, int ny, int batch = 1);

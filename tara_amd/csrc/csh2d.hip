@@ -27,6 +27,15 @@
 //                        (:108-125), add nu k^2 omega (:127-139), negate
 //                        (:141-145), then the fused update (RHS / AB2 / RK4 stage).
 //
+// What the passes carry (CshPlan::hk, band): the nonlinear term is zero outside the
+// dealiasing circle, so H is stored, read and transformed for kx < hk only (a
+// third of its columns less), whatever the state; and a state that is zero
+// outside the circle stays so, so its passes leave the columns kx >= hk of
+// G0..G3 and the state's modes outside the circle alone (all but 35 % of them at
+// Nx = Ny).  The passes' time at 1024^2 and above is that traffic and what it
+// waits for: RK4 step 4096^2 2.30 -> 1.61 ms, 2048^2 0.58 -> 0.415, 1024^2 0.147
+// -> 0.139 for such states; 1024^2 0.147 -> 0.143 for others.
+//
 // Wavenumbers: derive2csh uses pi = 3.1428 (a default-real literal) and
 // Lx = Ly = 2 pi (:16-21), so kx = i-1 and ky = j-1 or j-1-Ny are exact integers;
 // the host builds the tables with that exact expression (csh_plan_init).
@@ -126,7 +135,8 @@ template <int NY, bool SCR, int GS>
 __global__ __launch_bounds__((YiShape<NY, SCR>::NT), (YiShape<NY, SCR>::IL ? 4 : 1)) void k_csh_yinv(const double2* w, int nh,
                                                                     double2* __restrict__ g0, double2* __restrict__ g1,
                                                                     double2* __restrict__ g2, double2* __restrict__ g3,
-                                                                    const double2* tw, double lam, int ld, size_t bs)
+                                                                    const double2* tw, double lam, int ld, size_t bs,
+                                                                    CshBand bd)
 {
     // batched runs: blockIdx.y selects the run, every field is strided by bs
     const size_t rb = blockIdx.y * bs;
@@ -140,12 +150,20 @@ __global__ __launch_bounds__((YiShape<NY, SCR>::NT), (YiShape<NY, SCR>::IL ? 4 :
     __shared__ double2 lds[S::LDS_ELEMS];
     const int c = S::IL ? (int)threadIdx.x % S::CB : (int)threadIdx.x / T;
     const int t = S::IL ? (int)threadIdx.x / S::CB : (int)threadIdx.x % T;
-    const int i = xcd_remap(blockIdx.x, gridDim.x) * S::CB + c;
-    const bool live = i < nh;
+    // a limited state: the kx columns that hold something, and of them the modes
+    const bool lim = bd.limited(blockIdx.y);
+    const int ncol = lim ? bd.hk : nh, ntile = (ncol + S::CB - 1) / S::CB;
+    if ((int)blockIdx.x >= ntile) return;
+    const int i = xcd_remap(blockIdx.x, ntile) * S::CB + c;
+    const bool live = i < ncol;
     const size_t col = (size_t)(live ? i : 0) * NY;
     double2 wv[E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) wv[e] = live ? w[col + rf_first_idx<NY, csh_yem(NY)>(t, e)] : make_double2(0.0, 0.0);
+    for (int e = 0; e < E; ++e) {
+        const int j = rf_first_idx<NY, csh_yem(NY)>(t, e);
+        wv[e] = make_double2(0.0, 0.0);
+        if (live && (!lim || i < bd.imin[j])) wv[e] = w[col + j];
+    }
     csh_yinv_column<NY, SCR, GS, S::IL>(wv, i, live, t, lds + c * S::LDSC, tw, lam, ld, g0, g1, g2, g3);
 }
 
@@ -170,9 +188,10 @@ struct XShape {
 template <int NX, int EM, int RB, bool SPLIT>
 __global__ __launch_bounds__((XShape<NX, EM, RB, SPLIT>::NT)) void k_csh_x(
     const double2* g0, const double2* g1, const double2* g2, const double2* g3, double scale,
-    double2* __restrict__ h, const double2* tw_n, const double2* tw_m, const double2* rctw, size_t bs)
+    double2* __restrict__ h, const double2* tw_n, const double2* tw_m, const double2* rctw, size_t bs, CshBand bd)
 {
     const size_t rb = blockIdx.y * bs;  // batched runs
+    const int lim = bd.limited(blockIdx.y) ? bd.hk : bd.nh;
     g0 += rb;
     g1 += rb;
     g2 += rb;
@@ -187,10 +206,10 @@ __global__ __launch_bounds__((XShape<NX, EM, RB, SPLIT>::NT)) void k_csh_x(
     double2* xl = lds + r * S::LDSR;
     double nl[E];
     double2 v[E];
-    x_c2r_pair<NX, EM, SPLIT>(g0, g2, j, t, xl, tw_n, v);   // ux + i d omega/dx
+    x_c2r_pair<NX, EM, SPLIT>(g0, g2, j, lim, t, xl, tw_n, v);   // ux + i d omega/dx
 #pragma unroll
     for (int e = 0; e < E; ++e) nl[e] = v[e].x * v[e].y;
-    x_c2r_pair<NX, EM, SPLIT>(g1, g3, j, t, xl, tw_n, v);   // uy + i d omega/dy
+    x_c2r_pair<NX, EM, SPLIT>(g1, g3, j, lim, t, xl, tw_n, v);   // uy + i d omega/dy
 #pragma unroll
     for (int e = 0; e < E; ++e) nl[e] = (nl[e] + v[e].x * v[e].y) * scale;
     // forward x transform of the real product row: pack z[m] = nl[2m] + i nl[2m+1]
@@ -237,17 +256,18 @@ __global__ __launch_bounds__((XShape<NX, EM, RB, SPLIT>::NT)) void k_csh_x(
 #pragma unroll
     for (int u = 0; u < NK; ++u) {  // consecutive t -> consecutive kx
         const int k = t + u * T;
+        if (k >= bd.hk) continue;  // dealiased away at every ky
         const double2 zk = xl[rf_pad(k)];
         const double2 zmk = xl[rf_pad(k == 0 ? 0 : M - k)];
         double2 xm;
         h[blk8(k, j, M + 1)] = r2c_unpack_w(zk, zmk, k, wk[u], &xm);
-        if (k == 0) h[blk8(M, j, M + 1)] = xm;
+        if (k == 0 && M < bd.hk) h[blk8(M, j, M + 1)] = xm;
     }
 }
 
 // --------------------------------------------------------------------- pass 3
 template <int NY, int MODE>
-__global__ __launch_bounds__(YShape<NY>::NT) void k_csh_yfwd(YfwdArgs a, const double2* tw)
+__global__ __launch_bounds__(YShape<NY>::NT) void k_csh_yfwd(YfwdArgs a, CshBand bd, const double2* tw)
 {
     const size_t rb = blockIdx.y * a.bs;
     a.h += rb;
@@ -260,13 +280,22 @@ __global__ __launch_bounds__(YShape<NY>::NT) void k_csh_yfwd(YfwdArgs a, const d
     constexpr int E = RY<NY>::E, T = S::T;
     __shared__ double2 lds[S::CB * RY<NY>::LDS];
     const int c = threadIdx.x / T, t = threadIdx.x % T;
-    const int i = xcd_remap(blockIdx.x, gridDim.x) * S::CB + c;
-    const bool live = i < a.nh;
+    // tiles below hk have a nonlinear term; the others only the viscous one, and a
+    // limited state nothing
+    const bool lim = bd.limited(blockIdx.y);
+    const int nfwd = (bd.hk + S::CB - 1) / S::CB;
+    if (lim && (int)blockIdx.x >= nfwd) return;
+    const int tile = csh_tile(blockIdx.x, nfwd, gridDim.x);
+    const int i = tile * S::CB + c;
+    const bool live = i < (lim ? bd.hk : a.nh);
     const size_t col = (size_t)(live ? i : 0) * NY;
     double2 v[E];
+    if (tile < nfwd) {
 #pragma unroll
-    for (int e = 0; e < E; ++e) v[e] = live ? a.h[blk8(i, rf_first_idx<NY, csh_yem(NY)>(t, e), a.nh)] : make_double2(0.0, 0.0);
-    rf_fft<NY, -1, csh_yem(NY)>(v, t, lds + c * RY<NY>::LDS, tw);
+        for (int e = 0; e < E; ++e)
+            v[e] = i < bd.hk ? a.h[blk8(i, rf_first_idx<NY, csh_yem(NY)>(t, e), a.nh)] : make_double2(0.0, 0.0);
+        rf_fft<NY, -1, csh_yem(NY)>(v, t, lds + c * RY<NY>::LDS, tw);
+    }
     if (!live) return;
     const double kxv = (double)i;
     bool finite = true;  // the new state's values (AB2, RK4 stage 4)
@@ -275,7 +304,10 @@ __global__ __launch_bounds__(YShape<NY>::NT) void k_csh_yfwd(YfwdArgs a, const d
         const int j = rf_final_idx<NY, csh_yem(NY)>(t, e);
         const size_t q = col + j;
         double2 nl = v[e];
-        if (i >= a.imin[j]) nl = make_double2(0.0, 0.0);
+        if (i >= a.imin[j]) {
+            if (lim) continue;  // zero, and stays so
+            nl = make_double2(0.0, 0.0);
+        }
         const double kyv = csh_ky<NY>(j);
         const double k2 = kxv * kxv + kyv * kyv;
         double2 wn, av;
@@ -294,7 +326,7 @@ __global__ __launch_bounds__(YShape<NY>::NT) void k_csh_yfwd(YfwdArgs a, const d
 // LDS as the inverse y pass; the forward y pass of H uses the same lanes.
 template <int NY, int MODE, int GS>
 __global__ __launch_bounds__((YiShape<NY, false>::NT), (YiShape<NY, false>::IL ? 4 : 1)) void k_csh_yfwd_inv(
-    YfwdArgs a, const double2* tw, double2* __restrict__ g0, double2* __restrict__ g1, double2* __restrict__ g2,
+    YfwdArgs a, CshBand bd, const double2* tw, double2* __restrict__ g0, double2* __restrict__ g1, double2* __restrict__ g2,
     double2* __restrict__ g3, int ld)
 {
     static_assert(MODE != CSH_RHS, "the fused pass needs a stage update");
@@ -315,26 +347,40 @@ __global__ __launch_bounds__((YiShape<NY, false>::NT), (YiShape<NY, false>::IL ?
     __shared__ double2 lds[S::LDS_ELEMS];
     const int c = S::IL ? (int)threadIdx.x % S::CB : (int)threadIdx.x / T;
     const int t = S::IL ? (int)threadIdx.x / S::CB : (int)threadIdx.x % T;
-    const int i = xcd_remap(blockIdx.x, gridDim.x) * S::CB + c;
-    const bool live = i < a.nh;
+    // as k_csh_yfwd: tiles with a nonlinear term first, a limited state's only
+    const bool lim = bd.limited(blockIdx.y);
+    const int nfwd = (bd.hk + S::CB - 1) / S::CB;
+    if (lim && (int)blockIdx.x >= nfwd) return;
+    const int tile = csh_tile(blockIdx.x, nfwd, gridDim.x);
+    const int i = tile * S::CB + c;
+    const bool live = i < (lim ? bd.hk : a.nh);
     const size_t col = (size_t)(live ? i : 0) * NY;
     double2* xl = lds + c * S::LDSC;
     double2 v[E];
 #pragma unroll
-    for (int e = 0; e < E; ++e) v[e] = live ? a.h[blk8(i, rf_first_idx<NY, csh_yem(NY)>(t, e), a.nh)] : make_double2(0.0, 0.0);
-    rf_fft<NY, -1, csh_yem(NY)>(v, t, xl, tw);
+    for (int e = 0; e < E; ++e) v[e] = make_double2(0.0, 0.0);
+    if (tile < nfwd) {
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            if (i < bd.hk) v[e] = a.h[blk8(i, rf_first_idx<NY, csh_yem(NY)>(t, e), a.nh)];
+        rf_fft<NY, -1, csh_yem(NY)>(v, t, xl, tw);
+    }
     const double kxv = (double)i;
     bool finite = true;  // the new state's values (AB2, RK4 stage 4)
 #pragma unroll
     for (int e = 0; e < E; ++e) {
         const int j = rf_final_idx<NY, csh_yem(NY)>(t, e);
         const size_t q = col + j;
-        double2 nl = v[e];
-        if (!live || i >= a.imin[j]) nl = make_double2(0.0, 0.0);
+        const bool in = live && i < a.imin[j];
+        if (!in && (lim || !live)) {
+            v[e] = make_double2(0.0, 0.0);
+            continue;
+        }
+        const double2 nl = in ? v[e] : make_double2(0.0, 0.0);
         const double kyv = csh_ky<NY>(j);
         double2 wn, av;  // wn: the next stage's input
         csh_update<MODE>(a, q, false, nl, a.ws[q], kxv * kxv + kyv * kyv, &wn, &av);
-        if (live) finite = csh_store<MODE>(a, q, wn, av) && finite;
+        finite = csh_store<MODE>(a, q, wn, av) && finite;
         v[e] = wn;
     }
     if (!finite && a.bad) a.bad[blockIdx.y] = 1;
@@ -352,6 +398,23 @@ __global__ void k_ab2(const double2* w, double2* __restrict__ wn, const double2*
     }
 }
 
+// ------------------------------------------------------------ support of a state
+// band[r] = 1 unless run r's state has a mode outside the dealiasing circle.
+__global__ void k_csh_band_set(int* band, int run) { band[run] = 1; }
+
+__global__ __launch_bounds__(256) void k_csh_band(const double2* w, const int* imin, int nh, int ny, int* band, int run)
+{
+    const size_t n = (size_t)nh * ny;
+    bool any = false;
+    for (size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x; q < n; q += (size_t)gridDim.x * blockDim.x) {
+        const int i = (int)(q / ny), j = (int)(q % ny);
+        if (i < imin[j]) continue;
+        const double2 z = w[q];
+        any = any || !(z.x == 0.0 && z.y == 0.0);
+    }
+    if (any) band[run] = 0;
+}
+
 // ------------------------------------------------------------------ dispatch
 template <int NY, bool SCR, int GS>
 static int launch_yinv_t(const CshPlan& p, const double2* w, const CshPhys& ph, hipStream_t st)
@@ -359,7 +422,7 @@ static int launch_yinv_t(const CshPlan& p, const double2* w, const CshPhys& ph, 
     using S = YiShape<NY, SCR>;
     hipLaunchKernelGGL((k_csh_yinv<NY, SCR, GS>), dim3((p.nh + S::CB - 1) / S::CB, p.batch), dim3(S::NT), 0, st, w,
                        p.nh, p.g[0].as<double2>(), p.g[1].as<double2>(), p.g[2].as<double2>(), p.g[3].as<double2>(),
-                       p.tw_y, ph.lambda, p.gld, p.bstride);
+                       p.tw_y, ph.lambda, p.gld, p.bstride, csh_band(p));
     return TARA_OK;
 }
 
@@ -402,7 +465,7 @@ static int launch_x_shape(const CshPlan& p, hipStream_t st)
         TARA_CHECK(twn && twm, TARA_ERR_UNSUPPORTED, "x pass shape without its twiddle tables");
         hipLaunchKernelGGL((k_csh_x<NX, EM, RB, SPLIT>), dim3(p.ny / RB, p.batch), dim3(S::NT), 0, st,
                            p.g[0].as<double2>(), p.g[1].as<double2>(), p.g[2].as<double2>(), p.g[3].as<double2>(),
-                           scale, p.h.as<double2>(), twn, twm, p.rctw, p.bstride);
+                           scale, p.h.as<double2>(), twn, twm, p.rctw, p.bstride, csh_band(p));
         return TARA_OK;
     }
 }
@@ -449,12 +512,12 @@ static int launch_yfwd(const CshPlan& p, int mode, const YfwdArgs& a, hipStream_
     using S = YShape<NY>;
     dim3 g((p.nh + S::CB - 1) / S::CB, p.batch), b(S::NT);
     switch (mode) {
-        case CSH_RHS: hipLaunchKernelGGL((k_csh_yfwd<NY, CSH_RHS>), g, b, 0, st, a, p.tw_y); break;
-        case CSH_AB2: hipLaunchKernelGGL((k_csh_yfwd<NY, CSH_AB2>), g, b, 0, st, a, p.tw_y); break;
-        case CSH_RK4_1: hipLaunchKernelGGL((k_csh_yfwd<NY, CSH_RK4_1>), g, b, 0, st, a, p.tw_y); break;
-        case CSH_RK4_2: hipLaunchKernelGGL((k_csh_yfwd<NY, CSH_RK4_2>), g, b, 0, st, a, p.tw_y); break;
-        case CSH_RK4_3: hipLaunchKernelGGL((k_csh_yfwd<NY, CSH_RK4_3>), g, b, 0, st, a, p.tw_y); break;
-        case CSH_RK4_4: hipLaunchKernelGGL((k_csh_yfwd<NY, CSH_RK4_4>), g, b, 0, st, a, p.tw_y); break;
+        case CSH_RHS: hipLaunchKernelGGL((k_csh_yfwd<NY, CSH_RHS>), g, b, 0, st, a, csh_band(p), p.tw_y); break;
+        case CSH_AB2: hipLaunchKernelGGL((k_csh_yfwd<NY, CSH_AB2>), g, b, 0, st, a, csh_band(p), p.tw_y); break;
+        case CSH_RK4_1: hipLaunchKernelGGL((k_csh_yfwd<NY, CSH_RK4_1>), g, b, 0, st, a, csh_band(p), p.tw_y); break;
+        case CSH_RK4_2: hipLaunchKernelGGL((k_csh_yfwd<NY, CSH_RK4_2>), g, b, 0, st, a, csh_band(p), p.tw_y); break;
+        case CSH_RK4_3: hipLaunchKernelGGL((k_csh_yfwd<NY, CSH_RK4_3>), g, b, 0, st, a, csh_band(p), p.tw_y); break;
+        case CSH_RK4_4: hipLaunchKernelGGL((k_csh_yfwd<NY, CSH_RK4_4>), g, b, 0, st, a, csh_band(p), p.tw_y); break;
         default: set_error("bad mode %d", mode); return TARA_ERR_ARG;
     }
     return TARA_OK;
@@ -495,11 +558,11 @@ static int launch_yfwd_inv_g(const CshPlan& p, int mode, const YfwdArgs& a, hipS
     double2* const g2 = p.g[2].as<double2>();
     double2* const g3 = p.g[3].as<double2>();
     switch (mode) {
-        case CSH_AB2: hipLaunchKernelGGL((k_csh_yfwd_inv<NY, CSH_AB2, GS>), g, b, 0, st, a, p.tw_y, g0, g1, g2, g3, p.gld); break;
-        case CSH_RK4_1: hipLaunchKernelGGL((k_csh_yfwd_inv<NY, CSH_RK4_1, GS>), g, b, 0, st, a, p.tw_y, g0, g1, g2, g3, p.gld); break;
-        case CSH_RK4_2: hipLaunchKernelGGL((k_csh_yfwd_inv<NY, CSH_RK4_2, GS>), g, b, 0, st, a, p.tw_y, g0, g1, g2, g3, p.gld); break;
-        case CSH_RK4_3: hipLaunchKernelGGL((k_csh_yfwd_inv<NY, CSH_RK4_3, GS>), g, b, 0, st, a, p.tw_y, g0, g1, g2, g3, p.gld); break;
-        case CSH_RK4_4: hipLaunchKernelGGL((k_csh_yfwd_inv<NY, CSH_RK4_4, GS>), g, b, 0, st, a, p.tw_y, g0, g1, g2, g3, p.gld); break;
+        case CSH_AB2: hipLaunchKernelGGL((k_csh_yfwd_inv<NY, CSH_AB2, GS>), g, b, 0, st, a, csh_band(p), p.tw_y, g0, g1, g2, g3, p.gld); break;
+        case CSH_RK4_1: hipLaunchKernelGGL((k_csh_yfwd_inv<NY, CSH_RK4_1, GS>), g, b, 0, st, a, csh_band(p), p.tw_y, g0, g1, g2, g3, p.gld); break;
+        case CSH_RK4_2: hipLaunchKernelGGL((k_csh_yfwd_inv<NY, CSH_RK4_2, GS>), g, b, 0, st, a, csh_band(p), p.tw_y, g0, g1, g2, g3, p.gld); break;
+        case CSH_RK4_3: hipLaunchKernelGGL((k_csh_yfwd_inv<NY, CSH_RK4_3, GS>), g, b, 0, st, a, csh_band(p), p.tw_y, g0, g1, g2, g3, p.gld); break;
+        case CSH_RK4_4: hipLaunchKernelGGL((k_csh_yfwd_inv<NY, CSH_RK4_4, GS>), g, b, 0, st, a, csh_band(p), p.tw_y, g0, g1, g2, g3, p.gld); break;
         default: set_error("fused y pass: mode %d has no stage update", mode); return TARA_ERR_ARG;
     }
     return TARA_OK;
@@ -550,6 +613,25 @@ int csh_host_tables(int nx, int ny, std::vector<double>& kx, std::vector<double>
     return TARA_OK;
 }
 
+int csh_live_columns(int nx, int ny)
+{
+    const double cut = ((double)(nx + ny) / 2.0) / 3.0;
+    int i = 0;
+    while (i < nx / 2 + 1 && !((double)i >= cut)) ++i;  // imin at ky = 0, its largest
+    return i;
+}
+
+int csh_state_set(const CshPlan& p, const double2* w, int run, hipStream_t st)
+{
+    if (csh_small(p)) return TARA_OK;  // those passes take no account of it
+    const size_t n = (size_t)p.nh * p.ny, nb = (n + 255) / 256;
+    hipLaunchKernelGGL(k_csh_band_set, dim3(1), dim3(1), 0, st, p.band.as<int>(), run);
+    hipLaunchKernelGGL(k_csh_band, dim3((unsigned)(nb < 2048 ? nb : 2048)), dim3(256), 0, st, w, p.imin.as<int>(), p.nh,
+                       p.ny, p.band.as<int>(), run);
+    TARA_HIP(hipGetLastError());
+    return TARA_OK;
+}
+
 int csh_plan_init(CshPlan& p, int nx, int ny, int batch)
 {
     TARA_CHECK(batch >= 1 && batch <= 65535, TARA_ERR_ARG, "batch %d out of range", batch);
@@ -561,6 +643,7 @@ int csh_plan_init(CshPlan& p, int nx, int ny, int batch)
     p.nh = nx / 2 + 1;
     p.gld = csh_gld(p.nh);
     p.gsh = csh_gshift(p.nh);
+    p.hk = csh_live_columns(nx, ny);
     const size_t ns = (size_t)p.gld * ny;  // G0..G3 hold gld columns per row group
     p.batch = batch;
     p.bstride = ns;
@@ -570,7 +653,8 @@ int csh_plan_init(CshPlan& p, int nx, int ny, int batch)
         TARA_HIP(hipMemset(p.g[f].p, 0, batch * ns * sizeof(double2)));
     }
     if ((rc = p.h.alloc(batch * ns * sizeof(double2)))) return rc;
-    if ((rc = p.bad.alloc(batch * sizeof(int)))) return rc;
+    if ((rc = p.bad.alloc(batch * sizeof(int))) || (rc = p.band.alloc(batch * sizeof(int)))) return rc;
+    TARA_HIP(hipMemset(p.band.p, 0, batch * sizeof(int)));
     TARA_HIP(hipMemset(p.bad.p, 0, batch * sizeof(int)));
     std::vector<double> kx, ky;
     std::vector<int> imin;

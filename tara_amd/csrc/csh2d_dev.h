@@ -42,6 +42,33 @@ __device__ __forceinline__ size_t blkg(int i, int j, int ld, int gs)
     return ((size_t)(j >> gs) * ld + i) * (1 << gs) + (j & ((1 << gs) - 1));
 }
 
+// The state's support (CshPlan::band, hk): the dealiasing keeps the nonlinear
+// term to kx < hk, and inside the circle imin; where a state is zero outside the
+// circle (band flag of its run) it stays so, and the passes carry the circle only.
+struct CshBand {
+    static constexpr bool KNOWN = true;
+    const int* band;   // per run; null: unknown
+    const int* imin;
+    int hk, nh;
+    __device__ __forceinline__ bool limited(int run) const { return band && band[run] != 0; }
+};
+
+struct CshNoBand {
+    static constexpr bool KNOWN = false;
+};
+
+inline CshBand csh_band(const CshPlan& p)
+{
+    return CshBand{csh_small(p) ? nullptr : p.band.as<int>(), p.imin.as<int>(), p.hk, p.nh};
+}
+
+// Tile of workgroup w of ntiles: the first nfirst tiles (those with more to do, or
+// with anything to do) are spread over the XCDs first, the others after them.
+__device__ __forceinline__ int csh_tile(int w, int nfirst, int ntiles)
+{
+    return w < nfirst ? xcd_remap(w, nfirst) : nfirst + xcd_remap(w - nfirst, ntiles - nfirst);
+}
+
 // derive2csh's ky: j-1 for j <= Ny/2, j-1-Ny above (exact integers, checked on the host).
 template <int NY>
 __device__ __forceinline__ double csh_ky(int j)
@@ -53,10 +80,12 @@ __device__ __forceinline__ double csh_ky(int j)
 // spectra (kx = 0..M) of two real rows, Y[k] = X_a[k] + i X_b[k] over the full
 // length Nx (X[Nx-k] = conj X[k]) transforms to y = x_a + i x_b, so the product
 // x_a * x_b is Re(y) Im(y).  The imaginary parts of X[0] and X[M] are dropped,
-// as FFTW's c2r does.  Registers end with y at rf_final_idx<NX> positions.
-// WAVE: the row's threads sit in one wavefront.
-template <int NX, int EM, bool SPLIT, bool WAVE = false>
-__device__ __forceinline__ void x_c2r_pair(const double2* ga, const double2* gb, int j, int t,
+// as FFTW's c2r does; columns kx >= lim are zero and not read.  Registers end with
+// y at rf_final_idx<NX> positions.
+// WAVE: the row's threads sit in one wavefront.  BAND false: lim is nh, and the
+// loads go unguarded.
+template <int NX, int EM, bool SPLIT, bool WAVE = false, bool BAND = true>
+__device__ __forceinline__ void x_c2r_pair(const double2* ga, const double2* gb, int j, int lim, int t,
                                            double2* xl, const double2* tw, double2 (&v)[RF<NX, EM>::E])
 {
     constexpr int M = NX / 2;
@@ -65,7 +94,11 @@ __device__ __forceinline__ void x_c2r_pair(const double2* ga, const double2* gb,
     for (int e = 0; e < RF<NX, EM>::E; ++e) {
         const int k = rf_first_idx<NX, EM>(t, e);
         const int kk = k <= M ? k : NX - k;
-        double2 a = ga[blkg(kk, j, LD, GS)], b = gb[blkg(kk, j, LD, GS)];
+        double2 a = make_double2(0.0, 0.0), b = a;
+        if (!BAND || kk < lim) {
+            a = ga[blkg(kk, j, LD, GS)];
+            b = gb[blkg(kk, j, LD, GS)];
+        }
         if (kk == 0 || kk == M) {
             a.y = 0.0;
             b.y = 0.0;

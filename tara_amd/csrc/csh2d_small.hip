@@ -127,12 +127,14 @@ struct SXShape {
     static constexpr bool OK = NT <= 1024 && 2 * TM == T && 2 * RB * RF<NX>::LDS * 16 <= 160 * 1024;
 };
 
-template <int NX>
+template <int NX, typename Band>
 __global__ __launch_bounds__((SXShape<NX>::NT)) void k_csh_x_pairs(const double2* g0, const double2* g1,
                                                                    const double2* g2, const double2* g3, double scale,
                                                                    double2* __restrict__ h, const double2* tw_n,
-                                                                   const double2* tw_m, const double2* rctw, size_t bs)
+                                                                   const double2* tw_m, const double2* rctw, size_t bs,
+                                                                   Band bd)
 {
+    constexpr bool BAND = Band::KNOWN;
     using S = SXShape<NX>;
     static_assert(S::OK, "paired x pass does not fit");
     constexpr int E = RF<NX>::E, EH = RF<S::M>::E, T = S::T, M = S::M;
@@ -143,7 +145,10 @@ __global__ __launch_bounds__((SXShape<NX>::NT)) void k_csh_x_pairs(const double2
     double2* xl = lds + seq * RF<NX>::LDS;
     double2* x0 = lds + 2 * r * RF<NX>::LDS;  // the row's first buffer
     double2 v[E];
-    x_c2r_pair<NX, 8, false, S::WAVE>((p ? g2 : g0) + rb, (p ? g3 : g1) + rb, j, t, xl, tw_n, v);
+    int lim = M + 1;
+    if constexpr (BAND)
+        if (bd.limited(blockIdx.y)) lim = bd.hk;
+    x_c2r_pair<NX, 8, false, S::WAVE, BAND>((p ? g2 : g0) + rb, (p ? g3 : g1) + rb, j, lim, t, xl, tw_n, v);
 #pragma unroll
     for (int e = 0; e < E; ++e) xl[rf_pad(rf_final_idx<NX>(t, e))] = v[e];
     // the unpacking roots of this thread's kx, fetched before the stores
@@ -180,6 +185,8 @@ __global__ __launch_bounds__((SXShape<NX>::NT)) void k_csh_x_pairs(const double2
 #pragma unroll
     for (int u = 0; u < NK; ++u) {
         const int k = tt + u * 2 * T;
+        if constexpr (BAND)
+            if (k >= bd.hk) continue;  // dealiased away at every ky
         const double2 zk = x0[rf_pad(k)];
         const double2 zmk = x0[rf_pad(k == 0 ? 0 : M - k)];
         double2 xm;
@@ -281,15 +288,24 @@ int csh_small_yfwd(const CshPlan& p, int mode, const YfwdArgs& a, bool inv, hipS
     TARA_SMALL_Y_SWITCH(p.ny, launch_small_yfwd, p, mode, a, inv, st)
 }
 
-template <int NX>
-static int launch_x_pairs(const CshPlan& p, hipStream_t st)
+template <int NX, typename Band>
+static int launch_x_pairs_t(const CshPlan& p, Band bd, hipStream_t st)
 {
     using S = SXShape<NX>;
     const double scale = 1.0 / ((double)p.nx * (double)p.ny * (double)p.nx * (double)p.ny);
-    hipLaunchKernelGGL(k_csh_x_pairs<NX>, dim3(p.ny / S::RB, p.batch), dim3(S::NT), 0, st, p.g[0].as<double2>(),
-                       p.g[1].as<double2>(), p.g[2].as<double2>(), p.g[3].as<double2>(), scale, p.h.as<double2>(),
-                       p.tw_xn, p.tw_x, p.rctw, p.bstride);
+    hipLaunchKernelGGL((k_csh_x_pairs<NX, Band>), dim3(p.ny / S::RB, p.batch), dim3(S::NT), 0, st,
+                       p.g[0].as<double2>(), p.g[1].as<double2>(), p.g[2].as<double2>(), p.g[3].as<double2>(), scale,
+                       p.h.as<double2>(), p.tw_xn, p.tw_x, p.rctw, p.bstride, bd);
     return TARA_OK;
+}
+
+// The small grids' y passes write and read every column: guarding the loads and
+// stores by the support cost a 64^2 AB2 step 12 % there (and two more kernel
+// arguments alone 2.5 %).
+template <int NX>
+static int launch_x_pairs(const CshPlan& p, hipStream_t st)
+{
+    return csh_small(p) ? launch_x_pairs_t<NX>(p, CshNoBand{}, st) : launch_x_pairs_t<NX>(p, csh_band(p), st);
 }
 
 #define TARA_X_PAIRS_SWITCH(n, FN, ...)             \

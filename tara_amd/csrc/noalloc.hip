@@ -142,6 +142,7 @@ extern "C" int tara_derive2csh_noalloc(int nx, int ny, int nh, double nu, const 
     p.batch = 1;
     p.gld = csh_gld(nh);
     p.gsh = csh_gshift(nh);
+    p.hk = csh_live_columns(nx, ny);
     p.bstride = (size_t)p.gld * ny;
     const size_t fb = p.bstride * sizeof(double2);
     for (int k = 0; k < 4; ++k) p.g[k].view(base + L.g[k], fb);
