@@ -58,7 +58,7 @@ struct YiShape {
     static constexpr int CB = csh_yinv_cols(NY, SCR);
     static_assert(IL || CB == YShape<NY>::CB, "contiguous shape differs from the y passes'");
     static constexpr int NT = CB * T;
-    static constexpr int LDSC = RY<NY>::LDS + (IL ? 4 : 0);  // per-column exchange buffer
+    static constexpr int LDSC = IL ? NY : RY<NY>::LDS;  // per-column exchange buffer
     // Ny <= 512: at least 56 KB of LDS per workgroup, which holds the pass to
     // two 256-thread workgroups per CU.  Its registers would allow three, and
     // at three the ensemble step (128-512 grids) measured 6.67 against 6.42 ms.
@@ -69,9 +69,9 @@ struct YiShape {
 // positions): forms the four spectra of derive2csh.f95:29-71 (i kx omega,
 // i ky omega, i ky psi, -i kx psi; psi = omega/k^2, psi(0,0) = 0), or of
 // derive2css.f95:22-52 when SCR (screened), runs the backward y FFTs and writes
-// G0..G3 (row-group stride ld).  x is the column's LDS exchange buffer.
-template <int NY, bool SCR, int GS, bool OPQ>
-__device__ __forceinline__ void csh_yinv_column(double2 (&wv)[RY<NY>::E], int i, bool live, int t, double2* x,
+// G0..G3 (row-group stride ld).  sq: the column as the thread sees it.
+template <int NY, bool SCR, int GS, class SQ>
+__device__ __forceinline__ void csh_yinv_column(double2 (&wv)[RY<NY>::E], int i, bool live, const SQ& sq,
                                                 const double2* tw, double lam, int ld,
                                                 double2* __restrict__ g0, double2* __restrict__ g1,
                                                 double2* __restrict__ g2, double2* __restrict__ g3)
@@ -84,7 +84,7 @@ __device__ __forceinline__ void csh_yinv_column(double2 (&wv)[RY<NY>::E], int i,
     if constexpr (SCR) {
 #pragma unroll
         for (int e = 0; e < E; ++e) {
-            const int j = rf_first_idx<NY, csh_yem(NY)>(t, e);
+            const int j = rf_first_idx<NY, csh_yem(NY)>(sq.t, e);
             const double kyv = csh_ky<NY>(j);
             const double k2 = kxv * kxv + kyv * kyv;
             const double den = k2 + lam;
@@ -96,11 +96,9 @@ __device__ __forceinline__ void csh_yinv_column(double2 (&wv)[RY<NY>::E], int i,
 #pragma unroll 1
     for (int f = 0; f < 4; ++f) {
         double2 v[E];
-        // OPQ: the slot index is made opaque per transform so that the index
-        // arithmetic of the transform and the stores is recomputed here rather
-        // than hoisted out of the loop and held in registers (178 -> 117 VGPRs
-        // at Ny = 4096, which lets a 1024-thread workgroup run unspilled).
-        const int tt = OPQ ? rf_opaque(t) : t;
+        // the slot, opaque per transform: the index arithmetic of the stores is
+        // recomputed here rather than hoisted out of the loop and held in registers
+        const int tt = rf_opaque(sq.t);
         if (f == 2) {
 #pragma unroll
             for (int e = 0; e < E; ++e) {
@@ -121,13 +119,40 @@ __device__ __forceinline__ void csh_yinv_column(double2 (&wv)[RY<NY>::E], int i,
             v[e] = (f == 3) ? make_double2(kk * z.y, -(kk * z.x))     // -i kx psi
                             : make_double2(-(kk * z.y), kk * z.x);    // i k (omega | psi)
         }
-        rf_fft<NY, +1, csh_yem(NY)>(v, tt, x, tw);
+        sq.template fft<+1>(v, tw);
         // G0 = ux (f 2), G1 = uy (f 3), G2 = d omega/dx (f 0), G3 = d omega/dy (f 1)
         double2* o = f == 0 ? g2 : f == 1 ? g3 : f == 2 ? g0 : g1;
         if (live) {
 #pragma unroll
             for (int e = 0; e < E; ++e) o[blkg(i, rf_final_idx<NY, csh_yem(NY)>(tt, e), ld, GS)] = v[e];
         }
+    }
+}
+
+// The columns of a y pass's workgroup: CB side by side, of T threads each, or
+// (IL) interleaved over its lanes.  Columns of several wavefronts at radix cap 8
+// take rf_fft_w; columns of part of a wavefront exchange within it (171 runs of
+// 256^2: 1.18 against 1.20 ms a step with workgroup barriers).  A column that is
+// one whole wavefront (Ny = 512) keeps the barriers: its four columns write pieces
+// of the same 64-byte groups, and let apart they measured 4.55 against 4.36 ms
+// (171 runs of 512^2).
+template <int NY, int CB, bool IL>
+__device__ __forceinline__ auto csh_columns(double2* lds, int* c)
+{
+    constexpr int T = RY<NY>::T, EM = csh_yem(NY);
+    if constexpr (EM == 8 && T >= 128) {
+        if constexpr (IL) {
+            const RfWide<NY, CB> sq((int)threadIdx.x, lds);
+            *c = sq.c;
+            return sq;
+        } else {
+            *c = (int)threadIdx.x / T;
+            return RfWide<NY, 1>((int)threadIdx.x % T, lds + *c * RY<NY>::LDS);
+        }
+    } else {
+        static_assert(!IL, "interleaved columns are those of rf_fft_w");
+        *c = (int)threadIdx.x / T;
+        return RfSeq<NY, EM, (T < 64)>{(int)threadIdx.x % T, lds + *c * RY<NY>::LDS};
     }
 }
 
@@ -148,8 +173,9 @@ __global__ __launch_bounds__((YiShape<NY, SCR>::NT), (YiShape<NY, SCR>::IL ? 4 :
     using S = YiShape<NY, SCR>;
     constexpr int E = RY<NY>::E, T = S::T;
     __shared__ double2 lds[S::LDS_ELEMS];
-    const int c = S::IL ? (int)threadIdx.x % S::CB : (int)threadIdx.x / T;
-    const int t = S::IL ? (int)threadIdx.x / S::CB : (int)threadIdx.x % T;
+    int c;
+    const auto sq = csh_columns<NY, S::CB, S::IL>(lds, &c);
+    const int t = sq.t;
     // a limited state: the kx columns that hold something, and of them the modes
     const bool lim = bd.limited(blockIdx.y);
     const int ncol = lim ? bd.hk : nh, ntile = (ncol + S::CB - 1) / S::CB;
@@ -164,7 +190,7 @@ __global__ __launch_bounds__((YiShape<NY, SCR>::NT), (YiShape<NY, SCR>::IL ? 4 :
         wv[e] = make_double2(0.0, 0.0);
         if (live && (!lim || i < bd.imin[j])) wv[e] = w[col + j];
     }
-    csh_yinv_column<NY, SCR, GS, S::IL>(wv, i, live, t, lds + c * S::LDSC, tw, lam, ld, g0, g1, g2, g3);
+    csh_yinv_column<NY, SCR, GS>(wv, i, live, sq, tw, lam, ld, g0, g1, g2, g3);
 }
 
 // --------------------------------------------------------------------- pass 2
@@ -177,16 +203,19 @@ struct XShape {
     static constexpr int T = RF<NX, EM>::T;    // threads per row (backward transforms, length NX)
     static constexpr int TM = RF<M, EM>::T;    // of which active in the forward half-length transform
     static constexpr int NT = RB * T;
+    // rows of several wavefronts take rf_fft_w, their half-length transform too
+    static constexpr bool WIDE = EM == 8 && !SPLIT && T >= 128 && RB <= 8;
+    static constexpr bool WIDEM = WIDE && TM >= 128;
     // Per-row exchange buffer (complex elements).  Rows are interleaved across
     // lanes, so successive row buffers are offset by 4 elements (64 B) to land
     // on different LDS banks.
-    static constexpr int LDSR = (SPLIT ? RF<NX, EM>::LDS / 2 : RF<NX, EM>::LDS) + 4;
+    static constexpr int LDSR = WIDE && RB == 1 ? NX : (SPLIT ? RF<NX, EM>::LDS / 2 : RF<NX, EM>::LDS) + 4;
     // the forward half-length transform must use exactly half of the row's threads
     static constexpr bool OK = RB * LDSR * 16 <= 160 * 1024 && NT <= 1024 && NT >= 64 && 2 * TM == T;
 };
 
 template <int NX, int EM, int RB, bool SPLIT>
-__global__ __launch_bounds__((XShape<NX, EM, RB, SPLIT>::NT)) void k_csh_x(
+__global__ __launch_bounds__((XShape<NX, EM, RB, SPLIT>::NT), (XShape<NX, EM, RB, SPLIT>::WIDE ? 4 : 1)) void k_csh_x(
     const double2* g0, const double2* g1, const double2* g2, const double2* g3, double scale,
     double2* __restrict__ h, const double2* tw_n, const double2* tw_m, const double2* rctw, size_t bs, CshBand bd)
 {
@@ -201,15 +230,22 @@ __global__ __launch_bounds__((XShape<NX, EM, RB, SPLIT>::NT)) void k_csh_x(
     static_assert(S::OK, "x pass shape does not fit");
     constexpr int E = RF<NX, EM>::E, EH = RF<S::M, EM>::E, T = S::T, M = S::M;
     __shared__ double2 lds[RB * S::LDSR];
-    const int r = threadIdx.x % RB, t = threadIdx.x / RB;  // row fastest: RB-row chunks per kx
+    const int r = threadIdx.x % RB, tk = threadIdx.x / RB;  // row fastest: RB-row chunks per kx
     const int j = xcd_remap(blockIdx.x, gridDim.x) * RB + r;
     double2* xl = lds + r * S::LDSR;
+    const auto sq = [&] {
+        if constexpr (S::WIDE)
+            return RfWide<NX, RB>((int)threadIdx.x, lds);
+        else
+            return RfSeq<NX, EM, false, SPLIT>{tk, xl};
+    }();
+    const int t = sq.t;
     double nl[E];
     double2 v[E];
-    x_c2r_pair<NX, EM, SPLIT>(g0, g2, j, lim, t, xl, tw_n, v);   // ux + i d omega/dx
+    x_c2r_pair<NX, EM, true>(g0, g2, j, lim, sq, tw_n, v);   // ux + i d omega/dx
 #pragma unroll
     for (int e = 0; e < E; ++e) nl[e] = v[e].x * v[e].y;
-    x_c2r_pair<NX, EM, SPLIT>(g1, g3, j, lim, t, xl, tw_n, v);   // uy + i d omega/dy
+    x_c2r_pair<NX, EM, true>(g1, g3, j, lim, sq, tw_n, v);   // uy + i d omega/dy
 #pragma unroll
     for (int e = 0; e < E; ++e) nl[e] = (nl[e] + v[e].x * v[e].y) * scale;
     // forward x transform of the real product row: pack z[m] = nl[2m] + i nl[2m+1]
@@ -217,11 +253,14 @@ __global__ __launch_bounds__((XShape<NX, EM, RB, SPLIT>::NT)) void k_csh_x(
     // barriers where they fill whole waves, else run the same code on the
     // unused upper half of the row buffer so every barrier matches).
     double* xr = reinterpret_cast<double*>(xl);
+    if constexpr (S::WIDE) __syncthreads();
 #pragma unroll
     for (int e = 0; e < E; ++e) xr[rf_final_idx<NX, EM>(t, e)] = nl[e];
     __syncthreads();
     double2 z[EH];
-    const int tm = t % S::TM;
+    const bool half = tk < S::TM;  // threadIdx.x < TM RB
+    int tm = tk % S::TM;
+    if constexpr (S::WIDEM) tm = RfW<M, RB>((int)threadIdx.x % (S::TM * RB)).t;
 #pragma unroll
     for (int e = 0; e < EH; ++e) {
         const int m = rf_first_idx<M, EM>(tm, e);
@@ -234,28 +273,37 @@ __global__ __launch_bounds__((XShape<NX, EM, RB, SPLIT>::NT)) void k_csh_x(
     constexpr int NK = M / T;
     double2 wk[NK];
 #pragma unroll
-    for (int u = 0; u < NK; ++u) wk[u] = rctw[t + u * T];
+    for (int u = 0; u < NK; ++u) wk[u] = rctw[tk + u * T];
     __syncthreads();
-    if constexpr ((S::TM * RB) % 64 == 0) {
+    if constexpr (S::WIDEM) {
+        if (half) {
+            const RfWide<M, RB> sm((int)threadIdx.x, lds);
+            sm.template fft<-1>(z, tw_m);
+        } else {  // the barriers of rf_fft_w
+            __syncthreads();
+            __syncthreads();
+        }
+        __syncthreads();  // the waves' last exchanges
+    } else if constexpr ((S::TM * RB) % 64 == 0) {
         // the threads t >= TM (threadIdx.x >= TM RB) fill whole waves: they meet
         // the transform's barriers without running it
-        if (t < S::TM)
+        if (half)
             rf_fft<M, -1, EM, false, SPLIT>(z, tm, xl, tw_m);
         else
             rf_fft_barriers_only<M, EM, SPLIT>();
     } else {
         constexpr int HALF = SPLIT ? RF<M, EM>::LDS / 2 : RF<M, EM>::LDS;  // upper half, complex elements
-        double2* zl = xl + (t < S::TM ? 0 : HALF);
+        double2* zl = xl + (half ? 0 : HALF);
         rf_fft<M, -1, EM, false, SPLIT>(z, tm, zl, tw_m);
     }
-    if (t < S::TM) {
+    if (half) {
 #pragma unroll
         for (int e = 0; e < EH; ++e) xl[rf_pad(rf_final_idx<M, EM>(tm, e))] = z[e];
     }
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < NK; ++u) {  // consecutive t -> consecutive kx
-        const int k = t + u * T;
+        const int k = tk + u * T;
         if (k >= bd.hk) continue;  // dealiased away at every ky
         const double2 zk = xl[rf_pad(k)];
         const double2 zmk = xl[rf_pad(k == 0 ? 0 : M - k)];
@@ -279,7 +327,9 @@ __global__ __launch_bounds__(YShape<NY>::NT) void k_csh_yfwd(YfwdArgs a, CshBand
     using S = YShape<NY>;
     constexpr int E = RY<NY>::E, T = S::T;
     __shared__ double2 lds[S::CB * RY<NY>::LDS];
-    const int c = threadIdx.x / T, t = threadIdx.x % T;
+    int c;
+    const auto sq = csh_columns<NY, S::CB, false>(lds, &c);
+    const int t = sq.t;
     // tiles below hk have a nonlinear term; the others only the viscous one, and a
     // limited state nothing
     const bool lim = bd.limited(blockIdx.y);
@@ -294,7 +344,7 @@ __global__ __launch_bounds__(YShape<NY>::NT) void k_csh_yfwd(YfwdArgs a, CshBand
 #pragma unroll
         for (int e = 0; e < E; ++e)
             v[e] = i < bd.hk ? a.h[blk8(i, rf_first_idx<NY, csh_yem(NY)>(t, e), a.nh)] : make_double2(0.0, 0.0);
-        rf_fft<NY, -1, csh_yem(NY)>(v, t, lds + c * RY<NY>::LDS, tw);
+        sq.template fft<-1>(v, tw);
     }
     if (!live) return;
     const double kxv = (double)i;
@@ -345,8 +395,9 @@ __global__ __launch_bounds__((YiShape<NY, false>::NT), (YiShape<NY, false>::IL ?
     using S = YiShape<NY, false>;
     constexpr int E = RY<NY>::E, T = S::T;
     __shared__ double2 lds[S::LDS_ELEMS];
-    const int c = S::IL ? (int)threadIdx.x % S::CB : (int)threadIdx.x / T;
-    const int t = S::IL ? (int)threadIdx.x / S::CB : (int)threadIdx.x % T;
+    int c;
+    const auto sq = csh_columns<NY, S::CB, S::IL>(lds, &c);
+    const int t = sq.t;
     // as k_csh_yfwd: tiles with a nonlinear term first, a limited state's only
     const bool lim = bd.limited(blockIdx.y);
     const int nfwd = (bd.hk + S::CB - 1) / S::CB;
@@ -355,7 +406,6 @@ __global__ __launch_bounds__((YiShape<NY, false>::NT), (YiShape<NY, false>::IL ?
     const int i = tile * S::CB + c;
     const bool live = i < (lim ? bd.hk : a.nh);
     const size_t col = (size_t)(live ? i : 0) * NY;
-    double2* xl = lds + c * S::LDSC;
     double2 v[E];
 #pragma unroll
     for (int e = 0; e < E; ++e) v[e] = make_double2(0.0, 0.0);
@@ -363,7 +413,7 @@ __global__ __launch_bounds__((YiShape<NY, false>::NT), (YiShape<NY, false>::IL ?
 #pragma unroll
         for (int e = 0; e < E; ++e)
             if (i < bd.hk) v[e] = a.h[blk8(i, rf_first_idx<NY, csh_yem(NY)>(t, e), a.nh)];
-        rf_fft<NY, -1, csh_yem(NY)>(v, t, xl, tw);
+        sq.template fft<-1>(v, tw);
     }
     const double kxv = (double)i;
     bool finite = true;  // the new state's values (AB2, RK4 stage 4)
@@ -384,8 +434,8 @@ __global__ __launch_bounds__((YiShape<NY, false>::NT), (YiShape<NY, false>::IL ?
         v[e] = wn;
     }
     if (!finite && a.bad) a.bad[blockIdx.y] = 1;
-    rf_final_to_first<NY, csh_yem(NY)>(v, t, xl);
-    csh_yinv_column<NY, false, GS, S::IL>(v, i, live, t, xl, tw, 0.0, ld, g0, g1, g2, g3);
+    sq.final_to_first(v);
+    csh_yinv_column<NY, false, GS>(v, i, live, sq, tw, 0.0, ld, g0, g1, g2, g3);
 }
 
 // ------------------------------------------------------------ pointwise AB2
@@ -435,7 +485,11 @@ static int launch_yinv(const CshPlan& p, const double2* w, const CshPhys& ph, hi
 }
 
 // x-pass shapes the autotuner chooses among: {EM, RB, SPLIT}.  Shape 0 is
-// RB = min(8, 1024 / T) at EM = 8 without splitting (the largest workgroup);
+// RB = min(8, 512 / T) at EM = 8 without splitting: two workgroups a CU, one in
+// memory while the other transforms (RK4 step, one workgroup of twice the rows ->
+// two: 1024^2 0.172 -> 0.145 ms, 2048^2 0.303 -> 0.297, 2048 x 512 0.166 -> 0.151).
+// Nx = 4096 keeps two rows and one workgroup: of its 2-row groups a single row
+// reads half of every line (4096^2 1.51 ms, single rows 1.60).
 // shape kXPairs runs a row's two field pairs side by side (csh2d_small.hip).
 struct XCand {
     int em, rb, split;
@@ -447,7 +501,7 @@ constexpr int kNumXCands = sizeof(kXCands) / sizeof(kXCands[0]);
 template <int NX, int EM>
 constexpr int default_rb()
 {
-    return (1024 / RF<NX, EM>::T) < 1 ? 1 : (1024 / RF<NX, EM>::T) > 8 ? 8 : (1024 / RF<NX, EM>::T);
+    return NX == 4096 && EM == 8 ? 2 : (512 / RF<NX, EM>::T) < 1 ? 1 : (512 / RF<NX, EM>::T) > 8 ? 8 : (512 / RF<NX, EM>::T);
 }
 
 template <int NX, int EM, int RB, bool SPLIT>

@@ -82,17 +82,17 @@ __device__ __forceinline__ double csh_ky(int j)
 // x_a * x_b is Re(y) Im(y).  The imaginary parts of X[0] and X[M] are dropped,
 // as FFTW's c2r does; columns kx >= lim are zero and not read.  Registers end with
 // y at rf_final_idx<NX> positions.
-// WAVE: the row's threads sit in one wavefront.  BAND false: lim is nh, and the
-// loads go unguarded.
-template <int NX, int EM, bool SPLIT, bool WAVE = false, bool BAND = true>
-__device__ __forceinline__ void x_c2r_pair(const double2* ga, const double2* gb, int j, int lim, int t,
-                                           double2* xl, const double2* tw, double2 (&v)[RF<NX, EM>::E])
+// sq: the row as the thread sees it (RfSeq, RfWide).  BAND false: lim is nh, and
+// the loads go unguarded.
+template <int NX, int EM, bool BAND, class SQ>
+__device__ __forceinline__ void x_c2r_pair(const double2* ga, const double2* gb, int j, int lim, const SQ& sq,
+                                           const double2* tw, double2 (&v)[RF<NX, EM>::E])
 {
     constexpr int M = NX / 2;
     constexpr int LD = csh_gld(M + 1), GS = csh_gshift(M + 1);
 #pragma unroll
     for (int e = 0; e < RF<NX, EM>::E; ++e) {
-        const int k = rf_first_idx<NX, EM>(t, e);
+        const int k = rf_first_idx<NX, EM>(sq.t, e);
         const int kk = k <= M ? k : NX - k;
         double2 a = make_double2(0.0, 0.0), b = a;
         if (!BAND || kk < lim) {
@@ -109,7 +109,7 @@ __device__ __forceinline__ void x_c2r_pair(const double2* ga, const double2* gb,
         }
         v[e] = make_double2(a.x - b.y, a.y + b.x);
     }
-    rf_fft<NX, +1, EM, WAVE, SPLIT>(v, t, xl, tw);
+    sq.template fft<+1>(v, tw);
 }
 
 struct YfwdArgs {

@@ -148,7 +148,7 @@ __global__ __launch_bounds__((SXShape<NX>::NT)) void k_csh_x_pairs(const double2
     int lim = M + 1;
     if constexpr (BAND)
         if (bd.limited(blockIdx.y)) lim = bd.hk;
-    x_c2r_pair<NX, 8, false, S::WAVE, BAND>((p ? g2 : g0) + rb, (p ? g3 : g1) + rb, j, lim, t, xl, tw_n, v);
+    x_c2r_pair<NX, 8, BAND>((p ? g2 : g0) + rb, (p ? g3 : g1) + rb, j, lim, RfSeq<NX, 8, S::WAVE>{t, xl}, tw_n, v);
 #pragma unroll
     for (int e = 0; e < E; ++e) xl[rf_pad(rf_final_idx<NX>(t, e))] = v[e];
     // the unpacking roots of this thread's kx, fetched before the stores

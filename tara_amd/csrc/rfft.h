@@ -214,6 +214,89 @@ __device__ __forceinline__ void rf_fft(double2 (&v)[(RF<N, EM>::E)], int t, doub
     rf_rec<N, 1, DIR, EM, WAVE, SPLIT, TWPRE>(v, t, lds, tw, first);
 }
 
+// ------------------------------------------- sequences of several wavefronts
+// A transform of T = N/8 = 128, 256 or 512 threads with radix cap 8 (8 8 8 R,
+// R = N/512) that meets the workgroup's barriers once, not at every exchange.
+// Only 8 threads take part in an exchange of radix 8, those whose slots differ
+// in the digit that is exchanged.  The slots are dealt out so that for the first
+// and the last exchange these sit in one wavefront: slot t = (T/8) hi + m, where
+// a lane holds hi = lane/8 and of m the lowest bits (so that 8 / CI consecutive
+// slots, times the CI interleaved sequences, are 8 consecutive lanes: 128-byte
+// runs of global memory), the wave the others.  Those two exchanges then only
+// wait for the wave's own LDS operations, and the waves of a workgroup drift
+// apart, one in LDS while another computes.  Every exchange of a wave is laid out
+// in 512 elements of its own, [register][..][8 lanes], without padding: 8
+// consecutive lanes always meet 8 bank groups, in the second exchange, which
+// crosses the waves, by rotating the lanes' places by hi.
+// (2D incompressible RK4 step, six barriers a transform -> two: 4096^2 1.61 ->
+// 1.51 ms, 2048^2 0.415 -> 0.303, 1024^2 with the x pass's shape 0 0.195 -> 0.172.)
+//
+// lds: CI * N elements, shared by the interleaved sequences.  Between two
+// transforms through the same buffer no barrier is needed; before anything else
+// touches the buffer, a workgroup barrier is.
+template <int N, int CI>
+struct RfW {
+    static constexpr int T = N / 8, LO = 8 / CI, W = T * CI / 64;  // W waves
+    static constexpr bool OK = N >= 1024 && N <= 4096 && CI <= 8 && (8 % CI) == 0;
+    int t, hi, c, cl, base;  // slot, digit, sequence, lane % 8, the wave's elements
+    __device__ __forceinline__ explicit RfW(int tid)
+    {
+        const int lane = tid & 63, w = tid >> 6;
+        cl = lane & 7;
+        hi = lane >> 3;
+        c = cl % CI;
+        t = (T / 8) * hi + LO * w + cl / CI;
+        base = w * 512;
+    }
+    // place of lane low bits (lo, c) in a run of 8, for digit d
+    __device__ __forceinline__ static int turn(int lo, int c, int d) { return (lo ^ (d & (LO - 1))) * CI + c; }
+};
+
+template <int N, int DIR, int CI>
+__device__ __forceinline__ void rf_fft_w(double2 (&v)[8], const RfW<N, CI>& s, double2* lds, const double2* tw)
+{
+    using S = RfW<N, CI>;
+    static_assert(S::OK, "length or interleave out of range");
+    constexpr int T = S::T, R4 = N / 512;
+    double2* own = lds + s.base + s.cl;
+    const RfTw<N, 1, 8> w1{};
+    rf_compute<N, 1, DIR, 8>(v, w1);
+    RfTw<N, 8, 8> w2;
+    w2.load(s.hi, tw);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) own[(s.hi * 8 + q) * 8] = v[q];
+    rf_sync<true>();
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = own[(q * 8 + s.hi) * 8];
+    rf_sync<true>();
+    rf_compute<N, 8, DIR, 8>(v, w2);
+    RfTw<N, 64, 8> w3;
+    w3.load(s.t, tw);
+    {
+        double2* o = lds + s.base + s.hi * 8 + S::turn(s.cl / CI, s.c, s.hi);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) o[q * 64] = v[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const int m = s.t / 64 + (T / 64) * q;
+        v[q] = lds[(m / S::LO) * 512 + (s.t / 8 % 8) * 64 + (s.t % 8) * 8 + S::turn(m % S::LO, s.c, s.t % 8)];
+    }
+    __syncthreads();
+    rf_compute<N, 64, DIR, 8>(v, w3);
+    RfTw<N, 512, 8> w4;
+    w4.load(s.t, tw);
+    constexpr int HB = 8 / R4;  // hi = (t / 64) HB + (bits of t % 64)
+#pragma unroll
+    for (int q = 0; q < 8; ++q) own[(s.hi * 8 + q) * 8] = v[q];
+    rf_sync<true>();
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = own[((s.hi % HB + HB * (e % R4)) * 8 + s.hi / HB + (e / R4) * R4) * 8];
+    rf_sync<true>();
+    rf_compute<N, 512, DIR, 8>(v, w4);
+}
+
 // Number of LDS exchanges of a length-n transform with radix cap e: one
 // between consecutive passes of the schedule rf_rec walks (span L, radix
 // fft_radix(n / L, e), exchange while L * radix < n).
@@ -259,5 +342,47 @@ __device__ __forceinline__ void rf_final_to_first(double2 (&v)[(RF<N, EM>::E)], 
     for (int e = 0; e < E; ++e) v[e] = lds[rf_pad(rf_first_idx<N, EM>(t, e))];
     rf_sync<WAVE>();
 }
+
+// One sequence of a workgroup as a thread sees it: slot t, sequence c of CI
+// interleaved ones (c = 0 if contiguous), and the transform.  RfSeq: any length,
+// slot and sequence given; sequences of one wavefront exchange within it.
+// RfWide: several wavefronts, radix cap 8 (rf_fft_w), slot and sequence of the
+// workgroup's thread tid.
+template <int N, int EM, bool WAVE = false, bool SPLIT = false>
+struct RfSeq {
+    static constexpr int LEN = N;
+    int t;
+    double2* x;
+    template <int DIR>
+    __device__ __forceinline__ void fft(double2 (&v)[RF<N, EM>::E], const double2* tw) const
+    {
+        rf_fft<N, DIR, EM, WAVE, SPLIT>(v, t, x, tw);
+    }
+    __device__ __forceinline__ void final_to_first(double2 (&v)[RF<N, EM>::E]) const
+    {
+        rf_final_to_first<N, EM, WAVE>(v, t, x);
+    }
+};
+
+template <int N, int CI>
+struct RfWide {
+    static constexpr int LEN = N;
+    RfW<N, CI> s;
+    int t, c;
+    double2* x;
+    __device__ __forceinline__ RfWide(int tid, double2* lds) : s(tid), t(s.t), c(s.c), x(lds) {}
+    template <int DIR>
+    __device__ __forceinline__ void fft(double2 (&v)[8], const double2* tw) const
+    {
+        rf_fft_w<N, DIR, CI>(v, s, x, tw);
+    }
+    __device__ __forceinline__ void final_to_first(double2 (&v)[8]) const
+    {
+        if constexpr (rf_final_is_first<N, 8>()) return;
+        static_assert(rf_final_is_first<N, 8>() || CI == 1, "interleaved sequences share the buffer");
+        __syncthreads();
+        rf_final_to_first<N, 8>(v, t, x);
+    }
+};
 
 }  // namespace tara
