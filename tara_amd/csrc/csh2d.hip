@@ -14,10 +14,14 @@
 // (layout.hip).
 //
 //   pass 1  k_csh_yinv : per kx column read omega_hat, form the four spectra of
-//                        derive2csh.f95:29-71 (i kx omega, i ky omega, i ky psi,
-//                        -i kx psi; psi = omega/k^2, psi(0,0) = 0) and run the
-//                        backward y FFTs -> G0..G3.
-//   pass 2  k_csh_x    : per RB rows, four x c2r (half-length packing),
+//                        derive2csh.f95:29-71 (ux = i ky psi, uy = -i kx psi,
+//                        psi = omega/k^2, psi(0,0) = 0; i kx omega, i ky omega)
+//                        as the pairs ux +- i uy, dx omega +- i dy omega that the
+//                        x pass transforms, run the backward y FFTs -> G0..G3.
+//                        (4096^2 RK4 step 1.51 -> 1.44 ms, 512 runs of 128^2 ..
+//                        512^2 6.04 -> 5.84, against the four fields themselves,
+//                        each of which the x pass loaded twice.)
+//   pass 2  k_csh_x    : per RB rows, four x c2r (two pairs),
 //                        normalise by Nx*Ny and form ux*d_x omega + uy*d_y omega
 //                        (derive2csh.f95:89-98), one x r2c -> H.  (The reference
 //                        transforms the two products separately (:100-106); the
@@ -68,7 +72,7 @@ struct YiShape {
 // The inverse y pass of one kx column i given omega_hat (wv, at rf_first_idx
 // positions): forms the four spectra of derive2csh.f95:29-71 (i kx omega,
 // i ky omega, i ky psi, -i kx psi; psi = omega/k^2, psi(0,0) = 0), or of
-// derive2css.f95:22-52 when SCR (screened), runs the backward y FFTs and writes
+// derive2css.f95:22-52 when SCR (screened), pairwise (x_c2r_pair), runs the backward y FFTs and writes
 // G0..G3 (row-group stride ld).  sq: the column as the thread sees it.
 template <int NY, bool SCR, int GS, class SQ>
 __device__ __forceinline__ void csh_yinv_column(double2 (&wv)[RY<NY>::E], int i, bool live, const SQ& sq,
@@ -92,7 +96,8 @@ __device__ __forceinline__ void csh_yinv_column(double2 (&wv)[RY<NY>::E], int i,
             wv[e] = make_double2(k2 * ps[e].x, k2 * ps[e].y);
         }
     }
-    // i kx omega, i ky omega first; then omega -> psi in place; then +i ky psi, -i kx psi.
+    // i kx omega +- i (i ky omega) first; then omega -> psi in place; then
+    // i ky psi +- i (-i kx psi).
 #pragma unroll 1
     for (int f = 0; f < 4; ++f) {
         double2 v[E];
@@ -114,13 +119,12 @@ __device__ __forceinline__ void csh_yinv_column(double2 (&wv)[RY<NY>::E], int i,
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             const double kyv = csh_ky<NY>(rf_first_idx<NY, csh_yem(NY)>(tt, e));
-            const double kk = (f == 0 || f == 3) ? kxv : kyv;
+            const double cr = f == 0 ? -kyv : f == 1 ? kyv : f == 2 ? kxv : -kxv, ci = f < 2 ? kxv : kyv;
             const double2 z = wv[e];
-            v[e] = (f == 3) ? make_double2(kk * z.y, -(kk * z.x))     // -i kx psi
-                            : make_double2(-(kk * z.y), kk * z.x);    // i k (omega | psi)
+            v[e] = make_double2(cr * z.x - ci * z.y, cr * z.y + ci * z.x);
         }
         sq.template fft<+1>(v, tw);
-        // G0 = ux (f 2), G1 = uy (f 3), G2 = d omega/dx (f 0), G3 = d omega/dy (f 1)
+        // G0, G1 = ux +- i uy (f 2, 3), G2, G3 = d omega/dx +- i d omega/dy (f 0, 1)
         double2* o = f == 0 ? g2 : f == 1 ? g3 : f == 2 ? g0 : g1;
         if (live) {
 #pragma unroll
@@ -241,13 +245,11 @@ __global__ __launch_bounds__((XShape<NX, EM, RB, SPLIT>::NT), (XShape<NX, EM, RB
     }();
     const int t = sq.t;
     double nl[E];
-    double2 v[E];
-    x_c2r_pair<NX, EM, true>(g0, g2, j, lim, sq, tw_n, v);   // ux + i d omega/dx
+    double2 u[E], v[E];
+    x_c2r_pair<NX, EM, true>(g0, g1, j, lim, sq, tw_n, u);   // ux + i uy
+    x_c2r_pair<NX, EM, true>(g2, g3, j, lim, sq, tw_n, v);   // d omega/dx + i d omega/dy
 #pragma unroll
-    for (int e = 0; e < E; ++e) nl[e] = v[e].x * v[e].y;
-    x_c2r_pair<NX, EM, true>(g1, g3, j, lim, sq, tw_n, v);   // uy + i d omega/dy
-#pragma unroll
-    for (int e = 0; e < E; ++e) nl[e] = (nl[e] + v[e].x * v[e].y) * scale;
+    for (int e = 0; e < E; ++e) nl[e] = (u[e].x * v[e].x + u[e].y * v[e].y) * scale;
     // forward x transform of the real product row: pack z[m] = nl[2m] + i nl[2m+1]
     // for the half-length FFT (threads t < TM carry it; the others only meet its
     // barriers where they fill whole waves, else run the same code on the

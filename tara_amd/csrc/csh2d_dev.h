@@ -78,36 +78,38 @@ __device__ __forceinline__ double csh_ky(int j)
 
 // Two real c2r transforms in one complex FFT: with X_a, X_b the Hermitian half
 // spectra (kx = 0..M) of two real rows, Y[k] = X_a[k] + i X_b[k] over the full
-// length Nx (X[Nx-k] = conj X[k]) transforms to y = x_a + i x_b, so the product
-// x_a * x_b is Re(y) Im(y).  The imaginary parts of X[0] and X[M] are dropped,
-// as FFTW's c2r does; columns kx >= lim are zero and not read.  Registers end with
-// y at rf_final_idx<NX> positions.
+// length Nx (X[Nx-k] = conj X[k]) transforms to y = x_a + i x_b.  The y passes
+// store P = X_a + i X_b and Q = X_a - i X_b, so that Y[k] = P[k] up to M and
+// conj Q[Nx-k] above: one load an element, where X_a and X_b themselves were each
+// loaded at k and again at Nx-k.  At kx = 0 and M the imaginary parts of X_a and
+// X_b are dropped, as FFTW's c2r does: Y = (P + conj Q)/2.  Columns kx >= lim are
+// zero and not read.  Registers end with y at rf_final_idx<NX> positions.
+// A pair shares its rounding error, so fields of like size are paired.
 // sq: the row as the thread sees it (RfSeq, RfWide).  BAND false: lim is nh, and
 // the loads go unguarded.
 template <int NX, int EM, bool BAND, class SQ>
-__device__ __forceinline__ void x_c2r_pair(const double2* ga, const double2* gb, int j, int lim, const SQ& sq,
+__device__ __forceinline__ void x_c2r_pair(const double2* gp, const double2* gq, int j, int lim, const SQ& sq,
                                            const double2* tw, double2 (&v)[RF<NX, EM>::E])
 {
-    constexpr int M = NX / 2;
+    constexpr int M = NX / 2, E = RF<NX, EM>::E;
     constexpr int LD = csh_gld(M + 1), GS = csh_gshift(M + 1);
+    static_assert(rf_in_idx<NX, 1, EM>(1, E / 2) == 1 + M, "first pass of full radix");
+    double2 q0 = make_double2(0.0, 0.0), pm = q0;
+    if (sq.t == 0) {
+        q0 = gq[blkg(0, j, LD, GS)];
+        if (!BAND || M < lim) pm = gp[blkg(M, j, LD, GS)];
+    }
 #pragma unroll
-    for (int e = 0; e < RF<NX, EM>::E; ++e) {
+    for (int e = 0; e < E; ++e) {
         const int k = rf_first_idx<NX, EM>(sq.t, e);
-        const int kk = k <= M ? k : NX - k;
-        double2 a = make_double2(0.0, 0.0), b = a;
-        if (!BAND || kk < lim) {
-            a = ga[blkg(kk, j, LD, GS)];
-            b = gb[blkg(kk, j, LD, GS)];
-        }
-        if (kk == 0 || kk == M) {
-            a.y = 0.0;
-            b.y = 0.0;
-        }
-        if (k > M) {
-            a.y = -a.y;
-            b.y = -b.y;
-        }
-        v[e] = make_double2(a.x - b.y, a.y + b.x);
+        const int kk = e < E / 2 ? k : NX - k;
+        v[e] = make_double2(0.0, 0.0);
+        if (!BAND || kk < lim) v[e] = (e < E / 2 ? gp : gq)[blkg(kk, j, LD, GS)];
+        if (e >= E / 2) v[e].y = -v[e].y;
+    }
+    if (sq.t == 0) {
+        v[0] = make_double2(0.5 * (v[0].x + q0.x), 0.5 * (v[0].y - q0.y));
+        v[E / 2] = make_double2(0.5 * (v[E / 2].x + pm.x), 0.5 * (v[E / 2].y + pm.y));
     }
     sq.template fft<+1>(v, tw);
 }

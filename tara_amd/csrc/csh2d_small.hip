@@ -17,7 +17,7 @@ namespace tara {
 
 // --------------------------------------------------------------------- y pass
 // One kx column per 4 T threads: group g transforms field g of the inverse pass
-// (G0 = ux, G1 = uy, G2 = d omega/dx, G3 = d omega/dy).  The forward transform
+// (G0, G1 = ux +- i uy, G2, G3 = d omega/dx +- i d omega/dy).  The forward transform
 // and the update before it (FWD) are done by every group, so that each holds
 // the next stage's input in registers; group 0 stores it.
 template <int NY, int NG>
@@ -85,8 +85,9 @@ __global__ __launch_bounds__((SYShape<NY, INV ? 4 : 1>::NT)) void k_csh_small_y(
         for (int e = 0; e < E; ++e) v[e] = a.ws[(size_t)ic * a.si + (size_t)rf_first_idx<NY, EM>(t, e) * a.sj];
     }
     if constexpr (INV) {
-        // derive2csh.f95:29-71: groups 0, 1 i ky psi, -i kx psi with psi =
-        // omega/k^2, psi(0,0) = 0; groups 2, 3 i kx omega, i ky omega.  Screened
+        // derive2csh.f95:29-71: ux, uy = i ky psi, -i kx psi with psi = omega/k^2,
+        // psi(0,0) = 0; groups 0, 1 ux +- i uy, 2, 3 i kx omega +- i (i ky omega)
+        // (x_c2r_pair).  Screened
         // (derive2css.f95:22-52): psi = omega/(k^2 + lambda), omega_d = k^2 psi.
 #pragma unroll
         for (int e = 0; e < E; ++e) {
@@ -98,8 +99,8 @@ __global__ __launch_bounds__((SYShape<NY, INV ? 4 : 1>::NT)) void k_csh_small_y(
             double2 z = v[e];
             if (g < 2 || a.screened) z = zero ? make_double2(0.0, 0.0) : make_double2(z.x / den, z.y / den);
             if (g >= 2 && a.screened) z = make_double2(k2 * z.x, k2 * z.y);
-            const double kk = (g == 0 || g == 3) ? kyv : g == 1 ? -kxv : kxv;
-            v[e] = make_double2(-(kk * z.y), kk * z.x);
+            const double cr = g == 0 ? kxv : g == 1 ? -kxv : g == 2 ? -kyv : kyv, ci = g < 2 ? kyv : kxv;
+            v[e] = make_double2(cr * z.x - ci * z.y, cr * z.y + ci * z.x);
         }
         rf_fft<NY, +1, EM, S::WAVE>(v, t, xl, tw);
         double2* out = (g == 0 ? o.g0 : g == 1 ? o.g1 : g == 2 ? o.g2 : o.g3) + rb;
@@ -203,11 +204,11 @@ __global__ __launch_bounds__((SXShape<NX>::NT)) void k_csh_x_pairs(const double2
 // shorter chain gives: 512 x 1024 (4112) 139 / 112, 1024^2 (8208) 203 / 147; 64
 // runs of 128^2 (4160) 154 / 157 per ensemble step, 32 of 256^2 (8256) 242 / 242.
 //
-// The paired x pass is the default up to 2^20 points and Ny = 2048, against
-// shape 0 there: RK4 step 512^2 72.5 / 93.5 us, 1024 x 256 78.5 / 145, 1024^2
-// 153 / 192, 64^2 40 / 43; 256 x 4096 245 / 233, 2048 x 1024 276 / 260, 4096^2 2512 /
-// 2301.  (The autotuner times it among the other shapes.)
-constexpr size_t kSmallWaves = 2112, kSmallX = 1 << 20;
+// The paired x pass is the default up to 2^19 points and Ny = 2048, against
+// shape 0 there: RK4 step 512^2 70.1 / 92.6 us, 1024 x 512 118 / 123, 512 x 1024
+// 118 / 134, 2048 x 256 114.5 / 116, 64^2 40 / 44; beyond, 1024^2 145 / 142, 2048 x
+// 512 153 / 148, 2048^2 315 / 292.  (The autotuner times it among the other shapes.)
+constexpr size_t kSmallWaves = 2112, kSmallX = 1 << 19;
 
 bool csh_small(const CshPlan& p)
 {

@@ -66,7 +66,7 @@ __host__ __device__ constexpr int rf_last_span(int n, int rmax = 8)
 
 // Global index of register e's element before the pass of span L.
 template <int N, int L, int EM = 8>
-__device__ __forceinline__ int rf_in_idx(int t, int e)
+__host__ __device__ __forceinline__ constexpr int rf_in_idx(int t, int e)
 {
     constexpr int R = fft_radix(N / L, RF<N, EM>::E);
     const int b = t + (e / R) * RF<N, EM>::T;
