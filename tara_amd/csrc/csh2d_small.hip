@@ -16,10 +16,10 @@
 namespace tara {
 
 // --------------------------------------------------------------------- y pass
-// One kx column per 4 T threads: group g transforms field g of the inverse pass
-// (G0, G1 = ux +- i uy, G2, G3 = d omega/dx +- i d omega/dy).  The forward transform
-// and the update before it (FWD) are done by every group, so that each holds
-// the next stage's input in registers; group 0 stores it.
+// One kx column per NG T threads, NG = 4 or 2: group g transforms fields g, g + NG
+// of the inverse pass (G0, G1 = ux +- i uy, G2, G3 = d omega/dx +- i d omega/dy).
+// The forward transform and the update before it (FWD) are done by every group, so
+// that each holds the next stage's input in registers; group 0 stores it.
 template <int NY, int NG>
 struct SYShape {
     static constexpr int T = RY<NY>::T;                      // threads per sequence
@@ -34,10 +34,10 @@ struct SYInv {
     int ld;
 };
 
-template <int NY, int MODE, int GS, bool FWD, bool INV>
-__global__ __launch_bounds__((SYShape<NY, INV ? 4 : 1>::NT)) void k_csh_small_y(YfwdArgs a, SYInv o, const double2* tw)
+template <int NY, int MODE, int GS, bool FWD, int NG>
+__global__ __launch_bounds__((SYShape<NY, NG>::NT)) void k_csh_small_y(YfwdArgs a, SYInv o, const double2* tw)
 {
-    constexpr int NG = INV ? 4 : 1;
+    constexpr bool INV = NG > 1;
     using S = SYShape<NY, NG>;
     constexpr int E = RY<NY>::E, T = S::T, EM = csh_yem(NY);
     __shared__ double2 lds[S::CB * NG * RY<NY>::LDS];
@@ -86,27 +86,34 @@ __global__ __launch_bounds__((SYShape<NY, INV ? 4 : 1>::NT)) void k_csh_small_y(
     }
     if constexpr (INV) {
         // derive2csh.f95:29-71: ux, uy = i ky psi, -i kx psi with psi = omega/k^2,
-        // psi(0,0) = 0; groups 0, 1 ux +- i uy, 2, 3 i kx omega +- i (i ky omega)
-        // (x_c2r_pair).  Screened
-        // (derive2css.f95:22-52): psi = omega/(k^2 + lambda), omega_d = k^2 psi.
+        // psi(0,0) = 0; fields 0, 1 ux +- i uy, 2, 3 i kx omega +- i (i ky omega)
+        // (x_c2r_pair).  Screened (derive2css.f95:22-52): psi = omega/(k^2 +
+        // lambda), omega_d = k^2 psi.
+        double2 w[E];
 #pragma unroll
-        for (int e = 0; e < E; ++e) {
-            const int j = rf_first_idx<NY, EM>(t, e);
-            const double kyv = csh_ky<NY>(j);
-            const double k2 = kxv * kxv + kyv * kyv;
-            const double den = a.screened ? k2 + a.lam : k2;
-            const bool zero = a.screened ? ic == 0 && j == 0 : k2 == 0.0;
-            double2 z = v[e];
-            if (g < 2 || a.screened) z = zero ? make_double2(0.0, 0.0) : make_double2(z.x / den, z.y / den);
-            if (g >= 2 && a.screened) z = make_double2(k2 * z.x, k2 * z.y);
-            const double cr = g == 0 ? kxv : g == 1 ? -kxv : g == 2 ? -kyv : kyv, ci = g < 2 ? kyv : kxv;
-            v[e] = make_double2(cr * z.x - ci * z.y, cr * z.y + ci * z.x);
-        }
-        rf_fft<NY, +1, EM, S::WAVE>(v, t, xl, tw);
-        double2* out = (g == 0 ? o.g0 : g == 1 ? o.g1 : g == 2 ? o.g2 : o.g3) + rb;
-        if (live) {
+        for (int e = 0; e < E; ++e) w[e] = v[e];
+#pragma unroll 1
+        for (int f = g; f < 4; f += NG) {
 #pragma unroll
-            for (int e = 0; e < E; ++e) out[blkg(i, rf_final_idx<NY, EM>(t, e), o.ld, GS)] = v[e];
+            for (int e = 0; e < E; ++e) {
+                const int j = rf_first_idx<NY, EM>(t, e);
+                const double kyv = csh_ky<NY>(j);
+                const double k2 = kxv * kxv + kyv * kyv;
+                const double den = a.screened ? k2 + a.lam : k2;
+                const bool zero = a.screened ? ic == 0 && j == 0 : k2 == 0.0;
+                double2 z = w[e];
+                if (f < 2 || a.screened) z = zero ? make_double2(0.0, 0.0) : make_double2(z.x / den, z.y / den);
+                if (f >= 2 && a.screened) z = make_double2(k2 * z.x, k2 * z.y);
+                const double cr = f == 0 ? kxv : f == 1 ? -kxv : f == 2 ? -kyv : kyv, ci = f < 2 ? kyv : kxv;
+                v[e] = make_double2(cr * z.x - ci * z.y, cr * z.y + ci * z.x);
+            }
+            rf_fft<NY, +1, EM, S::WAVE>(v, t, xl, tw);
+            double2* out = (f == 0 ? o.g0 : f == 1 ? o.g1 : f == 2 ? o.g2 : o.g3) + rb;
+            if (live) {
+#pragma unroll
+                for (int e = 0; e < E; ++e) out[blkg(i, rf_final_idx<NY, EM>(t, e), o.ld, GS)] = v[e];
+            }
+            if (NG == 4) break;
         }
     }
 }
@@ -197,31 +204,42 @@ __global__ __launch_bounds__((SXShape<NX>::NT)) void k_csh_x_pairs(const double2
 }
 
 // ------------------------------------------------------------------- dispatch
-// The y passes run here while their threads come to at most 2112 wavefronts,
-// two per SIMD and the odd column of Nh.  RK4 step (tuned x shape) here against
-// the larger grids' passes: 1024 x 512 (2052 wavefronts) 117 / 146 us, 256 x 1024
-// (2064) 91.7 / 93.9; beyond, the repeated forward transform costs more than the
-// shorter chain gives: 512 x 1024 (4112) 139 / 112, 1024^2 (8208) 203 / 147; 64
-// runs of 128^2 (4160) 154 / 157 per ensemble step, 32 of 256^2 (8256) 242 / 242.
+// The y passes run here with four groups a column while their threads come to at
+// most 2112 wavefronts, two per SIMD and the odd column of Nh.  RK4 step (tuned x
+// shape) here against the larger grids' passes: 1024 x 512 (2052 wavefronts) 117 /
+// 146 us, 256 x 1024 (2064) 91.7 / 93.9; beyond, the repeated forward transform
+// costs more than the shorter chain gives: 512 x 1024 (4112) 139 / 112, 1024^2
+// (8208) 203 / 147.
+// Up to Ny = 512 and 6000 wavefronts two groups, two fields each, repeat it once
+// only.  A step here against the larger grids' passes: 64 runs of 128^2 (2080) 144
+// / 164 us, 200 of 64^2 (1650) 110 / 146, 512 of 64^2 (4224) 210 / 250, 32 of 256^2
+// (4128) 219 / 238, 8 of 512^2 (4112) 234 / 256, 2048 x 512 (4100) 150 / 159;
+// beyond, 64 of 256^2 (8256) 454 / 428, 16 of 512^2 (8224) 435 / 423.  Not at Nx =
+// 4096, whose 2-row groups one column a workgroup writes in pieces: 4096 x 512 234
+// / 190, 4096 x 256 165 / 161; and not at Ny = 1024: 512 x 1024 132 / 127.
 //
 // The paired x pass is the default up to 2^19 points and Ny = 2048, against
 // shape 0 there: RK4 step 512^2 70.1 / 92.6 us, 1024 x 512 118 / 123, 512 x 1024
 // 118 / 134, 2048 x 256 114.5 / 116, 64^2 40 / 44; beyond, 1024^2 145 / 142, 2048 x
 // 512 153 / 148, 2048^2 315 / 292.  (The autotuner times it among the other shapes.)
-constexpr size_t kSmallWaves = 2112, kSmallX = 1 << 19;
+constexpr size_t kSmallWaves = 2112, kPairWaves = 6000, kSmallX = 1 << 19;
 
-bool csh_small(const CshPlan& p)
+// Thread groups a column, 0 for the larger grids' passes.
+static int small_groups(const CshPlan& p)
 {
-    const size_t threads = (size_t)p.nh * 4 * (p.ny / csh_yem(p.ny)) * p.batch;
-    return p.ny <= 1024 && threads <= 64 * kSmallWaves;
+    const size_t threads = (size_t)p.nh * (p.ny / csh_yem(p.ny)) * p.batch;
+    if (p.ny <= 1024 && 4 * threads <= 64 * kSmallWaves) return 4;
+    return p.nx <= 2048 && p.ny <= 512 && 2 * threads <= 64 * kPairWaves ? 2 : 0;
 }
+
+bool csh_small(const CshPlan& p) { return small_groups(p) > 0; }
 
 bool csh_small_xrows(const CshPlan& p) { return p.ny <= 2048 && (size_t)p.nx * p.ny * p.batch <= kSmallX; }
 
-template <int NY, int MODE, bool FWD, bool INV>
+template <int NY, int MODE, bool FWD, int NG>
 static int launch_small_y(const CshPlan& p, const YfwdArgs& a, hipStream_t st)
 {
-    using S = SYShape<NY, INV ? 4 : 1>;
+    using S = SYShape<NY, NG>;
     if constexpr (!S::OK) {
         set_error("small y pass at Ny=%d", NY);
         return TARA_ERR_UNSUPPORTED;
@@ -229,26 +247,35 @@ static int launch_small_y(const CshPlan& p, const YfwdArgs& a, hipStream_t st)
         const SYInv o{p.g[0].as<double2>(), p.g[1].as<double2>(), p.g[2].as<double2>(), p.g[3].as<double2>(), p.gld};
         const dim3 grid((p.nh + S::CB - 1) / S::CB, p.batch), b(S::NT);
         if (p.gsh == 1)
-            hipLaunchKernelGGL((k_csh_small_y<NY, MODE, 1, FWD, INV>), grid, b, 0, st, a, o, p.tw_y);
+            hipLaunchKernelGGL((k_csh_small_y<NY, MODE, 1, FWD, NG>), grid, b, 0, st, a, o, p.tw_y);
         else
-            hipLaunchKernelGGL((k_csh_small_y<NY, MODE, 2, FWD, INV>), grid, b, 0, st, a, o, p.tw_y);
+            hipLaunchKernelGGL((k_csh_small_y<NY, MODE, 2, FWD, NG>), grid, b, 0, st, a, o, p.tw_y);
         return TARA_OK;
     }
+}
+
+// Two groups exist up to Ny = 512 (small_groups).
+template <int NY, int MODE, bool FWD>
+static int launch_small_inv(const CshPlan& p, const YfwdArgs& a, hipStream_t st)
+{
+    if constexpr (NY <= 512)
+        if (small_groups(p) == 2) return launch_small_y<NY, MODE, FWD, 2>(p, a, st);
+    return launch_small_y<NY, MODE, FWD, 4>(p, a, st);
 }
 
 template <int NY>
 static int launch_small_yinv(const CshPlan& p, const YfwdArgs& a, hipStream_t st)
 {
-    return launch_small_y<NY, CSH_RHS, false, true>(p, a, st);
+    return launch_small_inv<NY, CSH_RHS, false>(p, a, st);
 }
 
 template <int NY>
 static int launch_small_yfwd(const CshPlan& p, int mode, const YfwdArgs& a, bool inv, hipStream_t st)
 {
 #define TARA_SMALL_MODE(M) \
-    case M: return inv ? launch_small_y<NY, M, true, true>(p, a, st) : launch_small_y<NY, M, true, false>(p, a, st);
+    case M: return inv ? launch_small_inv<NY, M, true>(p, a, st) : launch_small_y<NY, M, true, 1>(p, a, st);
     switch (mode) {
-        case CSH_RHS: return launch_small_y<NY, CSH_RHS, true, false>(p, a, st);
+        case CSH_RHS: return launch_small_y<NY, CSH_RHS, true, 1>(p, a, st);
         TARA_SMALL_MODE(CSH_AB2)
         TARA_SMALL_MODE(CSH_RK4_1)
         TARA_SMALL_MODE(CSH_RK4_2)
