@@ -9,7 +9,7 @@
 //   m = L / r, p < m, q < s0, u < r,
 // and the output of the last pass is in natural order.  One thread computes
 // one output (O(r) work), so large prime factors still spread over the
-// device.  Roots come from one table of e^{-2 pi i k/n} (long double, rounded
+// device (in LDS radices 2 to 5 take a butterfly a thread).  Roots come from one table of e^{-2 pi i k/n} (long double, rounded
 // once).  Radices: 4 while possible, then 2, 3, 5, 7, then the remaining
 // primes.
 //
@@ -20,9 +20,10 @@
 //
 // Up to kAnyLds elements a workgroup runs whole sequences through all passes in
 // LDS, from and to the caller's arrays (k_any_lds): one launch per transform, no
-// work space, no synchronisation.  Longer sequences take one launch per pass over
-// two global buffers, allocated per call, and the stream is synchronised before
-// the call returns.
+// work space, no synchronisation.  Longer sequences, and few sequences of a large
+// prime (any_lds), take one launch per pass over two global buffers, allocated per
+// call, and the stream is synchronised before the call returns.
+#include <algorithm>
 #include <vector>
 
 #include "common.h"
@@ -227,7 +228,7 @@ __device__ __forceinline__ void any_butterfly(const double2* x, double2* y, int 
 // synchronisation around them, 1.5 ms for the six transforms of a derive2csh
 // call at 96 x 80 against 0.02 ms here (four launches of 6 us).
 template <AnyKind KIND>
-__global__ __launch_bounds__(256) void k_any_lds(AnyArgs a, const double2* __restrict__ tw)
+__global__ __launch_bounds__(1024) void k_any_lds(AnyArgs a, const double2* __restrict__ tw)
 {
     extern __shared__ double2 lds[];
     const unsigned n = a.n, S = a.seqs, tid = threadIdx.x, nt = blockDim.x;
@@ -273,13 +274,15 @@ __global__ __launch_bounds__(256) void k_any_lds(AnyArgs a, const double2* __res
                 }
             }
         } else {
-            // one output per thread: a large prime still spreads over the workgroup
+            // one output per thread: a large prime spreads over the workgroup, which
+            // has a thread for every one (launch_any_lds); four terms' loads in flight
             for (unsigned b = tid; b < S * n; b += nt) {
                 const unsigned c = b / n, e = b - c * n;
                 const unsigned rest = e / (unsigned)s0, q = e - rest * s0, p = rest / (unsigned)r, u = rest - p * r;
                 const double2* xs = x + c * n + q + s0 * p;
                 double2 acc = make_double2(0.0, 0.0);
                 unsigned k = 0;  // j u mod r
+#pragma unroll 4
                 for (int j = 0; j < r; ++j) {
                     const double2 v = xs[j * nr], w = root(tw, (long)k * nr, a.dir);
                     acc.x += v.x * w.x - v.y * w.y;
@@ -318,14 +321,21 @@ __global__ __launch_bounds__(256) void k_any_lds(AnyArgs a, const double2* __res
 
 // Whether length n runs in LDS; if so, the pass schedule and how many sequences
 // share a workgroup: up to 8 (columns: a 128-byte line) that fit 64 KB and still
-// leave 256 workgroups.
+// leave 256 workgroups.  A prime factor above 1000 sums n r terms a sequence, each
+// with a gathered root, which its one CU bounds: such sequences run here only if
+// there are enough of them, r / 12, to fill the chip.  Host r2c of n x rows here
+// against the passes over the whole chip: 2039 x 1 1178 / 545 us, x 128 1375 / 1202, x
+// 256 1628 / 2282; 1499 x 64 709 / 506, x 128 804 / 788; 1021 x 64 352 / 325, x 128 401
+// / 424; 1994 (2 x 997) x 1 327 / 310, x 64 418 / 436; 761 x 1 182 / 221.
 bool any_lds(int n, long ntrans, AnyArgs& a)
 {
     if (n > kAnyLds) return false;
+    const std::vector<int> rs = radices(n);  // ascending past the fours
+    if (!rs.empty() && rs.back() > 1000 && ntrans * 12 < rs.back()) return false;
     a = AnyArgs{};
     a.n = n;
     a.ntrans = ntrans;
-    for (int r : radices(n)) a.radix[a.npass++] = r;
+    for (int r : rs) a.radix[a.npass++] = r;
     a.seqs = 8;
     while (a.seqs > 1 && (2L * a.seqs * n * 16 > 65536 || ntrans / a.seqs < 256)) a.seqs /= 2;
     return true;
@@ -337,7 +347,11 @@ int launch_any_lds(const AnyArgs& a, hipStream_t st)
     const double2* tw = unit_roots(a.n);
     TARA_CHECK(tw, TARA_ERR_ALLOC, "root table allocation failed (n = %d)", a.n);
     const int work = a.seqs * a.n / 4;  // butterflies of a pass
-    const int nt = work >= 192 ? 256 : work >= 96 ? 128 : 64;
+    int nt = work >= 192 ? 256 : work >= 96 ? 128 : 64;
+    // a large prime: a thread per output, whose sum is a chain of r gathers (64 to
+    // 256 threads, one term after another / as here: 251 x 1 140 / 55 us, 509 x 1 243 /
+    // 98, 2036 x 1 572 / 167, 1021 x 512 1250 / 988)
+    if (a.npass && a.radix[a.npass - 1] > 64) nt = std::min(1024, (a.seqs * a.n + 63) / 64 * 64);
     const long blocks = (a.ntrans + a.seqs - 1) / a.seqs;
     TARA_CHECK(blocks <= 0x7fffffffL, TARA_ERR_UNSUPPORTED, "transform batch too large");
     hipLaunchKernelGGL(k_any_lds<KIND>, dim3((unsigned)blocks), dim3(nt), 2 * (size_t)a.seqs * a.n * sizeof(double2), st,
