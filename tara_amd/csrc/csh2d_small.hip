@@ -44,9 +44,11 @@ __global__ __launch_bounds__((SYShape<NY, NG>::NT)) void k_csh_small_y(YfwdArgs 
     const size_t rb = blockIdx.y * a.bs;  // batched runs
     a.ws += rb;
     const int t = threadIdx.x % T, seq = threadIdx.x / T, g = seq % NG;
-    const int i = xcd_remap(blockIdx.x, gridDim.x) * S::CB + seq / NG;
+    const int i0 = xcd_remap(blockIdx.x, gridDim.x) * S::CB, i = i0 + seq / NG;
     const bool live = i < a.nh;
-    const int ic = live ? i : 0;  // dead columns recompute column 0 and store nothing
+    // dead columns recompute the workgroup's first column and store nothing: one that
+    // no other workgroup writes
+    const int ic = live ? i : i0;
     double2* xl = lds + seq * RY<NY>::LDS;
     const double kxv = (double)ic;
     double2 v[E];
@@ -68,8 +70,8 @@ __global__ __launch_bounds__((SYShape<NY, NG>::NT)) void k_csh_small_y(YfwdArgs 
             const double kyv = csh_ky<NY>(j);
             csh_update<MODE>(a, q, ic == 0 && j == 0, nl, a.ws[q], kxv * kxv + kyv * kyv, &v[e], &av[e]);
         }
-        // every group has read the column before group 0 writes it
-        if constexpr (NG > 1) __syncthreads();
+        // every group and dead column has read the column before its group 0 writes it
+        if constexpr (NG > 1 || S::CB > 1) __syncthreads();
         if (live && g == 0) {
             bool finite = true;
 #pragma unroll
