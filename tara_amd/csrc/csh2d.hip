@@ -732,10 +732,16 @@ int csh_plan_init(CshPlan& p, int nx, int ny, int batch)
     TARA_CHECK(p.tw_y && p.tw_x && p.tw_xn && p.tw_x16 && p.tw_xn16 && p.tw_x4 && p.tw_xn4 && p.rctw, TARA_ERR_ALLOC,
                "twiddle table allocation failed");
     p.xcfg = csh_default_xshape(p);
+    TARA_CHECK(csh_xshape_ok(p, p.xcfg), TARA_ERR_UNSUPPORTED, "derive2csh: no x pass for %dx%d", nx, ny);
     return TARA_OK;
 }
 
-int csh_default_xshape(const CshPlan& p) { return csh_small_xrows(p) && shape_ok(p, kXPairs) == 1 ? kXPairs : 0; }
+// Nx = 32 has the paired pass only: eight rows of the others are half a wavefront.
+int csh_default_xshape(const CshPlan& p)
+{
+    const bool pairs = shape_ok(p, kXPairs) == 1;
+    return pairs && (csh_small_xrows(p) || shape_ok(p, 0) != 1) ? kXPairs : 0;
+}
 
 int csh_num_xshapes() { return kNumXCands; }
 

@@ -340,6 +340,7 @@ static int launch_x_pairs(const CshPlan& p, hipStream_t st)
 
 #define TARA_X_PAIRS_SWITCH(n, FN, ...)             \
     switch (n) {                                    \
+        case 32: return FN<32>(__VA_ARGS__);        \
         case 64: return FN<64>(__VA_ARGS__);        \
         case 128: return FN<128>(__VA_ARGS__);      \
         case 256: return FN<256>(__VA_ARGS__);      \
