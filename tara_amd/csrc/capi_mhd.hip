@@ -25,15 +25,39 @@ int check_dims(int nx, int ny, int nz, int nh)
     return TARA_OK;
 }
 
+// b[r*ld + i] = 0 for the padding columns nh <= i < ld of every row.
+__global__ void k_zero_padding(double2* b, int nh, int ld, size_t rows)
+{
+    const int w = ld - nh;
+    for (size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x; q < rows * w; q += (size_t)gridDim.x * blockDim.x)
+        b[q / w * ld + nh + q % w] = make_double2(0.0, 0.0);
+}
+
+// Zeroes the flux scratch's padding after rows were packed in it.  A step's x pass
+// writes columns below Nh only; where no live tile reaches past Nh (a 2 pi box of like
+// sides) no pass reads the padding, else what is left there would be transformed in
+// place at every step, growing without bound.
+int clear_padding(const MhdPlan& p, hipStream_t s)
+{
+    if (8 * p.ktiles <= p.nh) return TARA_OK;
+    const size_t rows = (size_t)12 * p.ny * p.nz, n = rows * (p.ld - p.nh);
+    hipLaunchKernelGGL(k_zero_padding, dim3((unsigned)std::min<size_t>((n + 255) / 256, 16384)), dim3(256), 0, s,
+                       p.b.as<double2>(), p.nh, p.ld, rows);
+    TARA_HIP(hipGetLastError());
+    return TARA_OK;
+}
+
 // nf fields, host (nh, ny, nz) contiguous <-> device (ld, ny, nz), through the
 // plan's flux scratch (12 fields, idle between steps of the same stream).
 int h2d(const MhdPlan& p, double2* const d[], const double* const h[], int nf, hipStream_t s)
 {
-    return rows_from_host(d, h, nf, p.nh, p.ld, (size_t)p.ny * p.nz, p.b, s);
+    int rc = rows_from_host(d, h, nf, p.nh, p.ld, (size_t)p.ny * p.nz, p.b, s);
+    return rc ? rc : clear_padding(p, s);
 }
 int d2h(const MhdPlan& p, double* const h[], const double2* const d[], int nf, hipStream_t s)
 {
-    return rows_to_host(h, d, nf, p.nh, p.ld, (size_t)p.ny * p.nz, p.b, s);
+    int rc = rows_to_host(h, d, nf, p.nh, p.ld, (size_t)p.ny * p.nz, p.b, s);
+    return rc ? rc : clear_padding(p, s);
 }
 
 struct DropIn {

@@ -11,7 +11,8 @@ enum MhdMode { MHD_RHS = 0, MHD_AB2 = 1 };
 
 // Plan + scratch of one (nx, ny, nz) grid.  Device spectra use the reference's
 // kx-fastest layout with the row length padded to ld = Nh rounded up to 8,
-// element (i, j, k) at (k*Ny + j)*ld + i; padding columns are kept at zero.
+// element (i, j, k) at (k*Ny + j)*ld + i; padding columns are kept at zero (those of
+// b, in which host copies pack their rows, where a live tile reaches past Nh).
 struct MhdPlan {
     int nx = 0, ny = 0, nz = 0, nh = 0, ld = 0;
     double lx = 0, ly = 0, lz = 0, mu = 0, eta = 0, cs = 0;
