@@ -15,8 +15,10 @@
 // transposes through LDS; the products take a tenth.
 //
 // The products are the GEMMs of gemm.hip in the same order of summation (32x32x16
-// MFMA, k ascending), so activations and spectra keep their bits; only the
-// projection's final sum over hidden channels is ordered differently (FP32).
+// MFMA, k ascending), and training evaluates the same GELU, so what it keeps has the
+// bits of the separate products.  Inference evaluates gelu_fast (within 4e-8 of Phi,
+// like erff), so its activations differ from training's where that moves a rounding
+// to bfloat16, and orders the projection's final sum over hidden channels differently.
 //
 // A workgroup of four wavefronts holds the row's c x n activations: Vt[x][i]
 // (k = channel contiguous, the mixing's operand), O[o][x] (k = x contiguous, the
