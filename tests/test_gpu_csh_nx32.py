@@ -12,6 +12,7 @@ from conftest import rel_l2
 from test_gpu_csh_small import _noise, _rhs, _steps
 
 pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")  # before the library opens the device
 
 NX = 32
 
@@ -37,7 +38,6 @@ def test_rhs_and_steps_vs_oracle(ny, screened):
 
 @pytest.mark.parametrize("ny", [16, 32, 512])
 def test_device_arrays(ny):
-    torch = pytest.importorskip("torch")
     print(f"device arrays {NX}x{ny}", flush=True)
     w = _noise(NX, ny, 3 * ny)
     d = torch.from_numpy(np.ascontiguousarray(w.T)).cuda()
