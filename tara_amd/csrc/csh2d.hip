@@ -492,7 +492,7 @@ static int launch_yinv(const CshPlan& p, const double2* w, const CshPhys& ph, hi
 // two: 1024^2 0.172 -> 0.145 ms, 2048^2 0.303 -> 0.297, 2048 x 512 0.166 -> 0.151).
 // Nx = 4096 keeps two rows and one workgroup: of its 2-row groups a single row
 // reads half of every line (4096^2 1.51 ms, single rows 1.60).
-// shape kXPairs runs a row's two field pairs side by side (csh2d_small.hip).
+// shape kXPairs runs a row's two field pairs side by side (csh2d_pairs.hip).
 struct XCand {
     int em, rb, split;
 };
