@@ -705,22 +705,18 @@ int refresh_weights(tara_fno* f)
                        f->wb.as<uint16_t>(), f->nparam);
     const int c = f->c, c2 = 2 * c;
     const size_t M = f->modes;
-    for (int l = 0; l < f->layers; ++l)
-        hipLaunchKernelGGL(k_build_rs, dim3(fno_grid(M * c2 * c2)), dim3(256), 0, f->st,
-                           f->par.as<float>() + f->o_r + (size_t)l * f->r_sz, P<float>(f->rs, l * M * c2 * c2),
-                           P<uint16_t>(f->rsb, l * M * c2 * c2), (int)M, c);
+    const size_t LM = (size_t)f->layers * M;  // the layers' blocks follow each other on both sides
+    hipLaunchKernelGGL(k_build_rs, dim3(fno_grid(LM * c2 * c2)), dim3(256), 0, f->st, f->par.as<float>() + f->o_r,
+                       P<float>(f->rs), P<uint16_t>(f->rsb), (int)LM, c);
     TARA_HIP(hipGetLastError());
     if (f->fused) {
-        const int CP = fno_pad(c);
-        int rc;
-        for (int l = 0; l < f->layers; ++l)
-            if ((rc = fno_pad_weights(f->par.as<float>() + f->o_w + (size_t)l * c * c, c, c,
-                                      P<uint16_t>(f->wp, (size_t)l * CP * CP), CP, CP, f->st)))
-                return rc;
-        if ((rc = fno_pad_weights(f->par.as<float>() + f->o_w1, 2 * c, c, P<uint16_t>(f->w1p), 2 * CP, CP, f->st)) ||
-            (rc = fno_pad_vector(f->par.as<float>() + f->o_b1, 2 * c, P<float>(f->b1p), 2 * CP, f->st)) ||
-            (rc = fno_pad_vector(f->par.as<float>() + f->o_w2, 2 * c, P<float>(f->w2p), 2 * CP, f->st)))
-            return rc;
+        const float* par = f->par.as<float>();
+        FnoPadArgs a{};
+        a.c = c, a.cp = fno_pad(c), a.layers = f->layers;
+        a.w = par + f->o_w, a.w1 = par + f->o_w1, a.b1 = par + f->o_b1, a.w2 = par + f->o_w2;
+        a.wp = P<uint16_t>(f->wp), a.w1p = P<uint16_t>(f->w1p), a.b1p = P<float>(f->b1p), a.w2p = P<float>(f->w2p);
+        int rc = fno_pad_weights(a, f->st);
+        if (rc) return rc;
     }
     return TARA_OK;
 }

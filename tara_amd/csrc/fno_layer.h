@@ -41,8 +41,13 @@ int fno_lift_x(const FnoLayerArgs& a, hipStream_t st);
 // One layer after its inverse y transform (z): v <- act(inverse x of z + W v + b),
 // then what the next step of the network reads: T1, or the projected output.
 int fno_layer(const FnoLayerArgs& a, hipStream_t st);
-// Padded bfloat16 copy of rows x cols FP32 weights into prow x pcol.
-int fno_pad_weights(const float* w, int rows, int cols, uint16_t* o, int prow, int pcol, hipStream_t st);
-int fno_pad_vector(const float* w, int n, float* o, int pn, hipStream_t st);
+// Padded copies of the weights (bfloat16 matrices, FP32 vectors), cp = fno_pad(c).
+struct FnoPadArgs {
+    int c, cp, layers;
+    const float *w, *w1, *b1, *w2;  // [layers][c][c], [2 c][c], [2 c], [2 c]
+    uint16_t *wp, *w1p;             // [layers][cp][cp], [2 cp][cp]
+    float *b1p, *w2p;               // [2 cp]
+};
+int fno_pad_weights(const FnoPadArgs& a, hipStream_t st);
 
 }  // namespace tara
