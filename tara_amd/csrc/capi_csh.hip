@@ -275,12 +275,12 @@ int csh_ctx_state(tara_csh* c, double2** w, const CshPlan** p, hipStream_t* st)
     return TARA_OK;
 }
 
-int csh_ctx_zero_history(tara_csh* c)
+int csh_ctx_zero_history(tara_csh* c, bool flags)
 {
     TARA_CHECK(c, TARA_ERR_ARG, "null context");
-    TARA_HIP(hipMemsetAsync(c->aux.p, 0, c->aux.bytes, c->st));
-    int rc = csh_clear_nonfinite(c->plan, -1, c->st);  // a new state: the guard starts over
-    if (rc || (rc = csh_state_set(c->plan, c->w.as<double2>(), 0, c->st))) return rc;
+    int rc = csh_state_set(c->plan, c->w.as<double2>(), c->aux.as<double2>(), c->aux.bytes / sizeof(double2), 0, flags,
+                           c->st);
+    if (rc) return rc;
     TARA_HIP(hipStreamSynchronize(c->st));
     return TARA_OK;
 }
@@ -291,9 +291,10 @@ extern "C" int tara_csh_upload(tara_csh* c, const double* omegak)
     TARA_CHECK(c && omegak, TARA_ERR_ARG, "null argument");
     const CshPlan& p = c->plan;
     TARA_HIP(hipMemcpyAsync(c->stage.p, omegak, c->stage.bytes, hipMemcpyHostToDevice, c->st));
-    int rc = to_kymajor(c->stage.as<double2>(), c->w.as<double2>(), p.nh, p.ny, 1, c->st);
+    int rc = to_kymajor(c->stage.as<double2>(), c->w.as<double2>(), p.nh, p.ny, 1, c->st, p.bad.as<int>(),
+                        p.band.as<int>());
     if (rc) return rc;
-    return csh_ctx_zero_history(c);
+    return csh_ctx_zero_history(c, false);
 }
 
 namespace {

@@ -115,6 +115,13 @@ int run_slot(tara_ens* e, int run, Bucket** b, int* slot)
     return TARA_OK;
 }
 
+// The run in this slot has a new state (flags: csh_state_set).
+int state_set(Bucket& b, int slot, bool flags, hipStream_t st)
+{
+    const size_t o = slot * b.plan.bstride;
+    return csh_state_set(b.plan, b.w.as<double2>() + o, b.aux.as<double2>() + o, b.plan.bstride, slot, flags, st);
+}
+
 // w[i*ny + j] = s[j*ld + i]: padded kx-fastest spectrum -> ky-major state
 __global__ void k_spec_to_state(const double2* s, int ld, int nh, int ny, double2* w)
 {
@@ -135,8 +142,13 @@ __global__ void k_state_to_spec(const double2* w, int nh, int ny, int ld, double
     }
 }
 
-__global__ void k_f32_to_f64(const float* a, double* b, size_t n)
+// b = a; *zero = 0, *one = 1 (the flags of the run whose state follows)
+__global__ void k_f32_to_f64(const float* a, double* b, size_t n, int* zero, int* one)
 {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *zero = 0;
+        *one = 1;
+    }
     for (size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x; q < n; q += (size_t)gridDim.x * blockDim.x)
         b[q] = (double)a[q];
 }
@@ -223,12 +235,10 @@ extern "C" int tara_ens_upload(tara_ens* e, int run, const double* omegak)
     const CshPlan& p = b->plan;
     TARA_HIP(hipStreamSynchronize(e->st));
     TARA_HIP(hipMemcpy(b->stage.p, omegak, b->stage.bytes, hipMemcpyHostToDevice));
-    if ((rc = to_kymajor(b->stage.as<double2>(), b->w.as<double2>() + slot * p.bstride, p.nh, p.ny, 1, nullptr)))
+    if ((rc = to_kymajor(b->stage.as<double2>(), b->w.as<double2>() + slot * p.bstride, p.nh, p.ny, 1, nullptr,
+                         p.bad.as<int>() + slot, p.band.as<int>() + slot)))
         return rc;
-    TARA_HIP(hipMemset(b->aux.as<double2>() + slot * p.bstride, 0, p.bstride * sizeof(double2)));
-    if ((rc = csh_clear_nonfinite(p, slot, nullptr)) ||
-        (rc = csh_state_set(p, b->w.as<double2>() + slot * p.bstride, slot, nullptr)))
-        return rc;
+    if ((rc = state_set(*b, slot, false, nullptr))) return rc;
     TARA_HIP(hipDeviceSynchronize());
     return TARA_OK;
 }
@@ -255,10 +265,7 @@ extern "C" int tara_ens_ic_random(tara_ens* e, int run, unsigned seed, double k0
     const CshPlan& p = b->plan;
     if ((rc = csh_random_phase(b->w.as<double2>() + slot * p.bstride, b->n, b->n, seed, k0, energy, e->st)))
         return rc;
-    TARA_HIP(hipMemsetAsync(b->aux.as<double2>() + slot * p.bstride, 0, p.bstride * sizeof(double2), e->st));
-    if ((rc = csh_clear_nonfinite(p, slot, e->st)) ||
-        (rc = csh_state_set(p, b->w.as<double2>() + slot * p.bstride, slot, e->st)))
-        return rc;
+    if ((rc = state_set(*b, slot, true, e->st))) return rc;
     TARA_HIP(hipStreamSynchronize(e->st));
     return TARA_OK;
 }
@@ -272,15 +279,14 @@ extern "C" int tara_ens_set_omega(tara_ens* e, int run, const float* omega)
     const CshPlan& p = b->plan;
     const int n = b->n, ld = spec_ld(n);
     const size_t np = (size_t)n * n;
-    hipLaunchKernelGGL(k_f32_to_f64, dim3(ens_grid(np)), dim3(256), 0, e->st, omega, b->real.as<double>(), np);
+    hipLaunchKernelGGL(k_f32_to_f64, dim3(ens_grid(np)), dim3(256), 0, e->st, omega, b->real.as<double>(), np,
+                       p.bad.as<int>() + slot, p.band.as<int>() + slot);
     if ((rc = row_r2c(b->real.as<double>(), b->spec.as<double2>(), n, ld, n, e->st))) return rc;
     if ((rc = col_fft(b->spec.as<double2>(), n, ld, ld, (long)ld * n, 1, -1, e->st))) return rc;
     hipLaunchKernelGGL(k_spec_to_state, dim3(ens_grid((size_t)p.nh * n)), dim3(256), 0, e->st,
                        b->spec.as<double2>(), ld, p.nh, n, b->w.as<double2>() + slot * p.bstride);
     TARA_HIP(hipGetLastError());
-    TARA_HIP(hipMemsetAsync(b->aux.as<double2>() + slot * p.bstride, 0, p.bstride * sizeof(double2), e->st));
-    if ((rc = csh_clear_nonfinite(p, slot, e->st))) return rc;
-    return csh_state_set(p, b->w.as<double2>() + slot * p.bstride, slot, e->st);
+    return state_set(*b, slot, false, e->st);
 }
 
 extern "C" int tara_ens_get_omega(tara_ens* e, int run, float* omega)

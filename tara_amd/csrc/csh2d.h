@@ -84,11 +84,9 @@ struct CshPlan {
     // reads none of them, and the update touches the circle only.
     DevBuf band;
 };
-// The per-run non-finite flags of a plan: csh_nonfinite synchronises st and
-// returns the number of flagged runs (flags[r] = 0 / 1 when flags is not null);
-// csh_clear_nonfinite clears run r's flag (every run's for r < 0), ordered on st.
+// The per-run non-finite flags of a plan: synchronises st and returns the number of
+// flagged runs (flags[r] = 0 / 1 when flags is not null).
 int csh_nonfinite(const CshPlan& p, int* flags, hipStream_t st);
-int csh_clear_nonfinite(const CshPlan& p, int r, hipStream_t st);
 
 // Physics of one right-hand side.  screened = 0: derive2csh (psi = omega/k^2,
 // derivatives and viscous term on omega).  screened = 1: derive2css
@@ -105,8 +103,10 @@ struct CshPhys {
 // Columns kx below the dealiasing cut at ky = 0 (CshPlan::hk).
 int csh_live_columns(int nx, int ny);
 // To be called, ordered on st, whenever run `run`'s state w was set (not by the
-// steps themselves): finds its support for the passes.
-int csh_state_set(const CshPlan& p, const double2* w, int run, hipStream_t st);
+// steps themselves): zeroes its history aux (naux elements) and finds the state's
+// support for the passes.  Before it, run's ints in bad and band are to be set to 0 and
+// 1: by the kernel that set the state, or with flags here in a launch of its own.
+int csh_state_set(const CshPlan& p, const double2* w, double2* aux, size_t naux, int run, bool flags, hipStream_t st);
 // batch: number of independent runs of this grid the launches cover; every
 // per-run field (state, G0..G3, H) is packed run after run, bstride apart.
 int csh_plan_init(CshPlan& p, int nx, int ny, int batch = 1);
@@ -164,7 +164,7 @@ int csh_random_phase(double2* w, int nx, int ny, unsigned seed, double k0, doubl
 // Access to a tara_csh context's device state (capi_csh.hip): the ky-major
 // omega_hat, the plan and the stream; and zeroing of its AB2 history.
 int csh_ctx_state(tara_csh* c, double2** w, const CshPlan** p, hipStream_t* st);
-int csh_ctx_zero_history(tara_csh* c);
+int csh_ctx_zero_history(tara_csh* c, bool flags = true);  // flags as csh_state_set
 int launch_ab2(const double2* w, double2* wn, const double2* fo, const double2* fn, double dt, size_t n,
                hipStream_t st);
 

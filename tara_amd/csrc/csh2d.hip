@@ -43,6 +43,8 @@
 // Wavenumbers: derive2csh uses pi = 3.1428 (a default-real literal) and
 // Lx = Ly = 2 pi (:16-21), so kx = i-1 and ky = j-1 or j-1-Ny are exact integers;
 // the host builds the tables with that exact expression (csh_plan_init).
+#include <algorithm>
+
 #include "csh2d_dev.h"
 
 namespace tara {
@@ -450,21 +452,32 @@ __global__ void k_ab2(const double2* w, double2* __restrict__ wn, const double2*
     }
 }
 
-// ------------------------------------------------------------ support of a state
-// band[r] = 1 unless run r's state has a mode outside the dealiasing circle.
-__global__ void k_csh_band_set(int* band, int run) { band[run] = 1; }
-
-__global__ __launch_bounds__(256) void k_csh_band(const double2* w, const int* imin, int nh, int ny, int* band, int run)
+// ------------------------------------------------------------ a state set anew
+// Zeroes a run's history (naux elements) and, with band, clears *band if the state w
+// has a mode outside the dealiasing circle.  As launches of their own beside memsets of
+// history and flag, finding the support took 15 to 25 us more of a call of 50 us
+// (tara_ens_set_omega, batches on the large grids' passes); as one launch whose last
+// workgroup sets the flag, 45 more at 1024^2, for the counting and its fences.
+__global__ __launch_bounds__(256) void k_csh_state_set(const double2* w, const int* imin, int nh, int ny, double2* aux,
+                                                       size_t naux, int* band)
 {
-    const size_t n = (size_t)nh * ny;
+    const size_t first = blockIdx.x * (size_t)blockDim.x + threadIdx.x, step = (size_t)gridDim.x * blockDim.x;
+    for (size_t q = first; q < naux; q += step) aux[q] = make_double2(0.0, 0.0);
+    if (!band) return;
     bool any = false;
-    for (size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x; q < n; q += (size_t)gridDim.x * blockDim.x) {
+    for (size_t q = first; q < (size_t)nh * ny; q += step) {
         const int i = (int)(q / ny), j = (int)(q % ny);
         if (i < imin[j]) continue;
         const double2 z = w[q];
         any = any || !(z.x == 0.0 && z.y == 0.0);
     }
-    if (any) band[run] = 0;
+    if (any) *band = 0;
+}
+
+__global__ void k_csh_state_flags(int* bad, int* band)
+{
+    *bad = 0;
+    *band = 1;
 }
 
 // ------------------------------------------------------------------ dispatch
@@ -677,13 +690,13 @@ int csh_live_columns(int nx, int ny)
     return i;
 }
 
-int csh_state_set(const CshPlan& p, const double2* w, int run, hipStream_t st)
+int csh_state_set(const CshPlan& p, const double2* w, double2* aux, size_t naux, int run, bool flags, hipStream_t st)
 {
-    if (csh_small(p)) return TARA_OK;  // those passes take no account of it
-    const size_t n = (size_t)p.nh * p.ny, nb = (n + 255) / 256;
-    hipLaunchKernelGGL(k_csh_band_set, dim3(1), dim3(1), 0, st, p.band.as<int>(), run);
-    hipLaunchKernelGGL(k_csh_band, dim3((unsigned)(nb < 2048 ? nb : 2048)), dim3(256), 0, st, w, p.imin.as<int>(), p.nh,
-                       p.ny, p.band.as<int>(), run);
+    int* band = p.band.as<int>() + run;
+    const size_t n = std::max(naux, (size_t)p.nh * p.ny), nb = (n + 255) / 256;
+    if (flags) hipLaunchKernelGGL(k_csh_state_flags, dim3(1), dim3(1), 0, st, p.bad.as<int>() + run, band);
+    hipLaunchKernelGGL(k_csh_state_set, dim3((unsigned)(nb < 2048 ? nb : 2048)), dim3(256), 0, st, w, p.imin.as<int>(),
+                       p.nh, p.ny, aux, naux, csh_small(p) ? nullptr : band);
     TARA_HIP(hipGetLastError());
     return TARA_OK;
 }
@@ -760,17 +773,6 @@ int csh_nonfinite(const CshPlan& p, int* flags, hipStream_t st)
         if (flags) flags[r] = f[r] != 0;
     }
     return n;
-}
-
-int csh_clear_nonfinite(const CshPlan& p, int r, hipStream_t st)
-{
-    if (r < 0) {
-        TARA_HIP(hipMemsetAsync(p.bad.p, 0, p.batch * sizeof(int), st));
-    } else {
-        TARA_CHECK(r < p.batch, TARA_ERR_ARG, "run %d out of range", r);
-        TARA_HIP(hipMemsetAsync(p.bad.as<int>() + r, 0, sizeof(int), st));
-    }
-    return TARA_OK;
 }
 
 // The arguments of a forward y pass whose stage input, base, accumulator and

@@ -6,7 +6,9 @@
 namespace tara {
 
 // dst[i*ny + j] = src[j*nh + i] for each of nplanes planes of nh*ny elements.
-int to_kymajor(const double2* src, double2* dst, int nh, int ny, int nplanes, hipStream_t st);
+// zero, one: ints that the launch sets to 0 and 1 besides (null: none).
+int to_kymajor(const double2* src, double2* dst, int nh, int ny, int nplanes, hipStream_t st, int* zero = nullptr,
+               int* one = nullptr);
 // dst[j*nh + i] = src[i*ny + j], the inverse.
 int from_kymajor(const double2* src, double2* dst, int nh, int ny, int nplanes, hipStream_t st);
 

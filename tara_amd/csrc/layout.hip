@@ -7,8 +7,12 @@ namespace tara {
 
 // out[c*rows + r] = in[r*cols + c] within each plane (rows x cols, row-major in).
 __global__ __launch_bounds__(256) void k_transpose(const double2* __restrict__ in, double2* __restrict__ out,
-                                                   int rows, int cols)
+                                                   int rows, int cols, int* zero, int* one)
 {
+    if (threadIdx.x == 0 && blockIdx.x + blockIdx.y + blockIdx.z == 0) {
+        if (zero) *zero = 0;
+        if (one) *one = 1;
+    }
     __shared__ double2 tile[32][33];
     const size_t plane = (size_t)blockIdx.z * rows * cols;
     const int c0 = blockIdx.x * 32, r0 = blockIdx.y * 32;
@@ -24,17 +28,18 @@ __global__ __launch_bounds__(256) void k_transpose(const double2* __restrict__ i
     }
 }
 
-static int transpose(const double2* in, double2* out, int rows, int cols, int nplanes, hipStream_t st)
+static int transpose(const double2* in, double2* out, int rows, int cols, int nplanes, hipStream_t st,
+                     int* zero = nullptr, int* one = nullptr)
 {
     dim3 g((cols + 31) / 32, (rows + 31) / 32, nplanes);
-    hipLaunchKernelGGL(k_transpose, g, dim3(256), 0, st, in, out, rows, cols);
+    hipLaunchKernelGGL(k_transpose, g, dim3(256), 0, st, in, out, rows, cols, zero, one);
     TARA_HIP(hipGetLastError());
     return TARA_OK;
 }
 
-int to_kymajor(const double2* src, double2* dst, int nh, int ny, int nplanes, hipStream_t st)
+int to_kymajor(const double2* src, double2* dst, int nh, int ny, int nplanes, hipStream_t st, int* zero, int* one)
 {
-    return transpose(src, dst, ny, nh, nplanes, st);
+    return transpose(src, dst, ny, nh, nplanes, st, zero, one);
 }
 
 int from_kymajor(const double2* src, double2* dst, int nh, int ny, int nplanes, hipStream_t st)
