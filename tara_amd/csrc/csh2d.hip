@@ -44,6 +44,7 @@
 // Lx = Ly = 2 pi (:16-21), so kx = i-1 and ky = j-1 or j-1-Ny are exact integers;
 // the host builds the tables with that exact expression (csh_plan_init).
 #include <algorithm>
+#include <type_traits>
 
 #include "csh2d_dev.h"
 
@@ -187,14 +188,22 @@ __global__ __launch_bounds__((YiShape<NY, SCR>::NT), (YiShape<NY, SCR>::IL ? 4 :
     const int ncol = lim ? bd.hk : nh, ntile = (ncol + S::CB - 1) / S::CB;
     if ((int)blockIdx.x >= ntile) return;
     const int i = xcd_remap(blockIdx.x, ntile) * S::CB + c;
-    const bool live = i < ncol;
+    const bool live = S::CB == 1 || i < ncol;
     const size_t col = (size_t)(live ? i : 0) * NY;
     double2 wv[E];
+    // Separate loads: a test of the circle before each would put its latency between
+    // every two loads of a state that holds everything.
+    if (lim) {
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const int j = rf_first_idx<NY, csh_yem(NY)>(t, e);
-        wv[e] = make_double2(0.0, 0.0);
-        if (live && (!lim || i < bd.imin[j])) wv[e] = w[col + j];
+        for (int e = 0; e < E; ++e) {
+            const int j = rf_first_idx<NY, csh_yem(NY)>(t, e);
+            wv[e] = make_double2(0.0, 0.0);
+            if (live && i < bd.imin[j]) wv[e] = w[col + j];
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            wv[e] = live ? w[col + rf_first_idx<NY, csh_yem(NY)>(t, e)] : make_double2(0.0, 0.0);
     }
     csh_yinv_column<NY, SCR, GS>(wv, i, live, sq, tw, lam, ld, g0, g1, g2, g3);
 }
@@ -341,33 +350,41 @@ __global__ __launch_bounds__(YShape<NY>::NT) void k_csh_yfwd(YfwdArgs a, CshBand
     if (lim && (int)blockIdx.x >= nfwd) return;
     const int tile = csh_tile(blockIdx.x, nfwd, gridDim.x);
     const int i = tile * S::CB + c;
-    const bool live = i < (lim ? bd.hk : a.nh);
+    const bool live = S::CB == 1 || i < (lim ? bd.hk : a.nh);
     const size_t col = (size_t)(live ? i : 0) * NY;
     double2 v[E];
     if (tile < nfwd) {
 #pragma unroll
         for (int e = 0; e < E; ++e)
-            v[e] = i < bd.hk ? a.h[blk8(i, rf_first_idx<NY, csh_yem(NY)>(t, e), a.nh)] : make_double2(0.0, 0.0);
+            v[e] = S::CB == 1 || i < bd.hk ? a.h[blk8(i, rf_first_idx<NY, csh_yem(NY)>(t, e), a.nh)]
+                                           : make_double2(0.0, 0.0);
         sq.template fft<-1>(v, tw);
     }
     if (!live) return;
     const double kxv = (double)i;
     bool finite = true;  // the new state's values (AB2, RK4 stage 4)
+    auto update = [&](auto limited) {
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const int j = rf_final_idx<NY, csh_yem(NY)>(t, e);
-        const size_t q = col + j;
-        double2 nl = v[e];
-        if (i >= a.imin[j]) {
-            if (lim) continue;  // zero, and stays so
-            nl = make_double2(0.0, 0.0);
+        for (int e = 0; e < E; ++e) {
+            const int j = rf_final_idx<NY, csh_yem(NY)>(t, e);
+            const size_t q = col + j;
+            double2 nl = v[e];
+            if (i >= a.imin[j]) {
+                if constexpr (limited.value) continue;  // zero, and stays so
+                nl = make_double2(0.0, 0.0);
+            }
+            const double kyv = csh_ky<NY>(j);
+            const double k2 = kxv * kxv + kyv * kyv;
+            double2 wn, av;
+            csh_update<MODE>(a, q, i == 0 && j == 0, nl, a.ws[q], k2, &wn, &av);
+            finite = csh_store<MODE>(a, q, wn, av) && finite;
         }
-        const double kyv = csh_ky<NY>(j);
-        const double k2 = kxv * kxv + kyv * kyv;
-        double2 wn, av;
-        csh_update<MODE>(a, q, i == 0 && j == 0, nl, a.ws[q], k2, &wn, &av);
-        finite = csh_store<MODE>(a, q, wn, av) && finite;
-    }
+    };
+    // apart as in k_csh_yinv
+    if (lim)
+        update(std::true_type{});
+    else
+        update(std::false_type{});
     if (!finite && a.bad) a.bad[blockIdx.y] = 1;
 }
 
@@ -408,35 +425,41 @@ __global__ __launch_bounds__((YiShape<NY, false>::NT), (YiShape<NY, false>::IL ?
     if (lim && (int)blockIdx.x >= nfwd) return;
     const int tile = csh_tile(blockIdx.x, nfwd, gridDim.x);
     const int i = tile * S::CB + c;
-    const bool live = i < (lim ? bd.hk : a.nh);
+    const bool live = S::CB == 1 || i < (lim ? bd.hk : a.nh);
     const size_t col = (size_t)(live ? i : 0) * NY;
     double2 v[E];
-#pragma unroll
-    for (int e = 0; e < E; ++e) v[e] = make_double2(0.0, 0.0);
     if (tile < nfwd) {
 #pragma unroll
         for (int e = 0; e < E; ++e)
-            if (i < bd.hk) v[e] = a.h[blk8(i, rf_first_idx<NY, csh_yem(NY)>(t, e), a.nh)];
+            v[e] = S::CB == 1 || i < bd.hk ? a.h[blk8(i, rf_first_idx<NY, csh_yem(NY)>(t, e), a.nh)]
+                                           : make_double2(0.0, 0.0);
         sq.template fft<-1>(v, tw);
     }
     const double kxv = (double)i;
     bool finite = true;  // the new state's values (AB2, RK4 stage 4)
+    auto update = [&](auto limited) {
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-        const int j = rf_final_idx<NY, csh_yem(NY)>(t, e);
-        const size_t q = col + j;
-        const bool in = live && i < a.imin[j];
-        if (!in && (lim || !live)) {
-            v[e] = make_double2(0.0, 0.0);
-            continue;
+        for (int e = 0; e < E; ++e) {
+            const int j = rf_final_idx<NY, csh_yem(NY)>(t, e);
+            const size_t q = col + j;
+            const bool in = live && i < a.imin[j];
+            if (limited.value ? !in : !live) {
+                v[e] = make_double2(0.0, 0.0);
+                continue;
+            }
+            const double2 nl = in ? v[e] : make_double2(0.0, 0.0);
+            const double kyv = csh_ky<NY>(j);
+            double2 wn, av;  // wn: the next stage's input
+            csh_update<MODE>(a, q, false, nl, a.ws[q], kxv * kxv + kyv * kyv, &wn, &av);
+            finite = csh_store<MODE>(a, q, wn, av) && finite;
+            v[e] = wn;
         }
-        const double2 nl = in ? v[e] : make_double2(0.0, 0.0);
-        const double kyv = csh_ky<NY>(j);
-        double2 wn, av;  // wn: the next stage's input
-        csh_update<MODE>(a, q, false, nl, a.ws[q], kxv * kxv + kyv * kyv, &wn, &av);
-        finite = csh_store<MODE>(a, q, wn, av) && finite;
-        v[e] = wn;
-    }
+    };
+    // apart as in k_csh_yinv
+    if (lim)
+        update(std::true_type{});
+    else
+        update(std::false_type{});
     if (!finite && a.bad) a.bad[blockIdx.y] = 1;
     sq.final_to_first(v);
     csh_yinv_column<NY, false, GS>(v, i, live, sq, tw, 0.0, ld, g0, g1, g2, g3);
