@@ -15,8 +15,8 @@ struct CShape {
 };
 
 struct ColArgs {
-    const double2* src[14];
-    double2* dst[14];
+    const double2* src[12];
+    double2* dst[12];
     long es;       // element stride along the transform (complex elements)
     long pstride;  // plane stride
     int tpp;       // tiles (of 8 columns) per plane

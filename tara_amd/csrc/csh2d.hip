@@ -224,7 +224,7 @@ struct XShape {
     // Per-row exchange buffer (complex elements).  Rows are interleaved across
     // lanes, so successive row buffers are offset by 4 elements (64 B) to land
     // on different LDS banks.
-    static constexpr int LDSR = WIDE && RB == 1 ? NX : (SPLIT ? RF<NX, EM>::LDS / 2 : RF<NX, EM>::LDS) + 4;
+    static constexpr int LDSR = (SPLIT ? RF<NX, EM>::LDS / 2 : RF<NX, EM>::LDS) + 4;
     // the forward half-length transform must use exactly half of the row's threads
     static constexpr bool OK = RB * LDSR * 16 <= 160 * 1024 && NT <= 1024 && NT >= 64 && 2 * TM == T;
 };
@@ -514,27 +514,27 @@ static int launch_yinv_t(const CshPlan& p, const double2* w, const CshPhys& ph, 
     return TARA_OK;
 }
 
+// Below Ny = 256 only batches come here (csh_small): square grids of derive2csh.
 template <int NY>
 static int launch_yinv(const CshPlan& p, const double2* w, const CshPhys& ph, hipStream_t st)
 {
-    if (p.gsh == 1)
-        return ph.screened ? launch_yinv_t<NY, true, 1>(p, w, ph, st) : launch_yinv_t<NY, false, 1>(p, w, ph, st);
-    return ph.screened ? launch_yinv_t<NY, true, 2>(p, w, ph, st) : launch_yinv_t<NY, false, 2>(p, w, ph, st);
+    if constexpr (NY >= 256) {
+        if (p.gsh == 1)
+            return ph.screened ? launch_yinv_t<NY, true, 1>(p, w, ph, st) : launch_yinv_t<NY, false, 1>(p, w, ph, st);
+        if (ph.screened) return launch_yinv_t<NY, true, 2>(p, w, ph, st);
+    }
+    TARA_CHECK(p.gsh == 2 && !ph.screened, TARA_ERR_UNSUPPORTED, "inverse y pass of large grids at %dx%d", p.nx, p.ny);
+    return launch_yinv_t<NY, false, 2>(p, w, ph, st);
 }
 
-// x-pass shapes the autotuner chooses among: {EM, RB, SPLIT}.  Shape 0 is
+// x-pass shapes the autotuner chooses among (launch_x).  Shape 0 is
 // RB = min(8, 512 / T) at EM = 8 without splitting: two workgroups a CU, one in
 // memory while the other transforms (RK4 step, one workgroup of twice the rows ->
 // two: 1024^2 0.172 -> 0.145 ms, 2048^2 0.303 -> 0.297, 2048 x 512 0.166 -> 0.151).
 // Nx = 4096 keeps two rows and one workgroup: of its 2-row groups a single row
 // reads half of every line (4096^2 1.51 ms, single rows 1.60).
-// shape kXPairs runs a row's two field pairs side by side (csh2d_pairs.hip).
-struct XCand {
-    int em, rb, split;
-};
-constexpr XCand kXCands[] = {{8, 0, 0}, {16, 2, 1}, {8, 1, 1}, {16, 4, 1}, {8, 2, 1}, {16, 1, 0},
-                              {4, 1, 0}, {4, 2, 0}, {4, 4, 1}, {8, 0, 0}};
-constexpr int kNumXCands = sizeof(kXCands) / sizeof(kXCands[0]);
+// Shape kXPairs runs a row's two field pairs side by side (csh2d_pairs.hip).
+constexpr int kNumXCands = 10;
 
 template <int NX, int EM>
 constexpr int default_rb()
@@ -617,7 +617,6 @@ static int launch_yfwd(const CshPlan& p, int mode, const YfwdArgs& a, hipStream_
 
 #define TARA_CSH_SWITCH(n, FN, ...)                 \
     switch (n) {                                    \
-        case 16: return FN<16>(__VA_ARGS__);        \
         case 32: return FN<32>(__VA_ARGS__);        \
         case 64: return FN<64>(__VA_ARGS__);        \
         case 128: return FN<128>(__VA_ARGS__);      \
@@ -668,7 +667,12 @@ static int launch_yfwd_inv(const CshPlan& p, int mode, const YfwdArgs& a, hipStr
 
 static int yfwd_inv(const CshPlan& p, int mode, const YfwdArgs& a, hipStream_t st)
 {
-    TARA_CSH_SWITCH(p.ny, launch_yfwd_inv, p, mode, a, st)
+    switch (p.ny) {  // fuse_y: from Ny = 1024
+        case 1024: return launch_yfwd_inv<1024>(p, mode, a, st);
+        case 2048: return launch_yfwd_inv<2048>(p, mode, a, st);
+        case 4096: return launch_yfwd_inv<4096>(p, mode, a, st);
+        default: set_error("fused y pass of large grids at Ny=%d", p.ny); return TARA_ERR_UNSUPPORTED;
+    }
 }
 
 static int yfwd(const CshPlan& p, int mode, const YfwdArgs& a, hipStream_t st)
