@@ -3,7 +3,8 @@
 // advanced together.  Runs are grouped by grid size into buckets; each bucket's
 // passes are single batched launches over all its runs (blockIdx.y = run), the
 // buckets run on streams of their own, and one whole step (every bucket, every
-// stage) is captured once in a hipGraph and replayed per step.
+// stage) is captured once in a hipGraph and replayed per step; so are a call's first
+// and last step, where a bucket's steps are fused (StepKind).
 #include <algorithm>
 #include <map>
 #include <memory>
@@ -30,6 +31,12 @@ struct Bucket {
     hipEvent_t done = nullptr;
 };
 
+// A step of a bucket whose y passes are fused expects G0..G3 to hold the inverse y pass
+// of its state and leaves them holding that of the new one.  A call's first step begins
+// with that pass (the state may have been set since the last call) and its last one does
+// not end with it.  Where no bucket fuses, all steps are STEP_MID.
+enum StepKind { STEP_MID, STEP_FIRST, STEP_LAST, STEP_ONLY, STEP_KINDS };
+
 }  // namespace
 
 struct tara_ens {
@@ -40,61 +47,48 @@ struct tara_ens {
     double dt = 0;
     int scheme = 0;
     bool use_graph = true;
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
+    bool fused = false;  // some bucket's y passes are
+    hipGraph_t graph[STEP_KINDS] = {};
+    hipGraphExec_t exec[STEP_KINDS] = {};
+    long uses[STEP_KINDS] = {};
 };
 
 namespace {
 
 void drop_graph(tara_ens* e)
 {
-    if (e->exec) (void)hipGraphExecDestroy(e->exec);
-    if (e->graph) (void)hipGraphDestroy(e->graph);
-    e->exec = nullptr;
-    e->graph = nullptr;
+    for (int k = 0; k < STEP_KINDS; ++k) {
+        if (e->exec[k]) (void)hipGraphExecDestroy(e->exec[k]);
+        if (e->graph[k]) (void)hipGraphDestroy(e->graph[k]);
+        e->exec[k] = nullptr;
+        e->graph[k] = nullptr;
+    }
 }
 
 // One step of every bucket, forked onto the bucket streams and joined back.
-// Each forward y pass is fused with the following inverse y pass, the last
-// stage's too: a step expects G0..G3 to hold the inverse y pass of the state
-// (enqueue_head) and leaves them holding that of the new state, so that the
-// captured step can be replayed back to back.
-int enqueue_step(tara_ens* e)
+int enqueue_step(tara_ens* e, StepKind kind)
 {
+    const bool first = kind == STEP_FIRST || kind == STEP_ONLY, last = kind == STEP_LAST || kind == STEP_ONLY;
     TARA_HIP(hipEventRecord(e->fork, e->st));
     for (auto& bp : e->b) {
         Bucket& b = *bp;
         TARA_HIP(hipStreamWaitEvent(b.st, e->fork, 0));
-        int rc = csh_fused_step(b.plan, e->scheme, b.ph, e->dt, b.w.as<double2>(), b.aux.as<double2>(),
-                                b.next.as<double2>(), false, b.st, nullptr);
-        if (rc) return rc;
+        int rc;
+        if ((first && (rc = csh_yinv_pass(b.plan, b.w.as<double2>(), b.ph, b.st))) ||
+            (rc = csh_fused_step(b.plan, e->scheme, b.ph, e->dt, b.w.as<double2>(), b.aux.as<double2>(),
+                                 b.next.as<double2>(), last, b.st, nullptr)))
+            return rc;
         TARA_HIP(hipEventRecord(b.done, b.st));
         TARA_HIP(hipStreamWaitEvent(e->st, b.done, 0));
     }
     return TARA_OK;
 }
 
-// The inverse y pass of every bucket's state, once per advance call (the state
-// may have been set or uploaded since the last step).
-int enqueue_head(tara_ens* e)
+int capture(tara_ens* e, StepKind kind)
 {
-    TARA_HIP(hipEventRecord(e->fork, e->st));
-    for (auto& bp : e->b) {
-        Bucket& b = *bp;
-        TARA_HIP(hipStreamWaitEvent(b.st, e->fork, 0));
-        int rc = csh_yinv_pass(b.plan, b.w.as<double2>(), b.ph, b.st);
-        if (rc) return rc;
-        TARA_HIP(hipEventRecord(b.done, b.st));
-        TARA_HIP(hipStreamWaitEvent(e->st, b.done, 0));
-    }
-    return TARA_OK;
-}
-
-int capture(tara_ens* e)
-{
-    drop_graph(e);
+    if (e->exec[kind]) return TARA_OK;
     TARA_HIP(hipStreamBeginCapture(e->st, hipStreamCaptureModeThreadLocal));
-    int rc = enqueue_step(e);
+    int rc = enqueue_step(e, kind);
     hipGraph_t g = nullptr;
     hipError_t ce = hipStreamEndCapture(e->st, &g);
     if (rc) {
@@ -102,8 +96,9 @@ int capture(tara_ens* e)
         return rc;
     }
     TARA_HIP(ce);
-    e->graph = g;
-    TARA_HIP(hipGraphInstantiate(&e->exec, e->graph, nullptr, nullptr, 0));
+    if (e->graph[kind]) (void)hipGraphDestroy(e->graph[kind]);  // of a failed instantiation
+    e->graph[kind] = g;
+    TARA_HIP(hipGraphInstantiate(&e->exec[kind], g, nullptr, nullptr, 0));
     return TARA_OK;
 }
 
@@ -201,6 +196,7 @@ extern "C" int tara_ens_create(int nruns, const int* n, const double* nu, double
         Bucket& b = *bp;
         const int cnt = (int)b.runs.size();
         if ((rc = csh_plan_init(b.plan, b.n, b.n, cnt))) return rc;
+        e->fused = e->fused || csh_fuses_y(b.plan);
         // per-run slots are bstride apart (padded); the host-side staging
         // buffer holds exactly one reference-layout spectrum (nh x ny)
         const size_t bytes = b.plan.bstride * sizeof(double2);
@@ -312,15 +308,26 @@ extern "C" int tara_ens_advance(tara_ens* e, int nsteps)
 {
     TARA_CHECK(e && nsteps >= 0, TARA_ERR_ARG, "bad argument");
     int rc;
-    // the step graph is captured on the first call, also with nsteps = 0 (a
-    // caller can then capture before any work is in flight)
-    if (e->use_graph && !e->exec && (rc = capture(e))) return rc;
-    if (nsteps == 0) return TARA_OK;
-    if ((rc = enqueue_head(e))) return rc;
+    // the step graph is captured on the first call, also with nsteps = 0 (a caller can
+    // then capture before any work is in flight; all kinds of step are then).  The
+    // first and last step of a call are captured when they come a second time: a graph
+    // costs 0.1 to 0.2 ms to make and saves 20 to 100 us each time.
+    if (e->use_graph) {
+        if ((rc = capture(e, STEP_MID))) return rc;
+        for (StepKind k : {STEP_FIRST, STEP_LAST, STEP_ONLY})
+            if (e->fused && (nsteps == 0 || ((nsteps == 1) == (k == STEP_ONLY) && e->uses[k]++ > 0)) &&
+                (rc = capture(e, k)))
+                return rc;
+    }
     for (int s = 0; s < nsteps; ++s) {
-        if (e->use_graph) {
-            TARA_HIP(hipGraphLaunch(e->exec, e->st));
-        } else if ((rc = enqueue_step(e))) {
+        const StepKind k = !e->fused         ? STEP_MID
+                           : nsteps == 1     ? STEP_ONLY
+                           : s == 0          ? STEP_FIRST
+                           : s == nsteps - 1 ? STEP_LAST
+                                             : STEP_MID;
+        if (e->use_graph && e->exec[k]) {
+            TARA_HIP(hipGraphLaunch(e->exec[k], e->st));
+        } else if ((rc = enqueue_step(e, k))) {
             return rc;
         }
     }
@@ -332,13 +339,14 @@ extern "C" int tara_ens_graph_nodes(tara_ens* e, long* nodes, long* kernels)
     TARA_CHECK(e && nodes, TARA_ERR_ARG, "null argument");
     *nodes = 0;
     if (kernels) *kernels = 0;
-    if (!e->graph) return TARA_OK;
+    const hipGraph_t graph = e->graph[STEP_MID];
+    if (!graph) return TARA_OK;
     size_t n = 0;
-    TARA_HIP(hipGraphGetNodes(e->graph, nullptr, &n));
+    TARA_HIP(hipGraphGetNodes(graph, nullptr, &n));
     *nodes = (long)n;
     if (kernels && n) {
         std::vector<hipGraphNode_t> v(n);
-        TARA_HIP(hipGraphGetNodes(e->graph, v.data(), &n));
+        TARA_HIP(hipGraphGetNodes(graph, v.data(), &n));
         long k = 0;
         for (size_t i = 0; i < n; ++i) {
             hipGraphNodeType t;

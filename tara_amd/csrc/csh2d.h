@@ -125,6 +125,7 @@ int csh_advance(const CshPlan& p, int scheme, int nsteps, const CshPhys& ph, dou
 // G0..G3 are left holding the inverse y pass of the new state).  For Ny < 1024
 // and enough columns to fill the chip the passes are not fused: csh_yinv_pass
 // does nothing and the step runs csh_rhs_stage per stage.
+bool csh_fuses_y(const CshPlan& p);  // whether they are
 int csh_yinv_pass(const CshPlan& p, const double2* w, const CshPhys& ph, hipStream_t st);
 int csh_fused_step(const CshPlan& p, int scheme, const CshPhys& ph, double dt, double2* w, double2* aux,
                    double2* next, bool plain_last, hipStream_t st, EventTimer* tm);

@@ -667,7 +667,7 @@ static int launch_yfwd_inv(const CshPlan& p, int mode, const YfwdArgs& a, hipStr
 
 static int yfwd_inv(const CshPlan& p, int mode, const YfwdArgs& a, hipStream_t st)
 {
-    switch (p.ny) {  // fuse_y: from Ny = 1024
+    switch (p.ny) {  // csh_fuses_y: from Ny = 1024
         case 1024: return launch_yfwd_inv<1024>(p, mode, a, st);
         case 2048: return launch_yfwd_inv<2048>(p, mode, a, st);
         case 4096: return launch_yfwd_inv<4096>(p, mode, a, st);
@@ -866,11 +866,11 @@ int csh_rhs_direct(const CshPlan& p, const double2* w, double2* f, const CshPhys
 // small to fill the chip (csh2d_small.hip); else, below 1024, the fused pass
 // holds fewer waves per CU than the separate forward y pass, and the 128-512
 // ensemble step measured 6.65 ms fused against 6.43 ms separate.
-static bool fuse_y(const CshPlan& p) { return p.ny >= 1024 || csh_small(p); }
+bool csh_fuses_y(const CshPlan& p) { return p.ny >= 1024 || csh_small(p); }
 
 int csh_yinv_pass(const CshPlan& p, const double2* w, const CshPhys& ph, hipStream_t st)
 {
-    if (!fuse_y(p)) return TARA_OK;  // the unfused step runs its own inverse y passes
+    if (!csh_fuses_y(p)) return TARA_OK;  // the unfused step runs its own inverse y passes
     int rc = csh_small(p) ? csh_small_yinv(p, w, ph, p.ny, 1, st) : yinv(p, w, ph, st);
     if (rc) return rc;
     TARA_HIP(hipGetLastError());
@@ -883,7 +883,7 @@ int csh_fused_step(const CshPlan& p, int scheme, const CshPhys& ph, double dt, d
     const bool small = csh_small(p);
     TARA_CHECK(!ph.screened || small, TARA_ERR_ARG, "the fused step of large grids covers derive2csh only");
     int rc;
-    if (!fuse_y(p)) {
+    if (!csh_fuses_y(p)) {
         if (scheme == TARA_SCHEME_AB2) return csh_rhs_stage(p, w, CSH_AB2, ph, dt, w, aux, nullptr, st, tm);
         for (int k = 0; k < 4; ++k)
             if ((rc = csh_rhs_stage(p, k == 0 ? w : next, CSH_RK4_1 + k, ph, dt, w, aux, next, st, tm))) return rc;
