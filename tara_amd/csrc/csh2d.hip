@@ -443,7 +443,7 @@ __global__ __launch_bounds__((YiShape<NY, false>::NT), (YiShape<NY, false>::IL ?
             const int j = rf_final_idx<NY, csh_yem(NY)>(t, e);
             const size_t q = col + j;
             const bool in = live && i < a.imin[j];
-            if (limited.value ? !in : !live) {
+            if (!in && (limited || !live)) {
                 v[e] = make_double2(0.0, 0.0);
                 continue;
             }
@@ -455,8 +455,12 @@ __global__ __launch_bounds__((YiShape<NY, false>::NT), (YiShape<NY, false>::IL ?
             v[e] = wn;
         }
     };
-    // apart as in k_csh_yinv
-    if (lim)
+    // apart as in k_csh_yinv; with one workgroup of 16 wavefronts a CU (IL) the other
+    // waves cover the latency, and together they are faster (4096^2 RK4 step of a
+    // general state 2.161 against 2.177 ms)
+    if constexpr (S::IL)
+        update(lim);
+    else if (lim)
         update(std::true_type{});
     else
         update(std::false_type{});
