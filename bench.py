@@ -34,17 +34,22 @@ FP64_PEAK_TFLOPS = 78.6  # MI355X vector FP64
 # --no-cpu-baseline --no-ensemble --no-fno), each scaled by what the counter reads for a device copy
 # of known size (tara_amd/calib/copy_probe: FETCH_SIZE x 2.0, WRITE_SIZE x 1.0).
 MEASURED_TRAFFIC = {
-    ("k_csh_yinv", 4096): 4.267e8,
-    ("k_csh_yfwd_inv", 4096): 6.832e8,  # mean over the four RK4 stage variants
+    ("k_csh_yinv", 4096): 4.260e8,
+    ("k_csh_yfwd_inv", 4096): 6.875e8,  # mean over the four RK4 stage variants
     # k_csh_x per x-pass shape (the autotuner's choice, see tara_csh_tune)
     ("k_csh_x", 4096, 0): 4.546e8,
-    ("k_csh_x", 4096, 1): 5.983e8,
-    ("k_csh_x", 4096, 2): 4.505e8,
-    ("k_csh_x", 4096, 3): 2.791e9,
-    ("k_csh_x", 4096, 4): 7.494e8,
-    ("k_csh_x", 4096, 5): 4.503e8,
-    ("k_csh_x", 4096, 6): 4.500e8,
-    ("k_csh_x", 4096, 9): 4.502e8,
+    ("k_csh_x", 4096, 1): 5.978e8,
+    ("k_csh_x", 4096, 2): 4.503e8,
+    ("k_csh_x", 4096, 3): 2.797e9,
+    ("k_csh_x", 4096, 4): 7.484e8,
+    ("k_csh_x", 4096, 5): 4.505e8,
+    ("k_csh_x", 4096, 6): 4.501e8,
+    ("k_csh_x", 4096, 9): 4.501e8,
+    # 3D: the passes whose launches are alike (the inverse ones of a call's first step
+    # carry every tile)
+    ("k_mhd_x", 256): 2.106e9,
+    ("k_mhd_col_forward", 256): 1.702e9,
+    ("k_mhd_zfwd", 256): 1.993e9,  # with the next step's inverse (all but a call's last)
 }
 METRIC = "grid-pt steps/s FP64 (2D 4096², 3D 256³ MHD); FNO sim-time/s at ≤5% L2 err"
 

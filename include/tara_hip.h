@@ -102,9 +102,9 @@ int tara_csh_destroy(tara_csh* ctx);
  * context's stream.  tara_csh_kernel_stats returns, per kernel class
  * (0 = inverse y pass, 1 = x pass, 2 = forward y pass + update), the number of
  * timed launches and their summed duration in milliseconds, then resets.  For
- * the derive2csh solver at Ny >= 1024, class 2 launches (all but each advance
- * call's last) also run the next stage's inverse y pass, and class 0 holds one
- * launch per advance call. */
+ * the derive2csh solver at Ny >= 1024, and either solver on grids too small to
+ * fill the chip, class 2 launches (all but each advance call's last) also run the
+ * next stage's inverse y pass, and class 0 holds one launch per advance call. */
 int tara_csh_set_timing(tara_csh* ctx, int on);
 int tara_csh_kernel_stats(tara_csh* ctx, int nclass, long* counts, double* ms);
 /* Autotuner (no counterpart in the reference, whose FFTW planner runs in
@@ -157,7 +157,8 @@ int tara_philox4x32_10(const unsigned ctr[4], const unsigned key[2], unsigned ou
  * viscosity nu[r], common dt, classic RK4 or AB2).  Runs of one grid size form a
  * bucket whose passes are single batched launches; one step of every bucket is
  * captured once in a hipGraph (tara_ens_use_graph(ctx, 0) launches eagerly
- * instead) and replayed per step.  upload/download take one run's (Nh, N) half
+ * instead) and replayed per step, a call's first and last step from their second
+ * time on.  upload/download take one run's (Nh, N) half
  * spectrum in the reference layout; upload zeroes that run's AB2 history.
  * tara_ens_tune runs the x-pass autotuner per bucket.
  */
@@ -277,8 +278,9 @@ int tara_ab2com(int nx, int ny, int nh, double dt, const double* const state[6],
 /* Device-resident AB2 stepping of either family (the derive + ab2 + rotation
  * loops of src/main2coh.f95:278-300 and src/main2com.f95:364-380, without the
  * diagnostics).  upload/download take 3 (coh) or 6 (com) arrays; the AB2
- * history starts at zero on upload.  Timing classes: 0 = prep + inverse y,
- * 1 = x passes (+ the com middle pass), 2 = forward y + assembly.  sync and
+ * history starts at zero on upload.  Timing classes: 0 = prep + inverse y (once
+ * per advance call), 1 = x passes (+ the com middle pass), 2 = forward y + assembly
+ * (+ prep and inverse y of the new state, all but a call's last).  sync and
  * download return TARA_ERR_NONFINITE once an update has stored a NaN or Inf
  * (the flag clears on upload). */
 typedef struct tara_f2 tara_f2;
@@ -363,8 +365,9 @@ int tara_mhd_ic_random(tara_mhd* ctx, unsigned seed, double k0, double e_kin, do
  * spectral fields). */
 int tara_mhd_energy(tara_mhd* ctx, double out[10]);
 int tara_mhd_record_energy(tara_mhd* ctx, int nrec, int every, double* rows);
-/* Kernel timing as for tara_csh: classes 0 = inverse z+y passes, 1 = x pass,
- * 2 = forward y pass, 3 = forward z pass + assembly + update. */
+/* Kernel timing as for tara_csh: classes 0 = inverse y pass (and, in an advance
+ * call's first step, inverse z), 1 = x pass, 2 = forward y pass, 3 = forward z pass +
+ * assembly + update (+ inverse z of the new state, all but a call's last). */
 int tara_mhd_set_timing(tara_mhd* ctx, int on);
 int tara_mhd_kernel_stats(tara_mhd* ctx, int nclass, long* counts, double* ms);
 

@@ -865,11 +865,14 @@ int csh_rhs_direct(const CshPlan& p, const double2* w, double2* f, const CshPhys
     return TARA_OK;
 }
 
-// Fusing the forward y pass with the next inverse y pass pays from Ny = 1024
-// (1024^2 RK4 step 0.181 -> 0.168 ms, 4096^2 2.41 -> 2.36 ms) and on grids too
-// small to fill the chip (csh2d_small.hip); else, below 1024, the fused pass
-// holds fewer waves per CU than the separate forward y pass, and the 128-512
-// ensemble step measured 6.65 ms fused against 6.43 ms separate.
+// Fusing the forward y pass with the next inverse y pass pays at Ny = 1024 and 2048
+// (RK4 step apart -> fused, general / limited state: 1024^2 0.154 -> 0.138 / 0.151 ->
+// 0.138 ms, 2048^2 0.406 -> 0.391 / 0.301 -> 0.271) and on grids too small to fill the
+// chip (csh2d_small.hip).  At 4096^2 it did with the four fields in G0..G3 (2.41 ->
+// 2.36); with the pairs the passes apart are faster (2.06 against 2.16 / 1.403 against
+// 1.427), not taken up yet.  Below 1024 the fused pass holds fewer waves per CU than the
+// separate forward y pass: the 128-512 ensemble step measured 6.65 ms fused against 6.43
+// separate, with the four fields in G0..G3.
 bool csh_fuses_y(const CshPlan& p) { return p.ny >= 1024 || csh_small(p); }
 
 int csh_yinv_pass(const CshPlan& p, const double2* w, const CshPhys& ph, hipStream_t st)

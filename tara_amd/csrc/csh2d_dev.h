@@ -28,15 +28,16 @@ __device__ __forceinline__ size_t blk8(int i, int j, int nh)
 
 // Offset of element (i, j) in the intermediates G0..G3: groups of 2^gs rows
 // interleaved per kx, ld columns per group (CshPlan::gsh, CshPlan::gld).
-// Ny = 4096, 2-row groups: a wave of the x pass reading two rows reads
-// contiguous 32-byte pairs over consecutive kx, and the inverse y pass writes
-// its two interleaved columns' pairs together (YiShape); 0.195 ms inverse y +
-// 0.276 ms x at 4096^2, against 0.186 + 0.311 ms with 4-row groups.  Smaller
-// Ny, 4-row groups and contiguous columns: at 1024^2 0.0201 ms inverse y +
-// 0.0186 ms x, against 0.0236 + 0.0179 ms with 2-row groups and four
-// interleaved columns.  (With one column per inverse-y workgroup at 4096^2,
-// 4-row groups had measured faster than 8-row (0.20, 0.39 ms), 2-row (0.25,
-// 0.31) and plain row-major (0.34, 0.31).)
+// The groups follow Nx, which the x pass knows at compile time.  Nx = 4096, 2-row
+// groups: a wave of the x pass reading two rows reads contiguous 32-byte pairs over
+// consecutive kx.  Smaller Nx, 4-row groups.  Which columns an inverse y workgroup
+// holds follows Ny (YiShape): at Ny = 4096 two, interleaved over the lanes, so that at
+// 4096^2 their pairs of a row group are written together; else contiguous ones.
+// Measured with the four fields themselves in G0..G3 and every column carried: 4096^2
+// 0.195 ms inverse y + 0.276 ms x, against 0.186 + 0.311 ms with 4-row groups; 1024^2
+// 0.0201 + 0.0186 ms, against 0.0236 + 0.0179 ms with 2-row groups and four interleaved
+// columns.  (With one column per inverse-y workgroup at 4096^2, 4-row groups measured
+// faster than 8-row (0.20, 0.39 ms), 2-row (0.25, 0.31) and plain row-major (0.34, 0.31).)
 __device__ __forceinline__ size_t blkg(int i, int j, int ld, int gs)
 {
     return ((size_t)(j >> gs) * ld + i) * (1 << gs) + (j & ((1 << gs) - 1));
